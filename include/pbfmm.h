@@ -207,7 +207,8 @@ int pbfmm_vmult_dev(pbfmm_handle *h, const double *d_src, double *d_dst, int32_t
 /* pbfmm_vmult_dev on nrhs columns (device pointers, column r at d_src + r*ld
  * and d_dst + r*ld, ld >= n_dofs; the two ranges must not overlap).  One
  * operator application serves all columns: the translation pair lists are
- * expanded over them, so each level is one launch for every column.  Column
+ * expanded over them, so each level is one launch for every column, and the
+ * near field is read once for 8 or 16 of them.  Column
  * r equals pbfmm_vmult_dev of column r (FP64 to rounding; FP32 within its
  * rounding, as the atomics sum in another order).  Pure Neumann problems
  * keep vmult's norm shifts, which apply one column at a time.  The

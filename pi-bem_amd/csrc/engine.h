@@ -92,6 +92,7 @@ struct Engine {
   ChunkDev m2m_cl, m2l_cl, l2l_cl;
   ChunkDev m2m_g_cl;  // M2M two child levels per launch (FarPlan::m2m_g)
   ChunkDev l2l_g_cl;  // L2L two target levels per launch (FarPlan::l2l_g)
+  int near_max_rows = 0;  // rows of the near field's largest leaf
   DevBuf d_pval_beg;  // FP32 operator values: per-leaf offsets of the row-pair layout
   DevBuf d_row_leaf, d_row_beg, d_rows, d_col_beg, d_cols, d_val_beg, d_ent_beg, d_ent_cell,
       d_ent_mask, d_ent_near, d_ent_colpos, d_leaf_block;
@@ -292,6 +293,7 @@ struct Engine {
   ChunkList mr_m2m_h, mr_m2l_h, mr_l2l_h;
   ChunkDev mr_m2m, mr_m2l, mr_l2l;
   DevBuf mr_me64, mr_le64, mr_me32, mr_le32, mr_out;
+  DevBuf mr_xp;  // the vectors packed for k_spmm_cols, 16 right-hand sides of a DoF consecutive
   DevBuf mr_seg_off, mr_seg, mr_rch, mr_sch, mr_act, mr_segv;
   DevBuf mr_V, mr_w, mr_r, mr_d, mr_t1, mr_t2, mr_hs, mr_ys, mr_red;
   int mr_restart = 0;

@@ -585,6 +585,159 @@ __global__ void __launch_bounds__(256) k_spmv_cols(int nleaf, int per_xcd, NearA
   }
 }
 
+// Several right-hand sides: NR (8 or 16) columns of X per pass over the near
+// field (blockIdx.y: groups of NR), from the column-vector copy, so that the
+// values are read once for NR of them.  A launch of k_spmv_cols per
+// right-hand side is bound by HBM and reads them NR times.  Every (row,
+// right-hand side) sum runs in k_spmv_cols' own order (the same streams of
+// column vectors, the same partial sums), so a column of a lockstep call
+// equals the single-vector kernel's bit for bit.
+//   x: the inputs packed by k_pack_rhs, the NR of a DoF consecutive, so that
+//   staging a column is one contiguous run; in LDS a column vector's inputs
+//   are 16 bytes per right-hand side.
+//   A thread owns 2 rows (i, i + RP) and MU right-hand sides of one stream:
+//   two 16-byte loads of values and MU LDS reads feed 2 MU CW multiply-adds.
+//   RP = 4, 8, 16 or 32 row pairs for leaves (row blocks) of at most 8, 16,
+//   32 or 64 rows, so that narrow leaves still fill the workgroup's lanes.
+// Measured, 16 right-hand sides of a thin hull mirrored at its waterline
+// (22,876 DoFs, leaf 20: 7 rows and ~20,000 columns per leaf, 457 M values):
+// FP32 6.23 -> 1.09 ms, FP64 8.49 -> 1.86 ms, bound by the leaves' inputs
+// (64 bytes per column, 4.2 GB out of L2) beside the values.  16x16x4 MFMA
+// steps on 16-row tiles took the same time, and their longer FP32 chains were
+// four times further from FP64.  Workgroups of 128 threads: 1.45 ms.
+template <typename T, int NR>
+__global__ void __launch_bounds__(256) k_pack_rhs(int64_t n, int64_t stride, int nrhs, const double *__restrict__ x,
+                                                  T *__restrict__ xp) {
+  __shared__ T tile[64][NR + 1];
+  const int t = (int)threadIdx.x, r0 = NR * (int)blockIdx.y;
+  const int64_t i0 = 64 * (int64_t)blockIdx.x;
+  for (int m = t >> 6; m < NR; m += 4) {
+    const int64_t i = i0 + (t & 63);
+    tile[t & 63][m] = i < n && r0 + m < nrhs ? (T)x[(r0 + m) * stride + i] : T(0);
+  }
+  __syncthreads();
+  T *o = xp + ((int64_t)blockIdx.y * n + i0) * NR;
+  for (int k = t; k < 64 * NR; k += 256)
+    if (i0 + k / NR < n) o[k] = tile[k / NR][k % NR];
+}
+
+// One row block (rows row0 .. row0 + 2 RP of the leaf): all its columns, S
+// streams, a tile of 4 S column vectors at a time, pipelined: while a tile is
+// used, the next one's values and inputs and the one after's column numbers
+// are in flight (without that, leaves of a few hundred workgroups wait on
+// the chain column -> input -> LDS of every tile).
+template <typename T, int NR, int S, int RP>
+__device__ __forceinline__ void spmm_rows(const NearArgs<T> &a, const T *__restrict__ X, int cb, int C, int R, int r0,
+                                          int row0, const T *__restrict__ vals, unsigned char *smem, int rhs0,
+                                          int nrhs) {
+  using TV = std::conditional_t<sizeof(T) == 4, float4, double2>;
+  constexpr int CW = 16 / sizeof(T), MG = 256 / (S * RP), MU = NR / MG;
+  static_assert(S * RP * MG == 256 && MU * MG == NR, "a thread per (stream, row pair, group of right-hand sides)");
+  constexpr int Q = 4, QT = Q * S;           // vectors per stream and per tile
+  constexpr int NI = (QT * NR + 255) / 256;  // input vectors a thread stages per tile
+  const TV *VV = reinterpret_cast<const TV *>(vals);
+  TV *xs = reinterpret_cast<TV *>(smem);  // two tiles of [vector][NR]
+  T *part = reinterpret_cast<T *>(smem);  // [S][2 RP][NR], after the last tile
+  const int t = (int)threadIdx.x, mg = t % MG, i = (t / MG) % RP, s = t / (MG * RP);
+  const int NQ = (C + CW - 1) / CW, NT = (NQ + QT - 1) / QT;
+  const int ra = min(row0 + i, R - 1), rb = min(row0 + i + RP, R - 1);  // rows past the last: sums not stored
+  const int *cols = a.cols + cb;
+  T acc[2][MU] = {};
+  int ci[NI][CW];  // columns, -1 past the last one
+  TV xv[NI], mv[2][Q], mn[2][Q];
+  auto load_cols = [&](int tile) {
+#pragma unroll
+    for (int k = 0; k < NI; ++k) {
+      const int e = t + 256 * k, c = CW * (tile * QT + e / NR);
+#pragma unroll
+      for (int j = 0; j < CW; ++j) ci[k][j] = e < QT * NR && c + j < C ? cols[c + j] : -1;
+    }
+  };
+  auto load_x = [&]() {
+#pragma unroll
+    for (int k = 0; k < NI; ++k) {
+      __align__(16) T v[CW];
+#pragma unroll
+      for (int j = 0; j < CW; ++j) v[j] = ci[k][j] >= 0 ? X[(int64_t)ci[k][j] * NR + t % NR] : T(0);
+      xv[k] = *reinterpret_cast<const TV *>(v);
+    }
+  };
+  auto load_m = [&](int tile, TV (&m)[2][Q]) {
+#pragma unroll
+    for (int j = 0; j < Q; ++j) {
+      const int q = min(tile * QT + s + j * S, NQ - 1);  // past the last vector: read again, not used
+      m[0][j] = VV[(int64_t)q * R + ra];
+      m[1][j] = VV[(int64_t)q * R + rb];
+    }
+  };
+  if (NT > 0) {
+    load_cols(0);
+    load_x();
+    load_m(0, mv);
+    load_cols(1);
+  }
+  for (int tile = 0; tile < NT; ++tile) {
+    TV *buf = xs + (tile & 1) * (QT * NR);
+#pragma unroll
+    for (int k = 0; k < NI; ++k)
+      if (t + 256 * k < QT * NR) buf[t + 256 * k] = xv[k];
+    load_x();
+    load_m(tile + 1, mn);
+    load_cols(tile + 2);
+    __syncthreads();  // this tile's inputs stored; the other buffer's readers are past it
+    const int left = NQ - tile * QT - s;
+#pragma unroll
+    for (int j = 0; j < Q; ++j)
+      if (j * S < left) {
+#pragma unroll
+        for (int m = 0; m < MU; ++m) {
+          const TV x = buf[(s + j * S) * NR + mg * MU + m];
+          acc[0][m] += vdot16(mv[0][j], x);
+          acc[1][m] += vdot16(mv[1][j], x);
+        }
+      }
+#pragma unroll
+    for (int j = 0; j < Q; ++j) mv[0][j] = mn[0][j], mv[1][j] = mn[1][j];
+  }
+  __syncthreads();  // the last tile consumed: its LDS holds the partial sums now
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+#pragma unroll
+    for (int m = 0; m < MU; ++m) part[(s * 2 * RP + i + k * RP) * NR + mg * MU + m] = acc[k][m];
+  __syncthreads();
+  const int rows = min(2 * RP, R - row0);
+  for (int k = t; k < rows * NR; k += 256) {
+    const int m = k / rows, r = k - m * rows;
+    if (rhs0 + m >= nrhs) break;
+    T z = 0;
+    for (int q = 0; q < S; ++q) z += part[(q * 2 * RP + r) * NR + m];
+    a.outN[(int64_t)(rhs0 + m) * a.stride + a.rows[r0 + row0 + r]] = (double)z;
+  }
+}
+
+// blockIdx.z: blocks of 64 rows of a leaf.  The stream count is
+// k_spmv_cols': 16, 8 or 4 for leaves of at most 16, 32 or more rows.
+template <typename T, int NR>
+__global__ void __launch_bounds__(256) k_spmm_cols(int nleaf, int per_xcd, NearArgs<T> a, const T *__restrict__ xp,
+                                                   int64_t n, int nrhs) {
+  // two tiles of inputs (at most 64 vectors), or the partial sums (256 threads x 2 rows x NR / 2)
+  __shared__ __align__(16) unsigned char smem[2 * 64 * NR * 16];
+  static_assert(2 * 64 * NR * 16 >= 256 * NR * (int)sizeof(T), "partial sums fit the tiles");
+  const int leaf = (int)(blockIdx.x % kXcd) * per_xcd + (int)(blockIdx.x / kXcd);
+  if (leaf >= nleaf) return;
+  const int rhs0 = NR * (int)blockIdx.y, row0 = 64 * (int)blockIdx.z;
+  const int r0 = a.row_beg[leaf], R = a.row_beg[leaf + 1] - r0;
+  if (row0 >= R) return;
+  const int cb = a.col_beg[leaf], C = a.col_beg[leaf + 1] - cb;
+  const T *V = a.vals + a.val_beg[leaf], *X = xp + (int64_t)blockIdx.y * n * NR;
+  if (R <= 8) spmm_rows<T, NR, 16, 4>(a, X, cb, C, R, r0, 0, V, smem, rhs0, nrhs);
+  else if (R <= 16) spmm_rows<T, NR, 16, 8>(a, X, cb, C, R, r0, 0, V, smem, rhs0, nrhs);
+  else if (R <= 32) spmm_rows<T, NR, 8, 16>(a, X, cb, C, R, r0, 0, V, smem, rhs0, nrhs);
+  else if (R - row0 <= 16) spmm_rows<T, NR, 4, 8>(a, X, cb, C, R, r0, row0, V, smem, rhs0, nrhs);
+  else if (R - row0 <= 32) spmm_rows<T, NR, 4, 16>(a, X, cb, C, R, r0, row0, V, smem, rhs0, nrhs);
+  else spmm_rows<T, NR, 4, 32>(a, X, cb, C, R, r0, row0, V, smem, rhs0, nrhs);
+}
+
 // One leaf by one wavefront, no LDS and no barrier, RPI rows per iteration.
 // For each tile of 64 x CPL leaf columns (64 bytes of values per lane and
 // row: CPL = 8 / 4 for FP32 / FP64 pairs, 16 / 8 for single values) every
@@ -2225,6 +2378,8 @@ void Engine::upload_mesh_and_tree() {
 }
 
 void Engine::upload_near_plan() {
+  near_max_rows = 0;
+  for (int l = 0; l < near.nleaf; ++l) near_max_rows = std::max(near_max_rows, near.row_beg[l + 1] - near.row_beg[l]);
   up(d_row_leaf, near.row_leaf);
   up(d_row_beg, near.row_beg);
   up(d_rows, near.rows);
@@ -2661,6 +2816,43 @@ void Engine::launch_spmv(int variant, const double *phi, const double *dphi, dou
   } else {
     hipLaunchKernelGGL((k_spmv_wave<T, NK, 4>), dim3((near.nleaf + 3) / 4, R), dim3(256), 0, st, near.nleaf, a);
   }
+}
+
+// Whether R right-hand sides share passes over the near field (k_spmm_cols)
+// or take one SpMV each (blockIdx.y of the SpMV launch).  Values within the
+// 256 MB memory-side cache are read again at its rate, so that few
+// right-hand sides gain nothing there: 63 MB (9,602 DoFs, leaf 96), whole
+// operator, 2 / 4 / 8 / 16 right-hand sides, apart 74 / 86 / 124 / 209 us,
+// together 83 / 92 / 112 / 166 us; 290 MB (38,402 DoFs, Q2, leaf 80) apart
+// 357 / 558 / 963 / 1762 us, together 347 / 459 / 700 / 1173 us.  2 MB (1,538
+// DoFs, leaf 20), 8 / 16 / 32: apart 62 / 90 / 144 us, together 64 / 92 / 143.
+static bool use_spmm(const Engine &e, int R, size_t value_bytes) {
+  const int64_t bytes = e.near.nnz * (int64_t)value_bytes;
+  return bytes >= ((int64_t)256 << 20) ? R >= 2 : R >= (bytes >= ((int64_t)8 << 20) ? 8 : 16);
+}
+
+// The near field of R right-hand sides, n apart.  One (a single column of
+// the lockstep calls) takes the tuned SpMV; more are packed and share passes
+// over the values, 8 or 16 to a pass.
+template <typename T>
+static void launch_spmm(Engine &e, const double *x, double *out, int R) {
+  if (!use_spmm(e, R, sizeof(T))) {
+    e.launch_spmv<T, 1>(e.spmv_variant[sizeof(T) == 4 ? 1 : 0][0], x, nullptr, out, nullptr, R);
+    return;
+  }
+  NearArgs<T> a = near_args<T, 1>(e, x, nullptr, out, nullptr, kColsVariant<T>);
+  a.stride = e.n;
+  T *xp = e.mr_xp.as<T>();
+  const int nl = e.near.nleaf, per_xcd = (nl + kXcd - 1) / kXcd;
+  auto go = [&](auto NRC) {
+    constexpr int NR = decltype(NRC)::value;
+    const unsigned groups = (unsigned)((R + NR - 1) / NR);
+    hipLaunchKernelGGL((k_pack_rhs<T, NR>), dim3(nblk(e.n, 64), groups), dim3(256), 0, e.stream, e.n, e.n, R, x, xp);
+    hipLaunchKernelGGL((k_spmm_cols<T, NR>), dim3(per_xcd * kXcd, groups, (e.near_max_rows + 63) / 64), dim3(256), 0,
+                       e.stream, nl, per_xcd, a, xp, e.n, R);
+  };
+  if (R <= 8) go(std::integral_constant<int, 8>{});
+  else go(std::integral_constant<int, 16>{});
 }
 
 // Times the SpMV kernels (workgroup per leaf; wavefront per leaf with 2 or 4
@@ -4404,6 +4596,7 @@ void Engine::multi_setup(int R) {
   }
   const int64_t N = (int64_t)R * n;
   alloc(mr_out, N * 8);
+  if (R >= 2) alloc(mr_xp, (size_t)((R + 15) / 16 * 16) * n * 8);
   // parts of the lockstep solve: rhs r is entries r * n .. (r + 1) * n
   std::vector<int64_t> off(R + 1), rch{0};
   std::vector<int32_t> sg(N), sch{0};
@@ -4446,7 +4639,7 @@ void Engine::matvec_combined_multi(const double *x, double *out, int R) {
     launch_translate<T, 0, 1>(*this, stream, mr_m2m, lvl<1>(mr_m2m_h, l), lvl<1>(mr_m2m_h, l + 1),
                               F.m2m.template as<T>(), ME, ME);
   // near field, then the far field accumulated onto it
-  if (near.nleaf > 0) launch_spmv<T, 1>(spmv_variant[sizeof(T) == 4 ? 1 : 0][0], x, nullptr, out, nullptr, R);
+  if (near.nleaf > 0) launch_spmm<T>(*this, x, out, R);
   hipLaunchKernelGGL(k_fill<T>, dim3((unsigned)std::min<int64_t>(nblk(ne, 256), 4096)), dim3(256), 0, stream, LE,
                      ne, T(0));
   launch_translate<T, 1, 1>(*this, stream, mr_m2l, 0, nchunks<1>(mr_m2l_h), F.m2l.template as<T>(), ME, LE);
