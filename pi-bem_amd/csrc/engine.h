@@ -316,7 +316,7 @@ struct Engine {
     DevBuf d2c_ptr, d2c_cell, d2c_loc;      // dof -> (cell, local index), cells ascending
     DevBuf m_ptr, m_col, m_val, m_diag, m_pos;  // scalar mass matrix (CSR), pos[c][i][j]
     DevBuf loc;                             // per-cell local matrices / vectors
-    DevBuf b, x, r, z, pv, qv, cg, part;    // CG on three components at once
+    DevBuf x, r, z, pv, qv, cg, part;       // CG on three components at once (interleaved)
     DevBuf in1, in2, out, aux, mask;        // staging of host arrays
     DevBuf grad;                            // last compute_gradients result (3n)
     bool have_grad = false;

@@ -33,10 +33,9 @@ namespace pbfmm {
 namespace {
 
 constexpr int kPsThreads = 256;
-constexpr int kPsRedChunk = kPsThreads * 8;
 constexpr double kPsTol = 1e-13;   // relative CG residual per component
 constexpr int kPsMaxIt = 4000;
-constexpr int kPsCheck = 8;        // host reads the residuals every kPsCheck steps
+constexpr int kPsAhead = 12;       // steps enqueued before the host first reads the state, and between its reads
 
 template <typename T>
 void ps_up(DevBuf &b, const std::vector<T> &v) {
@@ -191,83 +190,190 @@ __global__ void k_ps_gather_mass(int64_t n, const int32_t *__restrict__ d2c_ptr,
   diag[r] = dg != 0.0 ? dg : 1.0;  // a DoF without cells keeps a zero solution
 }
 
-// b[d*n + r] = sum over the cells of r (ascending) of loc[c][d][i]
+// ---------------------------------------------------------------------------
+// Mass-matrix CG on the three components at once, two launches per step.
+// Vectors are interleaved, v[3 i + d], so that a column's three values are one
+// run of 24 bytes.  Each kernel finishes the dot products it needs from its
+// predecessor's partial sums (one per workgroup and component, at most
+// kPsParts), every workgroup in the same order, and workgroup 0 keeps the
+// scalars a later launch reads.  The product is taken of z instead of p:
+// with p = z + beta p_old, M p = M z + beta M p_old, so the new direction
+// needs no pass of its own before its product.  A step whose predecessor
+// converged (every component's |r|^2 <= kPsTol^2 |b|^2) does nothing, so the
+// host looks at the state only every few dozen steps.
+// Bound by latency: 98,306 DoFs (Q2, 1.6 M entries) stream 19 MB of matrix
+// per step.  Eight launches per step with one workgroup per 2048 rows took
+// 112 us a step, this form 25 us (a whole projection with pressure, force and
+// volume on host vectors 4.88 -> 1.80 ms).
+// ---------------------------------------------------------------------------
+constexpr int kPsParts = 512;
+constexpr int kPsLanes = 4;  // per row of M: 9 to 25 entries (8 and 16 lanes: 3 and 8% slower solves)
+// cg[]: rz of even and odd steps, |b|^2, converged, steps taken
+enum { kRZ = 0, kBB = 6, kDone = 9, kSteps = 10, kCgLen = 18 };
+
+// Sums of N values per thread over the workgroup, returned in every thread.
+template <int N>
+__device__ __forceinline__ void ps_block_sums(double (&v)[N], double (*sh)[N]) {
+#pragma unroll
+  for (int k = 0; k < N; ++k) v[k] = ps_wave_sum(v[k]);
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  __syncthreads();
+  if (lane == 0)
+    for (int k = 0; k < N; ++k) sh[wid][k] = v[k];
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < N; ++k) v[k] = (sh[0][k] + sh[1][k]) + (sh[2][k] + sh[3][k]);
+}
+// Partial sums [component][P] of three components
+__device__ __forceinline__ void ps_part_sums(const double *__restrict__ part, int P, double *v) {
+  for (int d = 0; d < 3; ++d) v[d] = 0.0;
+  for (int c = threadIdx.x; c < P; c += kPsThreads)
+    for (int d = 0; d < 3; ++d) v[d] += part[d * P + c];
+}
+__device__ __forceinline__ void ps_store_parts(const double *v, double *__restrict__ part) {
+  if (threadIdx.x == 0)
+    for (int d = 0; d < 3; ++d) part[d * gridDim.x + blockIdx.x] = v[d];
+}
+
+// b_d(r) = sum over the cells of r (ascending) of loc[c][d][i]; x = 0, r = b,
+// z = r / diag; partial sums of r.z and b.b
 template <int DPC>
-__global__ void k_ps_gather_rhs(int64_t n, const int32_t *__restrict__ d2c_ptr, const int32_t *__restrict__ d2c_cell,
-                                const int8_t *__restrict__ d2c_loc, const double *__restrict__ loc,
-                                double *__restrict__ b) {
-  const int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (r >= n) return;
-  double a0 = 0, a1 = 0, a2 = 0;
-  for (int32_t t = d2c_ptr[r]; t < d2c_ptr[r + 1]; ++t) {
-    const double *l = loc + (int64_t)d2c_cell[t] * 3 * DPC + d2c_loc[t];
-    a0 += l[0];
-    a1 += l[DPC];
-    a2 += l[2 * DPC];
-  }
-  b[r] = a0;
-  b[n + r] = a1;
-  b[2 * n + r] = a2;
-}
-
-// CG state cg[]: 0..2 rz, 3..5 pq, 6..8 rr, 9..11 bb, 12..14 alpha, 15..17 beta
-enum { kRZ = 0, kPQ = 3, kRR = 6, kBB = 9, kAL = 12, kBE = 15, kCgLen = 18 };
-
-// x = 0, r = b, z = r / diag, p = z; partial sums of r.z and b.b per component
 __global__ void __launch_bounds__(kPsThreads)
-    k_ps_cg_init(int64_t n, const double *__restrict__ b, const double *__restrict__ diag, double *__restrict__ x,
-                 double *__restrict__ r, double *__restrict__ z, double *__restrict__ p,
-                 double *__restrict__ part) {
-  __shared__ double sh[kPsThreads / 64];
-  const int64_t beg = (int64_t)blockIdx.x * kPsRedChunk, end = min(n, beg + (int64_t)kPsRedChunk);
-  for (int d = 0; d < 3; ++d) {
-    double rz = 0, bb = 0;
-    for (int64_t i = beg + threadIdx.x; i < end; i += kPsThreads) {
-      const int64_t k = d * n + i;
-      const double bi = b[k], zi = bi / diag[i];
-      x[k] = 0.0;
-      r[k] = bi;
-      z[k] = zi;
-      p[k] = zi;
-      rz += bi * zi;
-      bb += bi * bi;
+    k_ps_cg_init(int64_t n, const int32_t *__restrict__ d2c_ptr, const int32_t *__restrict__ d2c_cell,
+                 const int8_t *__restrict__ d2c_loc, const double *__restrict__ loc, const double *__restrict__ diag,
+                 double *__restrict__ x, double *__restrict__ r, double *__restrict__ z, double *__restrict__ rz_part,
+                 double *__restrict__ bb_part, double *__restrict__ cg) {
+  __shared__ double sh[kPsThreads / 64][6];
+  double s[6] = {0, 0, 0, 0, 0, 0};
+  for (int64_t i = blockIdx.x * (int64_t)kPsThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kPsThreads) {
+    double b[3] = {0, 0, 0};
+    for (int32_t t = d2c_ptr[i]; t < d2c_ptr[i + 1]; ++t) {
+      const double *l = loc + (int64_t)d2c_cell[t] * 3 * DPC + d2c_loc[t];
+      for (int d = 0; d < 3; ++d) b[d] += l[d * DPC];
     }
-    const double s0 = ps_block_sum(rz, sh);
-    if (threadIdx.x == 0) part[(kRZ + d) * gridDim.x + blockIdx.x] = s0;
-    const double s1 = ps_block_sum(bb, sh);
-    if (threadIdx.x == 0) part[(kBB + d) * gridDim.x + blockIdx.x] = s1;
+    const double dg = diag[i];
+    for (int d = 0; d < 3; ++d) {
+      const double zi = b[d] / dg;
+      x[3 * i + d] = 0.0;
+      r[3 * i + d] = b[d];
+      z[3 * i + d] = zi;
+      s[d] += b[d] * zi;
+      s[3 + d] += b[d] * b[d];
+    }
   }
+  ps_block_sums<6>(s, sh);
+  ps_store_parts(s, rz_part);
+  ps_store_parts(s + 3, bb_part);
+  if (blockIdx.x == 0 && threadIdx.x == 0) cg[kDone] = cg[kSteps] = 0.0;
 }
-// q = M p (three components), partial sums of p.q
+
+// Step k's direction and product: beta = rz_k / rz_k-1 (0 in step 0),
+// p = z + beta p, q = M z + beta q; partial sums of p.q.  kPsLanes lanes per row.
 __global__ void __launch_bounds__(kPsThreads)
-    k_ps_cg_spmv(int64_t n, const int32_t *__restrict__ m_ptr, const int32_t *__restrict__ m_col,
-                 const double *__restrict__ val, const double *__restrict__ p, double *__restrict__ q,
-                 double *__restrict__ part) {
-  __shared__ double sh[kPsThreads / 64];
-  const int64_t beg = (int64_t)blockIdx.x * kPsRedChunk, end = min(n, beg + (int64_t)kPsRedChunk);
+    k_ps_cg_dir(int64_t n, int k, const int32_t *__restrict__ m_ptr, const int32_t *__restrict__ m_col,
+                const double *__restrict__ val, const double *__restrict__ z, double *__restrict__ p,
+                double *__restrict__ q, const double *__restrict__ rz_part, const double *__restrict__ rr_part,
+                double *__restrict__ pq_part, double *__restrict__ cg) {
+  __shared__ double sh[kPsThreads / 64][6];
+  if (cg[kDone] != 0.0) return;
+  const int P = (int)gridDim.x;
+  // rz_k, and |r|^2 (|b|^2 in step 0: then rr_part is its array)
+  double s[6];
+  ps_part_sums(rz_part, P, s);
+  ps_part_sums(rr_part, P, s + 3);
+  ps_block_sums<6>(s, sh);
+  const double *rz_old = cg + kRZ + 3 * ((k + 1) & 1);
+  double be[3];
+  bool conv = true;
+  for (int d = 0; d < 3; ++d) {
+    be[d] = k > 0 && rz_old[d] > 0.0 ? s[d] / rz_old[d] : 0.0;
+    if (k > 0 ? s[3 + d] > kPsTol * kPsTol * cg[kBB + d] : s[3 + d] != 0.0) conv = false;
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    for (int d = 0; d < 3; ++d) {
+      cg[kRZ + 3 * (k & 1) + d] = s[d];
+      if (k == 0) cg[kBB + d] = s[3 + d];
+    }
+    cg[kSteps] = k;
+  }
+  if (conv) {
+    // the other workgroups decide the same from the same sums; the flag is for later launches
+    if (blockIdx.x == 0 && threadIdx.x == 0) cg[kDone] = 1.0;
+    return;
+  }
+  constexpr int RPB = kPsThreads / kPsLanes;
+  const int l = threadIdx.x % kPsLanes;
   double pq[3] = {0, 0, 0};
-  for (int64_t i = beg + threadIdx.x; i < end; i += kPsThreads) {
-    double a0 = 0, a1 = 0, a2 = 0;
-    for (int32_t k = m_ptr[i]; k < m_ptr[i + 1]; ++k) {
-      const double v = val[k];
-      const int64_t j = m_col[k];
-      a0 += v * p[j];
-      a1 += v * p[n + j];
-      a2 += v * p[2 * n + j];
+  // every lane runs every pass (the row sums need the whole group)
+  const int64_t rows = (n + RPB - 1) / RPB * RPB;
+  for (int64_t i = blockIdx.x * (int64_t)RPB + threadIdx.x / kPsLanes; i < rows; i += (int64_t)P * RPB) {
+    const bool in = i < n;
+    double a[3] = {0, 0, 0};
+    const int32_t e = in ? m_ptr[i + 1] : 0;
+    for (int32_t t = (in ? m_ptr[i] : 0) + l; t < e; t += kPsLanes) {
+      const double v = val[t];
+      const double *zj = z + 3 * (int64_t)m_col[t];
+      a[0] += v * zj[0];
+      a[1] += v * zj[1];
+      a[2] += v * zj[2];
     }
-    q[i] = a0;
-    q[n + i] = a1;
-    q[2 * n + i] = a2;
-    pq[0] += p[i] * a0;
-    pq[1] += p[n + i] * a1;
-    pq[2] += p[2 * n + i] * a2;
+#pragma unroll
+    for (int o = kPsLanes / 2; o > 0; o >>= 1)
+      for (int d = 0; d < 3; ++d) a[d] += __shfl_xor(a[d], o, 64);
+    if (in && l < 3) {
+      const double w = l == 0 ? a[0] : l == 1 ? a[1] : a[2], b = l == 0 ? be[0] : l == 1 ? be[1] : be[2];
+      const int64_t j = 3 * i + l;
+      const double pj = k > 0 ? z[j] + b * p[j] : z[j], qj = k > 0 ? w + b * q[j] : w;
+      p[j] = pj;
+      q[j] = qj;
+      const double t = pj * qj;
+      pq[0] += l == 0 ? t : 0.0;
+      pq[1] += l == 1 ? t : 0.0;
+      pq[2] += l == 2 ? t : 0.0;
+    }
   }
-  for (int d = 0; d < 3; ++d) {
-    const double s = ps_block_sum(pq[d], sh);
-    if (threadIdx.x == 0) part[(kPQ + d) * gridDim.x + blockIdx.x] = s;
-  }
+  ps_block_sums<3>(pq, reinterpret_cast<double(*)[3]>(sh));
+  ps_store_parts(pq, pq_part);
 }
-// finish the partial sums of slots [s0, s0 + cnt) of cg[]
+
+// x += alpha p, r -= alpha q, z = r / diag with alpha = rz / p.q; partial
+// sums of the new r.z and r.r
+__global__ void __launch_bounds__(kPsThreads)
+    k_ps_cg_update(int64_t n, int k, const double *__restrict__ diag, const double *__restrict__ p,
+                   const double *__restrict__ q, double *__restrict__ x, double *__restrict__ r,
+                   double *__restrict__ z, const double *__restrict__ pq_part, double *__restrict__ rz_part,
+                   double *__restrict__ rr_part, const double *__restrict__ cg) {
+  __shared__ double sh[kPsThreads / 64][6];
+  if (cg[kDone] != 0.0) return;
+  double pq[3];
+  ps_part_sums(pq_part, (int)gridDim.x, pq);
+  ps_block_sums<3>(pq, reinterpret_cast<double(*)[3]>(sh));
+  double al[3], s[6] = {0, 0, 0, 0, 0, 0};
+  for (int d = 0; d < 3; ++d) al[d] = pq[d] > 0.0 ? cg[kRZ + 3 * (k & 1) + d] / pq[d] : 0.0;
+  for (int64_t i = blockIdx.x * (int64_t)kPsThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kPsThreads) {
+    const double dg = diag[i];
+    for (int d = 0; d < 3; ++d) {
+      const int64_t j = 3 * i + d;
+      x[j] += al[d] * p[j];
+      const double ri = r[j] - al[d] * q[j], zi = ri / dg;
+      r[j] = ri;
+      z[j] = zi;
+      s[d] += ri * zi;
+      s[3 + d] += ri * ri;
+    }
+  }
+  ps_block_sums<6>(s, sh);
+  ps_store_parts(s, rz_part);
+  ps_store_parts(s + 3, rr_part);
+}
+// interleaved -> component-major
+__global__ void k_ps_deinterleave(int64_t n, const double *__restrict__ x, double *__restrict__ out) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  for (int d = 0; d < 3; ++d) out[d * n + i] = x[3 * i + d];
+}
+
+// out of the body integrals: slots [s0, s0 + gridDim.x) of cg[] from their partial sums
 __global__ void k_ps_finish(int nchunk, int s0, const double *__restrict__ part, double *__restrict__ cg) {
   __shared__ double sh[kPsThreads / 64];
   const int s = s0 + blockIdx.x;
@@ -279,53 +385,6 @@ __global__ void k_ps_finish(int nchunk, int s0, const double *__restrict__ part,
 __global__ void k_fill_zero6(double *out) {
   if (threadIdx.x < 6) out[threadIdx.x] = 0.0;
 }
-__global__ void k_ps_alpha(double *cg) {
-  const int d = threadIdx.x;
-  if (d < 3) cg[kAL + d] = cg[kPQ + d] > 0.0 ? cg[kRZ + d] / cg[kPQ + d] : 0.0;
-}
-// x += alpha p, r -= alpha q, z = r / diag; partial sums of r.r and the new r.z
-// (written to the pq slots, which are free until the next product)
-__global__ void __launch_bounds__(kPsThreads)
-    k_ps_cg_update(int64_t n, const double *__restrict__ cg, const double *__restrict__ diag,
-                   const double *__restrict__ p, const double *__restrict__ q, double *__restrict__ x,
-                   double *__restrict__ r, double *__restrict__ z, double *__restrict__ part) {
-  __shared__ double sh[kPsThreads / 64];
-  const int64_t beg = (int64_t)blockIdx.x * kPsRedChunk, end = min(n, beg + (int64_t)kPsRedChunk);
-  for (int d = 0; d < 3; ++d) {
-    const double al = cg[kAL + d];
-    double rr = 0, rz = 0;
-    for (int64_t i = beg + threadIdx.x; i < end; i += kPsThreads) {
-      const int64_t k = d * n + i;
-      x[k] += al * p[k];
-      const double ri = r[k] - al * q[k];
-      const double zi = ri / diag[i];
-      r[k] = ri;
-      z[k] = zi;
-      rr += ri * ri;
-      rz += ri * zi;
-    }
-    const double s0 = ps_block_sum(rr, sh);
-    if (threadIdx.x == 0) part[(kRR + d) * gridDim.x + blockIdx.x] = s0;
-    const double s1 = ps_block_sum(rz, sh);
-    if (threadIdx.x == 0) part[(kPQ + d) * gridDim.x + blockIdx.x] = s1;
-  }
-}
-// beta = rz_new / rz, rz = rz_new (rz_new was finished into the pq slots)
-__global__ void k_ps_beta(double *cg) {
-  const int d = threadIdx.x;
-  if (d < 3) {
-    const double rzn = cg[kPQ + d];
-    cg[kBE + d] = cg[kRZ + d] > 0.0 ? rzn / cg[kRZ + d] : 0.0;
-    cg[kRZ + d] = rzn;
-  }
-}
-__global__ void k_ps_cg_dir(int64_t n3, int64_t n, const double *__restrict__ cg, const double *__restrict__ z,
-                            double *__restrict__ p) {
-  const int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (k >= n3) return;
-  p[k] = z[k] + cg[kBE + (int)(k / n)] * p[k];
-}
-
 // hydrostatic_pressure (bem_problem.cc:2081-2117): p = -rho g (z - z0)
 __global__ void k_ps_hydrostatic(int64_t n, const double *__restrict__ xyz, double rg, double z0,
                                  double *__restrict__ p) {
@@ -511,11 +570,10 @@ void Engine::ps_setup(int quad_order) {
   ps_alloc(ps.m_val, (size_t)ps.nnz * 8);
   ps_alloc(ps.m_diag, (size_t)n * 8);
   ps_alloc(ps.loc, (size_t)nc * std::max(D * D, 3 * D) * 8);
-  for (DevBuf *b : {&ps.b, &ps.x, &ps.r, &ps.z, &ps.pv, &ps.qv}) ps_alloc(*b, (size_t)3 * n * 8);
+  for (DevBuf *b : {&ps.x, &ps.r, &ps.z, &ps.pv, &ps.qv}) ps_alloc(*b, (size_t)3 * n * 8);
   ps_alloc(ps.cg, kCgLen * 8);
-  const int64_t nblk_red = ps_blocks(n, kPsRedChunk);
   const int64_t nblk_cell = ps_blocks(nc, kPsThreads);
-  ps_alloc(ps.part, (size_t)std::max<int64_t>(kCgLen * nblk_red, 13 * nblk_cell) * 8);
+  ps_alloc(ps.part, (size_t)std::max<int64_t>(12 * kPsParts, 13 * nblk_cell) * 8);
   // assemble the mass matrix
   const unsigned gc = ps_blocks(nc, kPsThreads), gr = ps_blocks(n, kPsThreads);
   if (D == 4) {
@@ -554,56 +612,45 @@ static void ps_rhs(Engine &e, int mode, const double *in1, const double *in2) {
   else
     hipLaunchKernelGGL((k_ps_local<D, 3>), dim3(gc), dim3(kPsThreads), 0, e.stream, s.ncells, s.nq, tab, geom, cd,
                        in1, in2, loc);
-  hipLaunchKernelGGL((k_ps_gather_rhs<D>), dim3(ps_blocks(e.n, kPsThreads)), dim3(kPsThreads), 0, e.stream, e.n,
-                     s.d2c_ptr.as<int32_t>(), s.d2c_cell.as<int32_t>(), s.d2c_loc.as<int8_t>(), loc,
-                     s.b.as<double>());
 }
 
 void Engine::ps_project(int mode, const double *in1, const double *in2, double *out) {
   if (!ps.ready) throw std::runtime_error("post-solve data not set up");
-  if (mesh.dpc == 4)
-    ps_rhs<4>(*this, mode, in1, in2);
-  else
-    ps_rhs<9>(*this, mode, in1, in2);
-  const int nchunk = (int)ps_blocks(n, kPsRedChunk);
   double *cg = ps.cg.as<double>(), *part = ps.part.as<double>();
   double *x = ps.x.as<double>(), *r = ps.r.as<double>(), *z = ps.z.as<double>(), *p = ps.pv.as<double>(),
          *q = ps.qv.as<double>();
   const double *diag = ps.m_diag.as<double>();
-  hipLaunchKernelGGL(k_ps_cg_init, dim3(nchunk), dim3(kPsThreads), 0, stream, n, ps.b.as<double>(), diag, x, r, z,
-                     p, part);
-  hipLaunchKernelGGL(k_ps_finish, dim3(3), dim3(kPsThreads), 0, stream, nchunk, (int)kRZ, part, cg);
-  hipLaunchKernelGGL(k_ps_finish, dim3(3), dim3(kPsThreads), 0, stream, nchunk, (int)kBB, part, cg);
+  // workgroups (and partial sums per component) of every launch
+  const unsigned G = std::min<unsigned>(kPsParts, ps_blocks(n, kPsThreads / kPsLanes));
+  double *pq_part = part, *rr_part = part + 3 * G, *rz_part[2] = {part + 6 * G, part + 9 * G};
+  auto rhs = [&](auto D) {
+    constexpr int DPC = decltype(D)::value;
+    ps_rhs<DPC>(*this, mode, in1, in2);
+    hipLaunchKernelGGL((k_ps_cg_init<DPC>), dim3(G), dim3(kPsThreads), 0, stream, n, ps.d2c_ptr.as<int32_t>(),
+                       ps.d2c_cell.as<int32_t>(), ps.d2c_loc.as<int8_t>(), ps.loc.as<double>(), diag, x, r, z,
+                       rz_part[0], rr_part, cg);
+  };
+  if (mesh.dpc == 4)
+    rhs(std::integral_constant<int, 4>{});
+  else
+    rhs(std::integral_constant<int, 9>{});
   double h[kCgLen];
-  HIPCHK(hipMemcpyAsync(h, cg, sizeof(h), hipMemcpyDeviceToHost, stream));
-  sync();
-  double bb[3] = {h[kBB], h[kBB + 1], h[kBB + 2]};
-  int it = 0;
-  bool done = bb[0] == 0.0 && bb[1] == 0.0 && bb[2] == 0.0;
-  while (!done) {
+  for (int it = 0; ; ) {
     if (it >= kPsMaxIt) throw std::runtime_error("mass-matrix CG did not converge");
-    for (int k = 0; k < kPsCheck; ++k, ++it) {
-      hipLaunchKernelGGL(k_ps_cg_spmv, dim3(nchunk), dim3(kPsThreads), 0, stream, n, ps.m_ptr.as<int32_t>(),
-                         ps.m_col.as<int32_t>(), ps.m_val.as<double>(), p, q, part);
-      hipLaunchKernelGGL(k_ps_finish, dim3(3), dim3(kPsThreads), 0, stream, nchunk, (int)kPQ, part, cg);
-      hipLaunchKernelGGL(k_ps_alpha, dim3(1), dim3(64), 0, stream, cg);
-      hipLaunchKernelGGL(k_ps_cg_update, dim3(nchunk), dim3(kPsThreads), 0, stream, n, cg, diag, p, q, x, r, z,
-                         part);
-      hipLaunchKernelGGL(k_ps_finish, dim3(3), dim3(kPsThreads), 0, stream, nchunk, (int)kRR, part, cg);
-      hipLaunchKernelGGL(k_ps_finish, dim3(3), dim3(kPsThreads), 0, stream, nchunk, (int)kPQ, part, cg);
-      hipLaunchKernelGGL(k_ps_beta, dim3(1), dim3(64), 0, stream, cg);
-      hipLaunchKernelGGL(k_ps_cg_dir, dim3(ps_blocks(3 * n, kPsThreads)), dim3(kPsThreads), 0, stream, 3 * n, n, cg,
-                         z, p);
+    for (int k = 0; k < kPsAhead; ++k, ++it) {
+      hipLaunchKernelGGL(k_ps_cg_dir, dim3(G), dim3(kPsThreads), 0, stream, n, it, ps.m_ptr.as<int32_t>(),
+                         ps.m_col.as<int32_t>(), ps.m_val.as<double>(), z, p, q, rz_part[it & 1], rr_part, pq_part, cg);
+      hipLaunchKernelGGL(k_ps_cg_update, dim3(G), dim3(kPsThreads), 0, stream, n, it, diag, p, q, x, r, z, pq_part,
+                         rz_part[(it + 1) & 1], rr_part, cg);
     }
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(h, cg, sizeof(h), hipMemcpyDeviceToHost, stream));
     sync();
-    done = true;
-    for (int d = 0; d < 3; ++d)
-      if (h[kRR + d] > kPsTol * kPsTol * bb[d]) done = false;
+    if (h[kDone] != 0.0) break;
   }
-  ps.last_iters = it;
-  HIPCHK(hipMemcpyAsync(out, x, (size_t)3 * n * 8, hipMemcpyDeviceToDevice, stream));
+  ps.last_iters = (int)h[kSteps];
+  hipLaunchKernelGGL(k_ps_deinterleave, dim3(ps_blocks(n, kPsThreads)), dim3(kPsThreads), 0, stream, n, x, out);
+  HIPCHK(hipGetLastError());
 }
 
 void Engine::ps_hydrostatic(double gravity, double density, double z0, double *p) {
