@@ -131,155 +131,254 @@ __device__ __forceinline__ T wave_sum(T v) {
 // and singular, 997-1126 bigger blocks).  An item is a (row, entry) pair: the
 // regular rule over the entry's quad points, or the singular rule (Telles or
 // Duffy split, chosen at set-up) over the whole cell when the cell holds a
-// double of the row's node, both in FP64.  One workgroup per row; G lanes
-// (G >= quad points per cell) share an item, a lane per quad point (or every
-// G-th singular point), so that a load of the cell's quad data is one
-// contiguous run.  The group sums the (N, D) parts of the cell's shape
-// functions and adds them, a lane per value, into the row's (N, D) pairs in
-// LDS (columns in tiles of kAsmTile; a row with more columns computes its
-// items once per tile), and the row is stored once, whole.  The FP32
-// operator is this block rounded once (k_round_f32), since in FP32 the
-// difference R = y - x loses ~|x|/|R| ulps and R.n cancels again, which at a
-// radius-4 surface costs 1e-4 of the double-layer product.
+// double of the row's node, both in FP64.  The FP32 operator is this block
+// rounded once (k_round_f32), since in FP32 the difference R = y - x loses
+// ~|x|/|R| ulps and R.n cancels again, which at a radius-4 surface costs 1e-4
+// of the double-layer product.
+//
+// A workgroup owns a tile of kAsmRows rows x kAsmCols columns of one leaf's
+// block: it sums the tile's (N, D) pairs in LDS and stores them once, whole.
+// A thread takes a regular item whose cell has a column in the tile: it runs
+// over the cell's quad points with the shape values' sums in registers (the
+// shape values of the regular rule are the same for every cell, so they are
+// wavefront-uniform loads), and adds 2 DPC values into LDS; the kAsmRows
+// lanes of one cell read the same 64-byte quad point (k_pack_quads).  No sum
+// over lanes is needed.  Singular items, a handful per row, go to a list and
+// run afterwards, 16 lanes each.
+// Bound by FP64 arithmetic: about 45 operations per (row, quad point) for Q2
+// (one reciprocal square root, 18 multiply-adds).  A lane per quad point with
+// the 18 values summed over 16 lanes spent most of its time on those sums,
+// and a row with more columns than its tile computed every item once per
+// tile.  Measured: 393,218 DoFs (Q2, leaf 80, 960 columns per row) 49.6 ->
+// 14.5 ms, 24,578 DoFs (Q1, leaf 20) 2.72 -> 0.60 ms, a 12,376-DoF hull
+// mirrored at its waterline (leaf 20, 12,000 columns per row) 325 -> 14.0 ms.
 // ---------------------------------------------------------------------------
-// Contraction is off in this kernel: near a singular vertex R = X - x_i is
-// ~1e-5 of |X| and R.n cancels to O(r^2), so the singular double-layer
-// entries follow the last bit of X; evaluating X and R exactly as the
-// reference's FEValues path does (separately rounded products and sums) keeps
-// FP64 entries reproducible to rounding.
 template <int G>
 __device__ __forceinline__ double group_sum(double v) {
+  static_assert(G == 16, "one DPP row");
   v += dpp_move<0xB1>(v);   // quad_perm [1,0,3,2]
   v += dpp_move<0x4E>(v);   // quad_perm [2,3,0,1]
   v += dpp_move<0x141>(v);  // row_half_mirror
   v += dpp_move<0x140>(v);  // row_mirror: every lane holds its 16-lane row's sum
-  if constexpr (G >= 32) v += __shfl_xor(v, 16);
-  if constexpr (G >= 64) v += __shfl_xor(v, 32);
   return v;
 }
-constexpr int kAsmTile = 2048;
-template <int G>
-__global__ void __launch_bounds__(256) k_assemble_near(
-    int nleaf, const int *__restrict__ row_beg,
-    const int *__restrict__ rows, const int *__restrict__ col_beg, const int *__restrict__ ent_beg,
-    const int *__restrict__ ent_cell, const uint64_t *__restrict__ ent_mask,
-    const uint8_t *__restrict__ ent_near, const int *__restrict__ ent_colpos,
-    const int64_t *__restrict__ val_beg, const int *__restrict__ cdofs, int dpc, int nq,
-    const int *__restrict__ dbl_ptr, const int *__restrict__ dbl_idx, const double *__restrict__ xyz,
-    const double *__restrict__ qx, const double *__restrict__ qn, const double *__restrict__ qw,
-    const double *__restrict__ qsh, const double *__restrict__ geom, const double *__restrict__ sing,
-    const int *__restrict__ sing_cnt, int sing_stride, double *__restrict__ vals) {
-#pragma clang fp contract(off)
-  using T = double;
-  constexpr int IPB = 256 / G;  // items per workgroup pass
-  __shared__ double acc[2 * kAsmTile];
-  const int lane = (int)(threadIdx.x & (G - 1));
-  const int g = (int)blockIdx.x;  // row g of the leaf-ordered rows
-  int lo = 0, hi = nleaf - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (row_beg[mid] <= g) lo = mid;
-    else hi = mid - 1;
+
+// A quad point as 64 bytes: x, y, z, nx, ny, nz, weight, 0.
+__global__ void k_pack_quads(int64_t n, const double *__restrict__ qx, const double *__restrict__ qn,
+                             const double *__restrict__ qw, double2 *__restrict__ out) {
+  const int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (g >= n) return;
+  out[4 * g] = double2{qx[3 * g], qx[3 * g + 1]};
+  out[4 * g + 1] = double2{qx[3 * g + 2], qn[3 * g]};
+  out[4 * g + 2] = double2{qn[3 * g + 1], qn[3 * g + 2]};
+  out[4 * g + 3] = double2{qw[g], 0.0};
+}
+
+constexpr int kAsmRows = 8, kAsmCols = 512, kAsmThreads = 512;
+constexpr int kAsmStride = kAsmCols + 4;       // doubles per row of the LDS tile's N and D (the padding spreads rows over banks)
+constexpr int kAsmPlane = kAsmRows * kAsmStride;  // N, then D
+constexpr int kAsmList = 256;                  // singular items a tile's list holds; with more, all items are looked over
+
+struct AsmArgs {
+  const int *row_beg, *rows, *col_beg, *cols, *ent_beg, *ent_cell;
+  const uint64_t *ent_mask;
+  const uint8_t *ent_near;
+  const int *ent_colpos;
+  const int64_t *val_beg;
+  int nq;
+  const int *dbl_ptr, *dbl_idx;
+  const double *xyz;
+  const double2 *quads;  // k_pack_quads
+  const double *sh;      // shape values of the regular rule, [nq][DPC]
+  const double *geom, *sing;
+  const int *sing_cnt;
+  int sing_stride;
+  double *vals;
+};
+
+// The local support point of the cell at which it holds a double of the
+// node, or -1.  own: the column of the node's only double (itself), or -1 for
+// a node with several.
+template <int DPC>
+__device__ __forceinline__ int asm_singular(const AsmArgs &a, int node, int own, const int *cp, int cb) {
+  int js = -1;
+  if (own >= 0) {
+#pragma unroll
+    for (int j = DPC - 1; j >= 0; --j) js = cp[j] == own ? j : js;
+    return js;
   }
-  const int leaf = lo;
-  const int r = g - row_beg[leaf], node = rows[g];
-  const int e0 = ent_beg[leaf], e1 = ent_beg[leaf + 1];
-  const int C = col_beg[leaf + 1] - col_beg[leaf];
-  T *out = vals + 2 * (val_beg[leaf] + (int64_t)r * C);
-  const T x0 = (T)xyz[3 * node], x1 = (T)xyz[3 * node + 1], x2 = (T)xyz[3 * node + 2];
-  for (int c0 = 0; c0 < C; c0 += kAsmTile) {
-    const int cw = min(kAsmTile, C - c0);
-    for (int i = (int)threadIdx.x; i < 2 * cw; i += 256) acc[i] = 0.0;
-    __syncthreads();
-    // every lane runs every pass (the group sums need the whole wavefront)
-    for (int eb = e0; eb < e1; eb += IPB) {
-      const int e = eb + (int)(threadIdx.x / G);
-      const bool valid = e < e1;
-      T Nj[9], Dj[9];
-      for (int j = 0; j < 9; ++j) Nj[j] = Dj[j] = T(0);
-      const int *cp = nullptr;
-      if (valid) {
-        const int cell = ent_cell[e];
-        const int *cd = cdofs + (int64_t)cell * dpc;
-        int js = -1;
-        if (ent_near[e]) {
-          for (int j = 0; j < dpc && js < 0; ++j)
-            for (int k = dbl_ptr[node]; k < dbl_ptr[node + 1]; ++k)
-              if (dbl_idx[k] == cd[j]) {
-                js = j;
-                break;
-              }
-        }
-        cp = ent_colpos + (int64_t)e * dpc;
-        if (js < 0) {
-          const int q = lane;
-          if (q < nq && ((ent_mask[e] >> q) & 1)) {
-            const int64_t g = (int64_t)cell * nq + q;
-            const T R0 = qx[3 * g] - x0, R1 = qx[3 * g + 1] - x1, R2 = qx[3 * g + 2] - x2;
-            const T r = dsqrt(R0 * R0 + R1 * R1 + R2 * R2);
-            const T r2 = r * r;
-            const T s = T(1) / (r * T(4 * kPi));
-            const T den = T(-4 * kPi) * r2 * r;
-            const T dn = (R0 / den) * qn[3 * g] + (R1 / den) * qn[3 * g + 1] + (R2 / den) * qn[3 * g + 2];
-            const T wq = qw[g];
-            for (int j = 0; j < dpc; ++j) {
-              const T sh = qsh[g * dpc + j];
-              Nj[j] = dn * sh * wq;
-              Dj[j] = s * sh * wq;
-            }
-          }
-        } else {
-          const double *Gm = geom + (int64_t)cell * dpc * 3;
-          const double *rule = sing + (int64_t)js * sing_stride;
-          const int nsq = sing_cnt[js];
-          const int ps = 1 + 3 * dpc;
-          for (int q = lane; q < nsq; q += G) {
-            const double *pt = rule + q * ps;
-            double X[3] = {0, 0, 0}, a[3] = {0, 0, 0}, b[3] = {0, 0, 0};
-            for (int j = 0; j < dpc; ++j)
-              for (int k = 0; k < 3; ++k) {
-                X[k] += pt[1 + j] * Gm[3 * j + k];
-                a[k] += pt[1 + dpc + j] * Gm[3 * j + k];
-                b[k] += pt[1 + 2 * dpc + j] * Gm[3 * j + k];
-              }
-            const double cr0 = a[1] * b[2] - a[2] * b[1], cr1 = a[2] * b[0] - a[0] * b[2],
-                         cr2 = a[0] * b[1] - a[1] * b[0];
-            const double J = sqrt(cr0 * cr0 + cr1 * cr1 + cr2 * cr2);
-            const double R0 = X[0] - x0, R1 = X[1] - x1, R2 = X[2] - x2;
-            const double r = sqrt(R0 * R0 + R1 * R1 + R2 * R2);
-            const double r2 = r * r;
-            const double s = 1. / (r * 4 * kPi);
-            const double den = -4 * kPi * r2 * r;
-            const double dn = (R0 / den) * (cr0 / J) + (R1 / den) * (cr1 / J) + (R2 / den) * (cr2 / J);
-            const double wq = J * pt[0];
-            for (int j = 0; j < dpc; ++j) {
-              Nj[j] += dn * pt[1 + j] * wq;
-              Dj[j] += s * pt[1 + j] * wq;
-            }
-          }
-        }
+  for (int j = 0; j < DPC && js < 0; ++j)
+    for (int k = a.dbl_ptr[node]; k < a.dbl_ptr[node + 1]; ++k)
+      if (a.dbl_idx[k] == a.cols[cb + cp[j]]) js = j;
+  return js;
+}
+
+// Singular item by the lanes l = 0, L, .. < L of a group: this lane's share
+// of the DPC (N, D) sums.  Contraction is off: near a singular vertex R = X -
+// x_i is ~1e-5 of |X| and R.n cancels to O(r^2), so the singular double-layer
+// entries follow the last bit of X; evaluating X and R exactly as the
+// reference's FEValues path does (separately rounded products and sums) keeps
+// FP64 entries reproducible to rounding.
+template <int DPC>
+__device__ __forceinline__ void asm_singular_points(const AsmArgs &a, int cell, int js, const double *x, int l, int L,
+                                                    double *Nj, double *Dj) {
+#pragma clang fp contract(off)
+  const double *Gm = a.geom + (int64_t)cell * DPC * 3;
+  constexpr int ps = 1 + 3 * DPC;
+  const double *rule = a.sing + (int64_t)js * a.sing_stride;
+  for (int q = l; q < a.sing_cnt[js]; q += L) {
+    const double *pt = rule + q * ps;
+    double X[3] = {0, 0, 0}, t[3] = {0, 0, 0}, b[3] = {0, 0, 0};
+    for (int j = 0; j < DPC; ++j)
+      for (int k = 0; k < 3; ++k) {
+        X[k] += pt[1 + j] * Gm[3 * j + k];
+        t[k] += pt[1 + DPC + j] * Gm[3 * j + k];
+        b[k] += pt[1 + 2 * DPC + j] * Gm[3 * j + k];
       }
+    const double cr0 = t[1] * b[2] - t[2] * b[1], cr1 = t[2] * b[0] - t[0] * b[2], cr2 = t[0] * b[1] - t[1] * b[0];
+    const double J = sqrt(cr0 * cr0 + cr1 * cr1 + cr2 * cr2);
+    const double R0 = X[0] - x[0], R1 = X[1] - x[1], R2 = X[2] - x[2];
+    const double r = sqrt(R0 * R0 + R1 * R1 + R2 * R2);
+    const double r2 = r * r;
+    const double s = 1. / (r * 4 * kPi);
+    const double den = -4 * kPi * r2 * r;
+    const double dn = (R0 / den) * (cr0 / J) + (R1 / den) * (cr1 / J) + (R2 / den) * (cr2 / J);
+    const double wq = J * pt[0];
+    for (int j = 0; j < DPC; ++j) {
+      Nj[j] += dn * pt[1 + j] * wq;
+      Dj[j] += s * pt[1 + j] * wq;
+    }
+  }
+}
+
+template <int DPC>
+__global__ void __launch_bounds__(kAsmThreads, 4) k_assemble_near(int nunits, const int *__restrict__ units, AsmArgs a) {
+  __shared__ double acc[2 * kAsmPlane];
+  __shared__ int list_n, list_row[kAsmList], list_ent[kAsmList], list_js[kAsmList];
+  // neighbouring tiles read the same quad points: each XCD takes a run of them
+  const int per = (nunits + 7) / 8, u = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+  if ((int)(blockIdx.x / 8) >= per || u >= nunits) return;
+  const int leaf = units[3 * u], row0 = units[3 * u + 1], c0 = units[3 * u + 2];
+  const int t = (int)threadIdx.x, ri = t % kAsmRows;
+  const int r0 = a.row_beg[leaf], R = a.row_beg[leaf + 1] - r0;
+  const int e0 = a.ent_beg[leaf], e1 = a.ent_beg[leaf + 1];
+  const int cb = a.col_beg[leaf], C = a.col_beg[leaf + 1] - cb, cw = min(kAsmCols, C - c0);
+  const bool has_row = row0 + ri < R;
+  const int node = a.rows[r0 + min(row0 + ri, R - 1)];
+  const double x[3] = {a.xyz[3 * node], a.xyz[3 * node + 1], a.xyz[3 * node + 2]};
+  int own = -1;
+  if (a.dbl_ptr[node + 1] - a.dbl_ptr[node] == 1) {
+    const int d = a.dbl_idx[a.dbl_ptr[node]];
+    int lo = 0, hi = C - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (a.cols[cb + mid] < d) lo = mid + 1;
+      else hi = mid;
+    }
+    own = a.cols[cb + lo] == d ? lo : -1;
+  }
+  for (int i = t; i < 2 * kAsmPlane; i += kAsmThreads) acc[i] = 0.0;
+  if (t == 0) list_n = 0;
+  __syncthreads();
+  double *arow = acc + ri * kAsmStride;
+  for (int e = e0 + t / kAsmRows; e < e1; e += kAsmThreads / kAsmRows) {
+    const int *cp = a.ent_colpos + (int64_t)e * DPC;
+    int c[DPC];
+    bool any = false;
 #pragma unroll
-      for (int j = 0; j < 9; ++j) {
-        Nj[j] = group_sum<G>(Nj[j]);
-        Dj[j] = group_sum<G>(Dj[j]);
+    for (int j = 0; j < DPC; ++j) {
+      c[j] = cp[j] - c0;
+      any = any || (unsigned)c[j] < (unsigned)cw;
+    }
+    if (!any || !has_row) continue;
+    const int cell = a.ent_cell[e];
+    const int js = a.ent_near[e] ? asm_singular<DPC>(a, node, own, cp, cb) : -1;
+    if (js >= 0) {
+      const int at = atomicAdd(&list_n, 1);
+      if (at < kAsmList) {
+        list_row[at] = ri;
+        list_ent[at] = e;
+        list_js[at] = js;
       }
-      if (valid) {
-        // lane t adds value t of the item's 2 dpc: N of shape function t, or D of t - dpc
-        for (int t = lane; t < 2 * dpc; t += G) {
-          const int j = t < dpc ? t : t - dpc;
-          T v = T(0);
+      continue;
+    }
+    double Nj[DPC], Dj[DPC];
 #pragma unroll
-          for (int k = 0; k < 9; ++k)
-            if (k == j) v = t < dpc ? Nj[k] : Dj[k];
-          const int c = cp[j] - c0;
-          if (c >= 0 && c < cw) atomicAdd(&acc[2 * c + (t < dpc ? 0 : 1)], v);
+    for (int j = 0; j < DPC; ++j) Nj[j] = Dj[j] = 0.0;
+    const uint64_t mask = a.ent_mask[e];
+    const double2 *qd = a.quads + (int64_t)cell * a.nq * 4;
+    // the next point's 64 bytes are loaded before a point is used
+    double2 v0 = qd[0], v1 = qd[1], v2 = qd[2], v3 = qd[3];
+#pragma unroll 2
+    for (int q = 0; q < a.nq; ++q) {
+      const double2 *nx = qd + 4 * min(q + 1, a.nq - 1);
+      const double2 n0 = nx[0], n1 = nx[1], n2 = nx[2], n3 = nx[3];
+      const bool on = (mask >> q) & 1;  // a point of another leaf's list adds zero
+      const double R0 = v0.x - x[0], R1 = v0.y - x[1], R2 = v1.x - x[2];
+      const double r2 = R0 * R0 + R1 * R1 + R2 * R2;
+      const double inv = rsqrt(on ? r2 : 1.0);
+      const double D = on ? v3.x * inv * (1.0 / (4.0 * kPi)) : 0.0;
+      const double N = -(R0 * v1.y + R1 * v2.x + R2 * v2.y) * (inv * inv) * D;
+#pragma unroll
+      for (int j = 0; j < DPC; ++j) {
+        const double s = a.sh[q * DPC + j];
+        Nj[j] += N * s;
+        Dj[j] += D * s;
+      }
+      v0 = n0, v1 = n1, v2 = n2, v3 = n3;
+    }
+#pragma unroll
+    for (int j = 0; j < DPC; ++j)
+      if ((unsigned)c[j] < (unsigned)cw) {
+        atomicAdd(arow + c[j], Nj[j]);
+        atomicAdd(arow + kAsmPlane + c[j], Dj[j]);
+      }
+  }
+  __syncthreads();
+  // the singular items, 16 lanes each (every lane runs every pass: the sums
+  // need the whole group)
+  const int l = t & 15;
+  const bool listed = list_n <= kAsmList;
+  const int ns = listed ? list_n : kAsmRows * (e1 - e0);
+  for (int i0 = 0; i0 < ns; i0 += kAsmThreads / 16) {
+    const int i = i0 + t / 16;
+    bool valid = i < ns;
+    int row = 0, e = e0, js = -1;
+    if (valid) {
+      if (listed) {
+        row = list_row[i], e = list_ent[i], js = list_js[i];
+      } else {
+        row = i % kAsmRows, e = e0 + i / kAsmRows;
+        if (row0 + row < R && a.ent_near[e])
+          js = asm_singular<DPC>(a, a.rows[r0 + row0 + row], -1, a.ent_colpos + (int64_t)e * DPC, cb);
+        valid = js >= 0;
+      }
+    }
+    double Nj[DPC], Dj[DPC];
+#pragma unroll
+    for (int j = 0; j < DPC; ++j) Nj[j] = Dj[j] = 0.0;
+    if (valid) {
+      const int nd = a.rows[r0 + row0 + row];
+      const double xi[3] = {a.xyz[3 * nd], a.xyz[3 * nd + 1], a.xyz[3 * nd + 2]};
+      asm_singular_points<DPC>(a, a.ent_cell[e], js, xi, l, 16, Nj, Dj);
+    }
+#pragma unroll
+    for (int j = 0; j < DPC; ++j) {
+      const double N = group_sum<16>(Nj[j]), D = group_sum<16>(Dj[j]);
+      if (valid && l == j) {
+        const int c = a.ent_colpos[(int64_t)e * DPC + j] - c0;
+        if ((unsigned)c < (unsigned)cw) {
+          atomicAdd(acc + row * kAsmStride + c, N);
+          atomicAdd(acc + kAsmPlane + row * kAsmStride + c, D);
         }
       }
     }
-    __syncthreads();
-    for (int i = (int)threadIdx.x; i < 2 * cw; i += 256) out[2 * c0 + i] = acc[i];
-    __syncthreads();
+  }
+  __syncthreads();
+  for (int r = t / 64; r < min(kAsmRows, R - row0); r += kAsmThreads / 64) {
+    double2 *out = reinterpret_cast<double2 *>(a.vals + 2 * (a.val_beg[leaf] + (int64_t)(row0 + r) * C + c0));
+    const double *in = acc + r * kAsmStride;
+    for (int i = t & 63; i < cw; i += 64) out[i] = double2{in[i], in[kAsmPlane + i]};
   }
 }
 
@@ -2592,25 +2691,32 @@ void Engine::assemble_near(bool want_f32) {
 
   const int64_t nv = std::max<int64_t>(near.nnz, 1) * 2;
   alloc(f64.vals, (size_t)nv * sizeof(double));
-  HIPCHK(hipMemsetAsync(f64.vals.p, 0, f64.vals.bytes, stream));
-  const int64_t total = near.work_beg.back();
-  if (near.nleaf > 0 && total > 0) {
-    // G lanes per item: the quad points per cell (at most 64, the entry masks' width), rounded up
+  DevBuf d_quads, d_units;  // freed at the end, after the stream has run
+  if (near.nleaf > 0 && near.nnz > 0) {
     if (nq > 64 || dpc > 9) throw std::runtime_error("near assembly: more than 64 quad points or 9 DoFs per cell");
-    const int G = nq <= 16 ? 16 : nq <= 32 ? 32 : 64;
-    const unsigned grid = (unsigned)near.row_beg[near.nleaf];  // a workgroup per row
-#define PBFMM_ASM(GG)                                                                                              \
-  hipLaunchKernelGGL(k_assemble_near<GG>, dim3(grid), dim3(256), 0, stream, near.nleaf,                            \
-                     d_row_beg.as<int>(), d_rows.as<int>(), d_col_beg.as<int>(), d_ent_beg.as<int>(),                \
-                     d_ent_cell.as<int>(), d_ent_mask.as<uint64_t>(), d_ent_near.as<uint8_t>(),                    \
-                     d_ent_colpos.as<int>(), d_val_beg.as<int64_t>(), d_cdofs.as<int>(), dpc, nq,                  \
-                     d_dbl_ptr.as<int>(), d_dbl_idx.as<int>(), d_xyz.as<double>(), f64.qx.as<double>(),            \
-                     f64.qn.as<double>(), f64.qw.as<double>(), f64.qsh.as<double>(), d_geom.as<double>(),          \
-                     d_sing.as<double>(), d_scnt.as<int>(), maxq * ps, f64.vals.as<double>())
-    if (G == 16) PBFMM_ASM(16);
-    else if (G == 32) PBFMM_ASM(32);
-    else PBFMM_ASM(64);
-#undef PBFMM_ASM
+    // tiles of kAsmRows rows x kAsmCols columns of every leaf's block
+    std::vector<int32_t> units;
+    for (int l = 0; l < near.nleaf; ++l) {
+      const int R = near.row_beg[l + 1] - near.row_beg[l], C = near.col_beg[l + 1] - near.col_beg[l];
+      for (int r = 0; r < R; r += kAsmRows)
+        for (int c = 0; c < C; c += kAsmCols) units.insert(units.end(), {l, r, c});
+    }
+    up(d_units, units);
+    const int64_t npts = mesh.ncells * nq;
+    alloc(d_quads, (size_t)npts * 64);
+    hipLaunchKernelGGL(k_pack_quads, dim3(nblk(npts, 256)), dim3(256), 0, stream, npts, f64.qx.as<double>(),
+                       f64.qn.as<double>(), f64.qw.as<double>(), d_quads.as<double2>());
+    AsmArgs a{d_row_beg.as<int>(), d_rows.as<int>(), d_col_beg.as<int>(), d_cols.as<int>(), d_ent_beg.as<int>(),
+              d_ent_cell.as<int>(), d_ent_mask.as<uint64_t>(), d_ent_near.as<uint8_t>(), d_ent_colpos.as<int>(),
+              d_val_beg.as<int64_t>(), nq, d_dbl_ptr.as<int>(), d_dbl_idx.as<int>(), d_xyz.as<double>(),
+              d_quads.as<double2>(), f64.qsh.as<double>(), d_geom.as<double>(), d_sing.as<double>(),
+              d_scnt.as<int>(), maxq * ps, f64.vals.as<double>()};
+    const int nu = (int)(units.size() / 3);
+    const dim3 grid((unsigned)((nu + 7) / 8 * 8));
+    if (dpc == 4)
+      hipLaunchKernelGGL(k_assemble_near<4>, grid, dim3(kAsmThreads), 0, stream, nu, d_units.as<int>(), a);
+    else
+      hipLaunchKernelGGL(k_assemble_near<9>, grid, dim3(kAsmThreads), 0, stream, nu, d_units.as<int>(), a);
     HIPCHK(hipGetLastError());
   }
   // the operator's single-value near field (N on Neumann, -D on Dirichlet columns)
