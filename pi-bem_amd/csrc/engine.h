@@ -141,9 +141,9 @@ struct Engine {
   int nprec = 0;
   std::vector<int64_t> pinv_beg;
   std::vector<int32_t> prow_beg, prows;
-  DevBuf d_pinv_beg, d_pvec_beg[2], d_pinv[2], d_ptmp, d_ptmp2, d_prow_beg, d_prows, d_prow_blk;
+  DevBuf d_pvec_beg[2], d_pinv[2], d_ptmp, d_ptmp2, d_prow_beg, d_prows, d_prow_blk;
   void build_preconditioner();
-  std::vector<int32_t> prec_pos;  // block-ordered row -> leaf-ordered near row
+  DevBuf d_ppos;  // block-ordered row -> leaf-ordered near row
   void prec_blocks(std::vector<double> &blk);
   void apply_prec(const double *v, double *z, int R = 1);  // R right-hand sides, n apart
   DevBuf d_rhs_sum;  // per right-hand side sums of the lockstep operator's mean term

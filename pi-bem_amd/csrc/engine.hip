@@ -10,7 +10,6 @@
 #include <cstring>
 #include <stdexcept>
 #include <string>
-#include <thread>
 
 #include "engine.h"
 
@@ -1863,37 +1862,48 @@ __global__ void k_set_constrained(int64_t n, const uint8_t *__restrict__ is_c, c
 // Block g of the preconditioner (several leaves): row r of block g is
 // the leaf-ordered near row pos[r] (its leaf row_leaf[pos]); an entry is the
 // operator's near value when the column is in that leaf's column list, else
-// zero.
-__global__ void k_extract_groups(const int *__restrict__ grp_beg, const int *__restrict__ pos,
-                                 const int *__restrict__ row_leaf, const int *__restrict__ row_beg,
-                                 const int *__restrict__ rows, const int *__restrict__ col_beg,
-                                 const int *__restrict__ cols, const int64_t *__restrict__ val_beg,
-                                 const double *__restrict__ vals, const uint8_t *__restrict__ dir,
-                                 const double *__restrict__ alpha, const int64_t *__restrict__ blk_beg,
-                                 double *__restrict__ out) {
-  const int g = blockIdx.x;
-  const int g0 = grp_beg[g], R = grp_beg[g + 1] - g0;
-  for (int idx = threadIdx.x; idx < R * R; idx += blockDim.x) {
-    const int r = idx / R, c = idx - r * R;
-    const int pr = pos[g0 + r], leaf = row_leaf[pr];
-    const int node_r = rows[pr], node_c = rows[pos[g0 + c]];
-    const int cb = col_beg[leaf], C = col_beg[leaf + 1] - cb;
-    int lo = 0, hi = C - 1, at = -1;
-    while (lo <= hi) {
-      const int mid = (lo + hi) >> 1;
-      const int v = cols[cb + mid];
-      if (v == node_c) { at = mid; break; }
-      if (v < node_c) lo = mid + 1;
-      else hi = mid - 1;
-    }
-    double v = 0.0;
-    if (at >= 0) {
-      const double *q = vals + 2 * (val_beg[leaf] + (int64_t)(pr - row_beg[leaf]) * C + at);
-      v = dir[node_c] ? -q[1] : q[0];
-    }
-    if (r == c && !dir[node_r]) v += alpha[node_r];
-    out[blk_beg[g] + idx] = v;
+// zero, with alpha on the diagonal of Neumann rows.  A constrained row (is_c)
+// is src(i) - sum c_ij src(j) instead (constrained_matrix.h:109-121).
+struct PrecArgs {
+  const int *grp_beg, *pos, *row_leaf, *row_beg, *rows, *col_beg, *cols;
+  const int64_t *val_beg;
+  const double *vals;
+  const uint8_t *dir;
+  const double *alpha;
+  const uint8_t *is_c;  // null: no constraints
+  const int *c_ptr, *c_idx;
+  const double *c_val;
+};
+__device__ __forceinline__ double prec_entry(const PrecArgs &a, int g0, int r, int c) {
+  const int pr = a.pos[g0 + r], node_r = a.rows[pr], node_c = a.rows[a.pos[g0 + c]];
+  if (a.is_c && a.is_c[node_r]) {
+    double v = r == c ? 1.0 : 0.0;
+    for (int k = a.c_ptr[node_r]; k < a.c_ptr[node_r + 1]; ++k)
+      if (a.c_idx[k] == node_c) v -= a.c_val[k];
+    return v;
   }
+  const int leaf = a.row_leaf[pr], cb = a.col_beg[leaf], C = a.col_beg[leaf + 1] - cb;
+  int lo = 0, hi = C - 1, at = -1;
+  while (lo <= hi) {
+    const int mid = (lo + hi) >> 1;
+    const int v = a.cols[cb + mid];
+    if (v == node_c) { at = mid; break; }
+    if (v < node_c) lo = mid + 1;
+    else hi = mid - 1;
+  }
+  double v = 0.0;
+  if (at >= 0) {
+    const double *q = a.vals + 2 * (a.val_beg[leaf] + (int64_t)(pr - a.row_beg[leaf]) * C + at);
+    v = a.dir[node_c] ? -q[1] : q[0];
+  }
+  if (r == c && !a.dir[node_r]) v += a.alpha[node_r];
+  return v;
+}
+__global__ void k_extract_groups(PrecArgs a, const int64_t *__restrict__ blk_beg, double *__restrict__ out) {
+  const int g = blockIdx.x;
+  const int g0 = a.grp_beg[g], R = a.grp_beg[g + 1] - g0;
+  for (int idx = threadIdx.x; idx < R * R; idx += blockDim.x)
+    out[blk_beg[g] + idx] = prec_entry(a, g0, idx / R, idx % R);
 }
 
 // The inverse blocks are stored in column vectors of 16 bytes (PT = double:
@@ -1916,6 +1926,124 @@ __device__ __forceinline__ void pinv_load(const float *p, double *a) {
 __device__ __forceinline__ void pinv_load(const double *p, double *a) {
   const double2 u = *reinterpret_cast<const double2 *>(p);
   a[0] = u.x, a[1] = u.y;
+}
+
+// Inverts the preconditioner's blocks, a workgroup each: the block is
+// assembled where it is inverted (LDS, blocks of at most kInvRows rows; the
+// others, leaves larger than the row cap, in scratch memory), by Gauss-Jordan
+// in place with partial pivoting, FP64, and stored in both copies' layouts.
+// A block whose pivot vanishes (e.g. unconstrained double nodes) becomes
+// diagonal scaling.  A step finds the pivot (one wavefront), swaps and scales
+// the pivot row, and updates every other row: bound by LDS, 2 x 8 R^2 bytes
+// per step.  On the host this took a Gauss-Jordan per thread on 16 threads
+// and both copies over PCIe: 98,306 DoFs (Q2, leaf 80, blocks of up to 128
+// rows) 89 -> 2.1 ms for the whole preconditioner, 1,538 DoFs 1.5 -> 0.25 ms.
+constexpr int kInvRows = 128, kInvThreads = 1024;
+template <bool LDS>
+__global__ void __launch_bounds__(kInvThreads) k_invert_blocks(PrecArgs a, const int64_t *__restrict__ blk_beg,
+                                                               double *__restrict__ scratch,
+                                                               const int64_t *__restrict__ beg64,
+                                                               double *__restrict__ inv64,
+                                                               const int64_t *__restrict__ beg32,
+                                                               float *__restrict__ inv32, int max_rows,
+                                                               double *__restrict__ row_scratch) {
+  extern __shared__ double smem[];
+  __shared__ double s_scale, s_d;
+  __shared__ int s_piv, s_bad;
+  const int g = blockIdx.x, t = (int)threadIdx.x;
+  const int g0 = a.grp_beg[g], R = a.grp_beg[g + 1] - g0;
+  if ((R <= kInvRows) != LDS) return;
+  const int LD = LDS ? (R | 1) : R;
+  // the block, then the scaled pivot row, the pivot column and the pivots
+  double *A = LDS ? smem : scratch + blk_beg[g];
+  double *prow = LDS ? smem + R * LD : row_scratch + (int64_t)g * 3 * max_rows, *pcol = prow + R;
+  int *piv = reinterpret_cast<int *>(pcol + R);
+  for (int i = t; i < R * R; i += kInvThreads) A[(i / R) * LD + i % R] = prec_entry(a, g0, i / R, i % R);
+  if (t == 0) s_bad = 0;
+  __syncthreads();
+  {
+    double m = 0.0;
+    for (int i = t; i < R * R; i += kInvThreads) m = fmax(m, fabs(A[(i / R) * LD + i % R]));
+    for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
+    if (t < 64) prow[0] = 0.0;
+    __syncthreads();
+    // 16 wavefronts' maxima, one after the other's store
+    for (int w = 0; w < kInvThreads / 64; ++w) {
+      if (t == 64 * w) prow[0] = fmax(prow[0], m);
+      __syncthreads();
+    }
+    if (t == 0) s_scale = prow[0];
+  }
+  __syncthreads();
+  for (int c = 0; c < R; ++c) {
+    if (t < 64) {  // the first row of the largest entry of column c, from the diagonal down
+      double m = -1.0;
+      int at = c;
+      for (int r = c + t; r < R; r += 64) {
+        const double v = fabs(A[r * LD + c]);
+        if (v > m) m = v, at = r;
+      }
+      for (int o = 1; o < 64; o <<= 1) {
+        const double m2 = __shfl_xor(m, o, 64);
+        const int a2 = __shfl_xor(at, o, 64);
+        if (m2 > m || (m2 == m && a2 < at)) m = m2, at = a2;
+      }
+      if (t == 0) {
+        s_piv = piv[c] = at;
+        s_bad = !(m > 1e-13 * s_scale);
+        s_d = 1.0 / A[at * LD + c];
+      }
+    }
+    __syncthreads();
+    if (s_bad) break;
+    const int p = s_piv;
+    const double d = s_d;
+    // row c takes the scaled pivot row, the pivot's place the old row c
+    for (int k = t; k < R; k += kInvThreads) {
+      const double vp = A[p * LD + k], vc = A[c * LD + k];
+      prow[k] = k == c ? d : vp * d;
+      if (p != c) A[p * LD + k] = vc;
+      A[c * LD + k] = k == c ? d : vp * d;
+    }
+    __syncthreads();
+    for (int r = t; r < R; r += kInvThreads) pcol[r] = r == c ? 0.0 : A[r * LD + c];
+    __syncthreads();
+    constexpr int W = 128;  // columns side by side
+    for (int k = t % W; k < R; k += W) {
+      const double pk = prow[k];
+      for (int r = t / W; r < R; r += kInvThreads / W)
+        if (r != c) A[r * LD + k] = (k == c ? 0.0 : A[r * LD + k]) - pcol[r] * pk;
+    }
+    __syncthreads();
+  }
+  const bool bad = s_bad;
+  if (!bad && t == 0) {
+    // the row swaps as column swaps of the inverse, last first: column j of it is column perm[j] of A
+    int *perm = reinterpret_cast<int *>(prow);
+    for (int j = 0; j < R; ++j) perm[j] = j;
+    for (int c = R - 1; c >= 0; --c) {
+      const int q = perm[c];
+      perm[c] = perm[piv[c]];
+      perm[piv[c]] = q;
+    }
+  }
+  __syncthreads();
+  const int *perm = reinterpret_cast<const int *>(prow);
+  const int C4 = (R + 3) / 4 * 4, C2 = (R + 1) / 2 * 2;
+  for (int i = t; i < R * C4; i += kInvThreads) {
+    const int r = i / C4, c = i % C4;
+    double v = 0.0;
+    if (c < R) {
+      if (!bad) {
+        v = A[r * LD + perm[c]];
+      } else if (r == c) {
+        const double d = prec_entry(a, g0, r, r);
+        v = d != 0.0 ? 1.0 / d : 1.0;
+      }
+    }
+    if (c < C2) inv64[beg64[g] + pinv_vec_index<double>(r, c, R)] = v;
+    inv32[beg32[g] + pinv_vec_index<float>(r, c, R)] = (float)v;
+  }
 }
 
 // z[rows of block] = Pinv_block . v[rows of block]; one thread per block-ordered
@@ -3515,76 +3643,31 @@ void Engine::compute_rhs(const double *gvec, double *rhs) {
   HIPCHK(hipGetLastError());
 }
 
-// Gauss-Jordan inverse with partial pivoting of a row-major R x R block in
-// place; returns false when a pivot vanishes.
-static bool invert_block(std::vector<double> &A, int R) {
-  std::vector<double> I((size_t)R * R, 0.0);
-  for (int i = 0; i < R; ++i) I[(size_t)i * R + i] = 1.0;
-  double scale = 0;
-  for (double x : A) scale = std::max(scale, std::fabs(x));
-  for (int c = 0; c < R; ++c) {
-    int piv = c;
-    for (int r = c + 1; r < R; ++r)
-      if (std::fabs(A[(size_t)r * R + c]) > std::fabs(A[(size_t)piv * R + c])) piv = r;
-    if (!(std::fabs(A[(size_t)piv * R + c]) > 1e-13 * scale)) return false;
-    if (piv != c)
-      for (int k = 0; k < R; ++k) {
-        std::swap(A[(size_t)piv * R + k], A[(size_t)c * R + k]);
-        std::swap(I[(size_t)piv * R + k], I[(size_t)c * R + k]);
-      }
-    const double d = 1.0 / A[(size_t)c * R + c];
-    for (int k = 0; k < R; ++k) {
-      A[(size_t)c * R + k] *= d;
-      I[(size_t)c * R + k] *= d;
-    }
-    for (int r = 0; r < R; ++r) {
-      if (r == c) continue;
-      const double f = A[(size_t)r * R + c];
-      if (f == 0.0) continue;
-      for (int k = 0; k < R; ++k) {
-        A[(size_t)r * R + k] -= f * A[(size_t)c * R + k];
-        I[(size_t)r * R + k] -= f * I[(size_t)c * R + k];
-      }
-    }
-  }
-  A.swap(I);
-  return true;
+// What the preconditioner's kernels read of this handle.
+static PrecArgs prec_args(const Engine &e) {
+  const bool c = e.have_constraints;
+  return PrecArgs{e.d_prow_beg.as<int>(),    e.d_ppos.as<int>(),         e.d_row_leaf.as<int>(), e.d_row_beg.as<int>(),
+                  e.d_rows.as<int>(),        e.d_col_beg.as<int>(),      e.d_cols.as<int>(),     e.d_val_beg.as<int64_t>(),
+                  e.f64.vals.as<double>(),   e.d_dir.as<uint8_t>(),      e.d_alpha.as<double>(),
+                  c ? e.d_c_is.as<uint8_t>() : nullptr, c ? e.d_c_ptr.as<int>() : nullptr,
+                  c ? e.d_c_idx.as<int>() : nullptr,    c ? e.d_c_val.as<double>() : nullptr};
 }
 
 // The preconditioner's blocks before inversion, row-major, block g at
 // pinv_beg[g] over the rows prows[prow_beg[g] ..): the near field with -D in
-// Dirichlet and N in Neumann columns, alpha on the diagonal of Neumann rows
-// (k_extract_groups, on the GPU from the assembled FP64 near field), and
-// constrained rows replaced by their constraint row src(i) - sum c_ij src(j)
-// (constrained_matrix.h:109-121), on the host.
+// Dirichlet and N in Neumann columns, alpha on the diagonal of Neumann rows,
+// constrained rows replaced (prec_entry, from the assembled FP64 near field).
 void Engine::prec_blocks(std::vector<double> &blk) {
   blk.assign(pinv_beg.empty() ? 0 : pinv_beg[nprec], 0.0);
   if (nprec <= 0) return;
-  DevBuf d_pos, d_raw;
-  up(d_pos, prec_pos);
+  DevBuf d_raw, d_beg;
   alloc(d_raw, std::max<size_t>(blk.size(), 1) * 8);
-  hipLaunchKernelGGL(k_extract_groups, dim3(nprec), dim3(256), 0, stream, d_prow_beg.as<int>(), d_pos.as<int>(),
-                     d_row_leaf.as<int>(), d_row_beg.as<int>(), d_rows.as<int>(), d_col_beg.as<int>(),
-                     d_cols.as<int>(), d_val_beg.as<int64_t>(), f64.vals.as<double>(), d_dir.as<uint8_t>(),
-                     d_alpha.as<double>(), d_pinv_beg.as<int64_t>(), d_raw.as<double>());
+  up(d_beg, pinv_beg);
+  hipLaunchKernelGGL(k_extract_groups, dim3(nprec), dim3(256), 0, stream, prec_args(*this), d_beg.as<int64_t>(),
+                     d_raw.as<double>());
   HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpyAsync(blk.data(), d_raw.p, blk.size() * 8, hipMemcpyDeviceToHost, stream));
-  sync();  // d_pos and d_raw are freed on return
-  if (!have_constraints) return;
-  for (int g = 0; g < nprec; ++g) {
-    const int r0 = prow_beg[g], R = prow_beg[g + 1] - r0;
-    double *A = blk.data() + pinv_beg[g];
-    for (int r = 0; r < R; ++r) {
-      const int i = prows[r0 + r];
-      if (!hc_is[i]) continue;
-      for (int c = 0; c < R; ++c) A[(size_t)r * R + c] = (c == r) ? 1.0 : 0.0;
-      for (int k = hc_ptr[i]; k < hc_ptr[i + 1]; ++k) {
-        const int j = hc_idx[k];
-        for (int c = 0; c < R; ++c)
-          if (prows[r0 + c] == j) A[(size_t)r * R + c] -= hc_val[k];
-      }
-    }
-  }
+  sync();  // d_raw is freed on return
 }
 
 void Engine::build_preconditioner() {
@@ -3630,11 +3713,10 @@ void Engine::build_preconditioner() {
     max_leaf_rows = std::max(max_leaf_rows, (int)R);
     for (int r = prow_beg[g]; r < prow_beg[g + 1]; ++r) prow_blk[r] = g;
   }
-  up(d_pinv_beg, pinv_beg);
   up(d_prow_beg, prow_beg);
   up(d_prows, prows);
   up(d_prow_blk, prow_blk);
-  prec_pos = pos;
+  up(d_ppos, pos);
   // per copy f (0 FP64 pairs, 1 FP32 quads) the blocks' offsets
   std::vector<int64_t> pvb[2];
   for (int f = 0; f < 2; ++f) {
@@ -3646,46 +3728,32 @@ void Engine::build_preconditioner() {
     }
     up(d_pvec_beg[f], pvb[f]);
   }
-  std::vector<double> b64((size_t)pvb[0][nprec], 0.0);
-  std::vector<float> b32((size_t)pvb[1][nprec], 0.0f);
-  std::vector<double> blk;
-  prec_blocks(blk);
-  // invert the blocks on host threads
-  auto invert_range = [&](int g_lo, int g_hi) {
-    std::vector<double> A;
-    for (int g = g_lo; g < g_hi; ++g) {
-      const int R = prow_beg[g + 1] - prow_beg[g];
-      A.assign(blk.begin() + pinv_beg[g], blk.begin() + pinv_beg[g + 1]);
-      std::vector<double> keep = A;
-      if (!invert_block(A, R)) {
-        // singular block (e.g. unconstrained double nodes): diagonal scaling
-        for (int r = 0; r < R; ++r)
-          for (int c = 0; c < R; ++c) {
-            const double d = keep[(size_t)r * R + r];
-            A[(size_t)r * R + c] = (r == c) ? (d != 0.0 ? 1.0 / d : 1.0) : 0.0;
-          }
-      }
-      for (int r = 0; r < R; ++r)
-        for (int c = 0; c < R; ++c) {
-          const double a = A[(size_t)r * R + c];
-          b64[pvb[0][g] + pinv_vec_index<double>(r, c, R)] = a;
-          b32[pvb[1][g] + pinv_vec_index<float>(r, c, R)] = (float)a;
-        }
-    }
-  };
-  const int nth = (int)std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
-  if (nprec < 64 || nth == 1) {
-    invert_range(0, nprec);
-  } else {
-    std::vector<std::thread> th;
-    for (int k = 0; k < nth; ++k)
-      th.emplace_back(invert_range, (int)((int64_t)nprec * k / nth), (int)((int64_t)nprec * (k + 1) / nth));
-    for (auto &x : th) x.join();
-  }
-  up(d_pinv[0], b64);
-  up(d_pinv[1], b32);
+  alloc(d_pinv[0], (size_t)pvb[0][nprec] * 8);
+  alloc(d_pinv[1], (size_t)pvb[1][nprec] * 4);
   alloc(d_ptmp, n * 8);
   alloc(d_ptmp2, n * 8);
+  if (nprec > 0) {
+    const PrecArgs a = prec_args(*this);
+    const int Rl = std::min(max_leaf_rows, kInvRows);  // the largest block inverted in LDS
+    const size_t lds = ((size_t)Rl * (Rl | 1) + 2 * Rl) * 8 + (size_t)Rl * 4 + 16;
+    HIPCHK(hipFuncSetAttribute((const void *)k_invert_blocks<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)lds));
+    hipLaunchKernelGGL(k_invert_blocks<true>, dim3(nprec), dim3(kInvThreads), lds, stream, a, nullptr, nullptr,
+                       d_pvec_beg[0].as<int64_t>(), d_pinv[0].as<double>(), d_pvec_beg[1].as<int64_t>(),
+                       d_pinv[1].as<float>(), 0, nullptr);
+    HIPCHK(hipGetLastError());
+    if (max_leaf_rows > kInvRows) {
+      DevBuf raw, beg, row;
+      alloc(raw, (size_t)pinv_beg[nprec] * 8);
+      up(beg, pinv_beg);
+      alloc(row, (size_t)nprec * 3 * max_leaf_rows * 8);
+      hipLaunchKernelGGL(k_invert_blocks<false>, dim3(nprec), dim3(kInvThreads), 0, stream, a, beg.as<int64_t>(),
+                         raw.as<double>(), d_pvec_beg[0].as<int64_t>(), d_pinv[0].as<double>(),
+                         d_pvec_beg[1].as<int64_t>(), d_pinv[1].as<float>(), max_leaf_rows, row.as<double>());
+      HIPCHK(hipGetLastError());
+      sync();  // raw, beg and row are freed here
+    }
+  }
   have_prec = true;
 }
 
