@@ -351,8 +351,9 @@ int pbfmm_set_spmv_kernel(pbfmm_handle *h, int32_t precision, int32_t kernel);
  * the library, beside the whole FMM; 24 and 28: plans 8 and 12 with the
  * second stream forked after the M2M levels, beside M2L onwards; 56 and 60:
  * plans 24 and 28 with M2P following the SpMV on the second stream; 88 and
- * 92: with M2P before the SpMV there; -1 times them all again on the next
- * application).  For tests and tuning.  No
+ * 92: with M2P before the SpMV there; -1 times plans 0, 3, 5, 8, 24, 56 and
+ * 92 on the next application).  Without a call the plan is timed after the
+ * first 64 applications.  For tests and tuning.  No
  * counterpart in the reference. */
 int pbfmm_set_side_fusion(pbfmm_handle *h, int32_t precision, int32_t mode);
 
@@ -377,10 +378,11 @@ int pbfmm_tuning_state(pbfmm_handle *h, int32_t *state);
  * reference): the preconditioner and the operator application of one Arnoldi
  * step of pbfmm_gmres_dev / pbfmm_solve_system run from a fixed input into a
  * fixed output, so the launches can be captured once and replayed.  -1
- * (default): the first steps of each precision capture the graph and time
- * three replays against three direct runs, and the faster is kept; 0 direct
- * launches only; 1 graph replays.  A graph is captured again whenever a
- * choice or buffer it holds changes.  Batch handles and many right-hand
+ * (default): 16 steps after the launch plan is timed (in the next steps after
+ * a call with -1) the graph is captured and three replays are timed against
+ * three direct runs, and the faster is kept; 0 direct launches only; 1 graph
+ * replays.  A graph is captured again whenever a choice or buffer it holds
+ * changes.  Batch handles and many right-hand
  * sides launch directly. */
 int pbfmm_set_graph_mode(pbfmm_handle *h, int32_t mode);
 /* The timing behind the graph choice, ms per step: [0] [1] FP64 direct /

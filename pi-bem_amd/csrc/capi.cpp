@@ -1053,6 +1053,7 @@ int pbfmm_set_spmv_kernel(pbfmm_handle *h, int32_t precision, int32_t kernel) {
     if (precision == PBFMM_MIXED && !h->eng.have_f32)
       return fail(h, PBFMM_ERR_STATE, "set_spmv_kernel: handle was not created with PBFMM_MIXED");
     const int pi = precision == PBFMM_MIXED ? 1 : 0;
+    if (pi == 1 && kernel >= 3 && kernel <= 5) h->eng.ensure_row_pairs();
     h->eng.spmv_variant[pi][0] = kernel;
     h->eng.spmv_variant[pi][1] = kernel % 3;
     return PBFMM_OK;
@@ -1065,7 +1066,9 @@ int pbfmm_set_side_fusion(pbfmm_handle *h, int32_t precision, int32_t mode) {
     return fail(h, PBFMM_ERR_ARG, "set_side_fusion: plan must be -1, 0, 1, 2, 3, 4, 5, 8, 12, 24, 28, 56, 60, 88 or 92");
   if (precision != PBFMM_FP64 && precision != PBFMM_MIXED)
     return fail(h, PBFMM_ERR_ARG, "set_side_fusion: unknown precision");
-  h->eng.side_fusion[precision == PBFMM_MIXED ? 1 : 0] = mode;
+  const int pi = precision == PBFMM_MIXED ? 1 : 0;
+  h->eng.side_fusion[pi] = mode;
+  if (mode == -1) h->eng.plan_apps[pi] = Engine::kPlanAfter;  // timed on the next application
   return PBFMM_OK;
 }
 
@@ -1091,6 +1094,7 @@ int pbfmm_set_graph_mode(pbfmm_handle *h, int32_t mode) {
   Engine &e = h->eng;
   e.graph_enabled = mode != 0;
   e.graph_use[0] = e.graph_use[1] = mode;
+  e.graph_steps[0] = e.graph_steps[1] = Engine::kGraphAfter;  // -1: timed in the next steps
   return PBFMM_OK;
 }
 

@@ -181,8 +181,8 @@ struct Engine {
   // M2M level and M2P beside M2L, 3 both beside M2L)
   template <typename T>
   void matvec_fused(const double *x, double *out, double *dst, int side);
-  // side fusion mode per precision ([0] FP64, [1] FP32): -1 until timed on
-  // first use, then the fastest of the plans kPlans
+  // side fusion mode per precision ([0] FP64, [1] FP32): -1 until timed, then
+  // the fastest of plan 0 and kTimedPlans
   // Plans are bit sets: bits 0-1 the side placement above (0..3); bit 2
   // (plans 4, 5 with placements 0, 1) M2L into per-pair slots and a
   // per-target sum (k_translate<., ., 3, 1> + k_m2l_reduce) instead of atomic
@@ -197,6 +197,10 @@ struct Engine {
       if (v == m) return true;
     return false;
   }
+  static constexpr int kTimedPlans[] = {3, 5, 8, 24, 56, 92};  // besides 0 (use_side_fusion)
+  // applications before the plan is timed, and steps after that before the graph is
+  static constexpr int kPlanAfter = 64, kGraphAfter = 16;
+  int plan_apps[2] = {0, 0}, graph_steps[2] = {0, 0};
   hipStream_t side_stream = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   // slot M2L: targets, their slot ranges (CSR) and each pair's slot, the
@@ -227,9 +231,10 @@ struct Engine {
   int use_side_fusion(bool f32);
   // near-field SpMV kernel per precision ([0] FP64, [1] FP32) and storage
   // (pairs, single values): 0 workgroup per leaf with an LDS copy of the
-  // columns, 1 wavefront per leaf with 2 rows in flight, 2 with 4 rows;
-  // chosen by timing all three at set-up
+  // columns, 1 wavefront per leaf with 2 rows in flight, 2 with 4 rows, 3 (6
+  // for FP32) column vectors; chosen by timing at set-up (tune_spmv)
   int spmv_variant[2][2] = {{0, 0}, {0, 0}};  // [precision][NK - 1]
+  void ensure_row_pairs();
   template <typename T, int NK>
   void tune_spmv();
   template <typename T, int NK>

@@ -2818,6 +2818,7 @@ void Engine::assemble_near(bool want_f32) {
   up(d_scnt, cnt);
 
   const int64_t nv = std::max<int64_t>(near.nnz, 1) * 2;
+  f32.opvals_p.release();  // of an earlier mesh
   alloc(f64.vals, (size_t)nv * sizeof(double));
   DevBuf d_quads, d_units;  // freed at the end, after the stream has run
   if (near.nleaf > 0 && near.nnz > 0) {
@@ -2863,18 +2864,6 @@ void Engine::assemble_near(bool want_f32) {
     alloc(f32.opvals, (size_t)nop * sizeof(float));
     hipLaunchKernelGGL(k_round_f32, dim3((unsigned)std::min<int64_t>(nblk(nop, 256), 8192)), dim3(256), 0, stream,
                        nop, f64.opvals.as<double>(), f32.opvals.as<float>());
-    // and in row pairs, each leaf at an even (8-byte aligned) offset
-    std::vector<int64_t> pvb(near.nleaf + 1, 0);
-    for (int l = 0; l < near.nleaf; ++l) {
-      const int64_t sz = (int64_t)(near.row_beg[l + 1] - near.row_beg[l]) * (near.col_beg[l + 1] - near.col_beg[l]);
-      pvb[l + 1] = pvb[l] + ((sz + 1) & ~(int64_t)1);
-    }
-    up(d_pval_beg, pvb);
-    alloc(f32.opvals_p, (size_t)std::max<int64_t>(pvb[near.nleaf], 2) * sizeof(float));
-    if (near.nleaf > 0)
-      hipLaunchKernelGGL(k_round_f32_pairs, dim3(near.nleaf), dim3(256), 0, stream, near.nleaf, d_row_beg.as<int>(),
-                         d_col_beg.as<int>(), d_val_beg.as<int64_t>(), d_pval_beg.as<int64_t>(),
-                         f64.opvals.as<double>(), f32.opvals_p.as<float>());
     HIPCHK(hipGetLastError());
   }
   // and in column vectors, per precision
@@ -2901,6 +2890,26 @@ void Engine::assemble_near(bool want_f32) {
     tune_spmv<float, 2>();
     tune_spmv<float, 1>();
   }
+  sync();
+}
+
+// The FP32 operator's values in row pairs, for the kernels that read them
+// (variants 3..5, chosen by pbfmm_set_spmv_kernel only).
+void Engine::ensure_row_pairs() {
+  if (f32.opvals_p.p) return;
+  // each leaf at an even (8-byte aligned) offset
+  std::vector<int64_t> pvb(near.nleaf + 1, 0);
+  for (int l = 0; l < near.nleaf; ++l) {
+    const int64_t sz = (int64_t)(near.row_beg[l + 1] - near.row_beg[l]) * (near.col_beg[l + 1] - near.col_beg[l]);
+    pvb[l + 1] = pvb[l] + ((sz + 1) & ~(int64_t)1);
+  }
+  up(d_pval_beg, pvb);
+  alloc(f32.opvals_p, (size_t)std::max<int64_t>(pvb[near.nleaf], 2) * sizeof(float));
+  if (near.nleaf > 0)
+    hipLaunchKernelGGL(k_round_f32_pairs, dim3(near.nleaf), dim3(256), 0, stream, near.nleaf, d_row_beg.as<int>(),
+                       d_col_beg.as<int>(), d_val_beg.as<int64_t>(), d_pval_beg.as<int64_t>(),
+                       f64.opvals.as<double>(), f32.opvals_p.as<float>());
+  HIPCHK(hipGetLastError());
   sync();
 }
 
@@ -3089,33 +3098,37 @@ static void launch_spmm(Engine &e, const double *x, double *out, int R) {
   else go(std::integral_constant<int, 16>{});
 }
 
-// Times the SpMV kernels (workgroup per leaf; wavefront per leaf with 2 or 4
-// rows in flight) on the assembled near field (HIP events, scratch vectors)
-// and keeps the fastest for this precision and storage.
+// Times the SpMV kernels that are the fastest somewhere on the assembled near
+// field (HIP events, scratch vectors) and keeps the faster for this precision
+// and storage.  Pairs: workgroup per leaf, or wavefront per leaf with 2 rows in
+// flight (4 rows in flight were within 3% of the better of the two at twenty
+// problems of 602 to 393,218 DoFs and leaf sizes 20 to 96).  Single values:
+// column vectors, and the wavefront per leaf, which is faster for many narrow
+// leaves (393,218 DoFs, leaf 20: 0.158 against 0.253 ms FP32, 0.245 against
+// 0.303 ms FP64; leaf 80: 0.492 against 0.354, 0.929 against 0.674).  The
+// others stay for pbfmm_set_spmv_kernel.  A kernel whose first launch takes
+// half as long again as the best time so far is not timed further.
 template <typename T, int NK>
 void Engine::tune_spmv() {
   if (near.nleaf == 0) return;
   hipEvent_t e0, e1;
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));
-  float best = 0;
-  int pick = 0;
-  // one warm-up and three timed launches per variant (the variants differ by
-  // 5-30% at the sizes measured, the repetitions by ~1%)
-  for (int v = 0; v < (NK == 2 ? 3 : kColsVariant<T> + 1); ++v) {
-    launch_spmv<T, NK>(v, d_sp.as<double>(), d_sd.as<double>(), d_outN.as<double>(), d_outD.as<double>());
+  auto timed = [&](int v, int reps) {
     HIPCHK(hipEventRecord(e0, stream));
-    for (int rep = 0; rep < 3; ++rep)
+    for (int r = 0; r < reps; ++r)
       launch_spmv<T, NK>(v, d_sp.as<double>(), d_sd.as<double>(), d_outN.as<double>(), d_outD.as<double>());
     HIPCHK(hipEventRecord(e1, stream));
     HIPCHK(hipEventSynchronize(e1));
     float ms = 0;
     HIPCHK(hipEventElapsedTime(&ms, e0, e1));
-    if (v == 0 || ms < best) {
-      best = ms;
-      pick = v;
-    }
-  }
+    return ms / reps;
+  };
+  const int first = NK == 2 ? 0 : kColsVariant<T>;
+  int pick = first;
+  (void)timed(first, 1);
+  const float best = timed(first, 2);
+  if (timed(1, 1) < 1.5f * best && timed(1, 2) < best) pick = 1;
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   spmv_variant[sizeof(T) == 4 ? 1 : 0][NK - 1] = pick;
@@ -3517,15 +3530,21 @@ double Engine::norm2(const double *v) {
   return std::sqrt(h);
 }
 
-// Side fusion pays while the M2M / L2L level launches are latency-bound and
-// the SpMV and M2P are short beside them (tens of thousands of DoFs); on
-// large trees the fused workgroups only crowd each other.  The modes are
-// matvec_fused's side 0..3.  Timed once per precision, on the first operator
-// application: six applications each way on scratch vectors, after one
-// warm-up; a fused mode is kept only if it beats the unfused one by 2%.
+// The launch plan of the operator (matvec_fused).  Which is the fastest
+// depends on the problem (level launches that wait on latency, SpMV and M2L
+// that share the chip or crowd each other), by up to 1.7x, so it is timed, per
+// precision, on scratch vectors: kTimedPlans, of which one was within 2% of
+// the best of all fourteen at every one of twenty problems (602 to 393,218
+// DoFs, orders 4 to 8, leaf sizes 20 to 96, both precisions).  A plan other
+// than 0 is kept only if it beats plan 0 by 2%.  Timing costs two dozen
+// applications and a plan gains a tenth of one as a rule, so one solve does not
+// pay for it: the first kPlanAfter applications of a precision run plan 0
+// (98,306 DoFs, Q2, one mixed solve on a new handle: 75 ms of timing before a
+// solve of 16 ms).
 int Engine::use_side_fusion(bool f32) {
   int &mode = side_fusion[f32 ? 1 : 0];
   if (mode >= 0) return mode;
+  if (plan_apps[f32 ? 1 : 0]++ < kPlanAfter) return 0;
   const unsigned g = nblk(n, 256);
   if (d_cost.bytes < (size_t)2 * n * 8) alloc(d_cost, (size_t)2 * n * 8);
   double *u = d_cost.as<double>(), *v = d_cost.as<double>() + n;
@@ -3533,27 +3552,33 @@ int Engine::use_side_fusion(bool f32) {
   hipEvent_t t0, t1;
   HIPCHK(hipEventCreate(&t0));
   HIPCHK(hipEventCreate(&t1));
-  constexpr int np = (int)(sizeof(kPlans) / sizeof(kPlans[0]));
-  float ms[np] = {};
-  for (int s = 0; s < np; ++s)
-    for (int rep = 0; rep < 7; ++rep) {
+  auto timed = [&](int plan, int reps) {  // ms per application, after one more
+    for (int rep = 0; rep <= reps; ++rep) {
       if (rep == 1) HIPCHK(hipEventRecord(t0, stream));
       if (f32)
-        matvec_fused<float>(u, d_outN.as<double>(), v, kPlans[s]);
+        matvec_fused<float>(u, d_outN.as<double>(), v, plan);
       else
-        matvec_fused<double>(u, d_outN.as<double>(), v, kPlans[s]);
-      if (rep == 6) {
-        HIPCHK(hipEventRecord(t1, stream));
-        HIPCHK(hipEventSynchronize(t1));
-        HIPCHK(hipEventElapsedTime(&ms[s], t0, t1));
-      }
+        matvec_fused<double>(u, d_outN.as<double>(), v, plan);
     }
+    HIPCHK(hipEventRecord(t1, stream));
+    HIPCHK(hipEventSynchronize(t1));
+    float ms = 0;
+    HIPCHK(hipEventElapsedTime(&ms, t0, t1));
+    return ms / reps;
+  };
+  float plain = timed(0, 2);
+  // short applications are repeated up to 0.4 ms a plan
+  const int reps = (int)std::max(2.0f, std::min(6.0f, 0.4f / std::max(plain, 1e-3f)));
+  if (reps > 2) plain = timed(0, reps);
+  float best = 0.98f * plain;
+  int pick = 0;
+  for (int plan : kTimedPlans) {
+    const float ms = timed(plan, reps);
+    if (ms < best) best = ms, pick = plan;
+  }
   (void)hipEventDestroy(t0);
   (void)hipEventDestroy(t1);
-  int best = 0;
-  for (int s = 1; s < np; ++s)
-    if (ms[s] < ms[best]) best = s;
-  mode = ms[best] < 0.98f * ms[0] ? kPlans[best] : 0;
+  mode = pick;
   return mode;
 }
 
@@ -3807,15 +3832,16 @@ std::vector<int64_t> Engine::graph_key(int precision) const {
 }
 
 // step_op(d_vn -> d_wk) as a graph replay when that was measured faster.
-// The first call per step precision runs it directly (the side-fusion and
-// SpMV choices time themselves there), the next captures it after one more
-// direct run (allocations on first use happen outside the capture) and times
-// three direct runs against three replays; from then on the faster one runs,
-// recaptured whenever graph_key changes.
+// The first steps per precision run directly, until kGraphAfter have run with
+// a timed launch plan (the choice costs eight steps and a capture and gains 3%
+// where it gains), the next captures the step after one more direct run (allocations on first use happen outside the
+// capture) and times three direct runs against three replays; from then on
+// the faster one runs, recaptured whenever graph_key changes.
 void Engine::step_op_graph(int precision) {
   const int f = precision == PBFMM_MIXED && have_f32 ? 1 : 0;
   double *vin = d_vn.as<double>(), *w = d_wk.as<double>();
-  if (!graph_enabled || graph_use[f] == 0 || side_fusion[f] < 0) {
+  if (!graph_enabled || graph_use[f] == 0 || side_fusion[f] < 0 ||
+      (graph_use[f] < 0 && graph_steps[f]++ < kGraphAfter)) {
     step_op(vin, w, precision);
     return;
   }
