@@ -173,6 +173,26 @@ __global__ void k_pack_quads(int64_t n, const double *__restrict__ qx, const dou
   out[4 * g + 3] = double2{qw[g], 0.0};
 }
 
+// The column of each of an entry's DoFs in its leaf's sorted columns.
+__global__ void __launch_bounds__(256) k_entry_cols(const int *__restrict__ ent_beg, const int *__restrict__ ent_cell,
+                                                    const int *__restrict__ cdofs, int dpc,
+                                                    const int *__restrict__ col_beg, const int *__restrict__ cols,
+                                                    int *__restrict__ colpos) {
+  const int leaf = blockIdx.x;
+  const int64_t e0 = (int64_t)ent_beg[leaf] * dpc, e1 = (int64_t)ent_beg[leaf + 1] * dpc;
+  const int cb = col_beg[leaf], C = col_beg[leaf + 1] - cb;
+  for (int64_t i = e0 + blockIdx.y * 256 + threadIdx.x; i < e1; i += (int64_t)gridDim.y * 256) {
+    const int e = (int)(i / dpc), d = cdofs[(int64_t)ent_cell[e] * dpc + (int)(i - (int64_t)e * dpc)];
+    int lo = 0, hi = C - 1;  // every DoF of an entry is a column
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (cols[cb + mid] < d) lo = mid + 1;
+      else hi = mid;
+    }
+    colpos[i] = lo;
+  }
+}
+
 constexpr int kAsmRows = 8, kAsmCols = 512, kAsmThreads = 512;
 constexpr int kAsmStride = kAsmCols + 4;       // doubles per row of the LDS tile's N and D (the padding spreads rows over banks)
 constexpr int kAsmPlane = kAsmRows * kAsmStride;  // N, then D
@@ -986,7 +1006,7 @@ __device__ __forceinline__ T wave_allsum(T v) {
 // (for leaves whose unit multipoles do not fit in LDS).
 __global__ void __launch_bounds__(256) k_p2m_unit(
     int npts, int p, int kt, int kp, const int *__restrict__ qpt, const int *__restrict__ qleaf,
-    const int *__restrict__ leaves, const int *__restrict__ qcol, int dpc, const double *__restrict__ qx,
+    const int *__restrict__ leaves, const int *__restrict__ qcol, int dpc, int nrule, const double *__restrict__ qx,
     const double *__restrict__ qn, const double *__restrict__ qw, const double *__restrict__ qsh,
     const double *__restrict__ pmin, const double *__restrict__ delta, double *__restrict__ U) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1002,7 +1022,7 @@ __global__ void __launch_bounds__(256) k_p2m_unit(
   double wj[9];
   double *col[9];
   for (int j = 0; j < dpc; ++j) {
-    wj[j] = qsh[g * dpc + j] * qw[g] / (4 * kPi);
+    wj[j] = qsh[(g % nrule) * dpc + j] * qw[g] / (4 * kPi);
     col[j] = U + (int64_t)qcol[(int64_t)i * dpc + j] * 2 * kp;
   }
   // level-scaled multipoles: coefficient of degree n divided by delta^n
@@ -1041,6 +1061,23 @@ __global__ void __launch_bounds__(256) k_p2m_unit(
   }
 }
 
+// The column of each DoF of a quad point's cell among its leaf's columns.
+__global__ void k_quad_cols(int64_t n, int dpc, int nrule, const int *__restrict__ qpt, const int *__restrict__ qleaf,
+                            const int *__restrict__ cdofs, const int *__restrict__ col_beg,
+                            const int *__restrict__ col_dof, int *__restrict__ qcol) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int64_t pt = i / dpc;
+  const int d = cdofs[(int64_t)(qpt[pt] / nrule) * dpc + (int)(i - pt * dpc)];
+  int lo = col_beg[qleaf[pt]], hi = col_beg[qleaf[pt] + 1] - 1;  // every DoF of its cells is a column
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (col_dof[mid] < d) lo = mid + 1;
+    else hi = mid;
+  }
+  qcol[i] = lo;
+}
+
 // Set-up, FP64, one workgroup per leaf whose unit multipoles fit in LDS: the
 // block [column][2 kp] of the leaf is summed in LDS (atomic adds there) and
 // written once with plain stores, since no other leaf owns those columns.
@@ -1053,7 +1090,7 @@ __global__ void __launch_bounds__(256) k_p2m_unit(
 __global__ void __launch_bounds__(256) k_p2m_unit_leaf(
     int p, int kt, int kp, const int *__restrict__ leaf_ids, const int *__restrict__ leaves,
     const int *__restrict__ qbeg, const int *__restrict__ col_beg, const int *__restrict__ qpt,
-    const int *__restrict__ qcol, int dpc, const double *__restrict__ qx, const double *__restrict__ qn,
+    const int *__restrict__ qcol, int dpc, int nrule, const double *__restrict__ qx, const double *__restrict__ qn,
     const double *__restrict__ qw, const double *__restrict__ qsh, const double *__restrict__ pmin,
     const double *__restrict__ delta, double *__restrict__ U, int half) {
   extern __shared__ double sU[];
@@ -1077,7 +1114,7 @@ __global__ void __launch_bounds__(256) k_p2m_unit_leaf(
     double wj[9];
     int cj[9];
     for (int j = 0; j < dpc; ++j) {
-      wj[j] = qsh[g * dpc + j] * qw[g] / (4 * kPi);
+      wj[j] = qsh[(g % nrule) * dpc + j] * qw[g] / (4 * kPi);
       cj[j] = (qcol[(int64_t)i * dpc + j] - c0) * S;
     }
     double Rmr = 1, Rmi = 0, Gmr = 0, Gmi = 0;  // R_m^m, D R_m^m
@@ -2486,8 +2523,8 @@ static inline unsigned nblk(int64_t n, int t) { return (unsigned)((n + t - 1) / 
 // holds the addresses it was captured with: one captured before the last
 // allocation is captured again).
 static int64_t g_alloc_epoch = 0;
-template <typename T>
-static void up(DevBuf &b, const std::vector<T> &v) {
+template <typename T, typename A>
+static void up(DevBuf &b, const std::vector<T, A> &v) {
   b.release();
   const size_t bytes = std::max<size_t>(v.size() * sizeof(T), 16);
   HIPCHK(hipMalloc(&b.p, bytes));
@@ -2617,7 +2654,6 @@ void Engine::upload_near_plan() {
   up(d_ent_cell, near.ent_cell);
   up(d_ent_mask, near.ent_mask);
   up(d_ent_near, near.ent_near);
-  up(d_ent_colpos, near.ent_colpos);
   up(d_leaf_block, near.leaf_block);
 }
 
@@ -2686,7 +2722,7 @@ void Engine::build_unit_multipoles(bool want_f32) {
     const int nleaf = (int)far.p2m_leaf.size();
     const size_t col_bytes = (size_t)2 * kp * sizeof(double);
     constexpr size_t kLdsMax = 160 * 1024 - 1024;
-    std::vector<int32_t> qbeg(nleaf + 1, 0), fit, fit_half, big_qpt, big_qleaf, big_qcol;
+    std::vector<int32_t> qbeg(nleaf + 1, 0), fit, fit_half, big_qpt, big_qleaf;
     for (int i = 0; i < npts; ++i) qbeg[far.p2m_qleaf[i] + 1]++;
     for (int li = 0; li < nleaf; ++li) qbeg[li + 1] += qbeg[li];
     size_t max_bytes = 0, max_half = 0;
@@ -2702,13 +2738,19 @@ void Engine::build_unit_multipoles(bool want_f32) {
         for (int i = qbeg[li]; i < qbeg[li + 1]; ++i) {
           big_qpt.push_back(far.p2m_qpt[i]);
           big_qleaf.push_back(li);
-          for (int j = 0; j < dpc; ++j) big_qcol.push_back(far.p2m_qcol[(size_t)i * dpc + j]);
         }
       }
     }
-    DevBuf qpt, qcol, dqbeg, dfit, dfit_half;
+    DevBuf qpt, qleaf, qcol, dqbeg, dfit, dfit_half;
+    auto quad_cols = [&](const DevBuf &pt, const DevBuf &leaf, DevBuf &col, int64_t count) {
+      alloc(col, (size_t)count * dpc * sizeof(int));
+      hipLaunchKernelGGL(k_quad_cols, dim3(nblk(count * dpc, 256)), dim3(256), 0, stream, count * dpc, dpc, nq,
+                         pt.as<int>(), leaf.as<int>(), d_cdofs.as<int>(), d_p2m_col_beg.as<int>(),
+                         d_p2m_col_dof.as<int>(), col.as<int>());
+    };
     up(qpt, far.p2m_qpt);
-    up(qcol, far.p2m_qcol);
+    up(qleaf, far.p2m_qleaf);
+    quad_cols(qpt, qleaf, qcol, npts);
     up(dqbeg, qbeg);
     up(dfit, fit);
     up(dfit_half, fit_half);
@@ -2718,7 +2760,7 @@ void Engine::build_unit_multipoles(bool want_f32) {
     if (!fit.empty()) {
       hipLaunchKernelGGL(k_p2m_unit_leaf, dim3((unsigned)fit.size()), dim3(256), max_bytes, stream, p, kt, kp,
                          dfit.as<int>(), d_p2m_leaf.as<int>(), dqbeg.as<int>(), d_p2m_col_beg.as<int>(),
-                         qpt.as<int>(), qcol.as<int>(), dpc, f64.qx.as<double>(), f64.qn.as<double>(),
+                         qpt.as<int>(), qcol.as<int>(), dpc, nq, f64.qx.as<double>(), f64.qn.as<double>(),
                          f64.qw.as<double>(), f64.qsh.as<double>(), d_pmin.as<double>(), d_delta.as<double>(),
                          f64.unit.as<double>(), -1);
       HIPCHK(hipGetLastError());
@@ -2726,7 +2768,7 @@ void Engine::build_unit_multipoles(bool want_f32) {
     for (int half = 0; half < 2 && !fit_half.empty(); ++half) {
       hipLaunchKernelGGL(k_p2m_unit_leaf, dim3((unsigned)fit_half.size()), dim3(256), max_half, stream, p, kt, kp,
                          dfit_half.as<int>(), d_p2m_leaf.as<int>(), dqbeg.as<int>(), d_p2m_col_beg.as<int>(),
-                         qpt.as<int>(), qcol.as<int>(), dpc, f64.qx.as<double>(), f64.qn.as<double>(),
+                         qpt.as<int>(), qcol.as<int>(), dpc, nq, f64.qx.as<double>(), f64.qn.as<double>(),
                          f64.qw.as<double>(), f64.qsh.as<double>(), d_pmin.as<double>(), d_delta.as<double>(),
                          f64.unit.as<double>(), half);
       HIPCHK(hipGetLastError());
@@ -2735,16 +2777,16 @@ void Engine::build_unit_multipoles(bool want_f32) {
       DevBuf bqpt, bqleaf, bqcol;
       up(bqpt, big_qpt);
       up(bqleaf, big_qleaf);
-      up(bqcol, big_qcol);
       const int nb = (int)big_qpt.size();
+      quad_cols(bqpt, bqleaf, bqcol, nb);
       hipLaunchKernelGGL(k_p2m_unit, dim3(nblk(nb, 256)), dim3(256), 0, stream, nb, p, kt, kp, bqpt.as<int>(),
-                         bqleaf.as<int>(), d_p2m_leaf.as<int>(), bqcol.as<int>(), dpc, f64.qx.as<double>(),
+                         bqleaf.as<int>(), d_p2m_leaf.as<int>(), bqcol.as<int>(), dpc, nq, f64.qx.as<double>(),
                          f64.qn.as<double>(), f64.qw.as<double>(), f64.qsh.as<double>(), d_pmin.as<double>(),
                          d_delta.as<double>(), f64.unit.as<double>());
       HIPCHK(hipGetLastError());
       sync();  // the index copies are freed on return
     }
-    sync();  // qpt, qcol, dqbeg, dfit, dfit_half are freed on return
+    sync();  // qpt, qleaf, qcol, dqbeg, dfit, dfit_half are freed on return
   }
   // the operator's unit multipoles (U1 on Neumann, -U2 on Dirichlet DoFs),
   // compact: the real parts, then the imaginary parts of m >= 1 (those of
@@ -2820,7 +2862,7 @@ void Engine::assemble_near(bool want_f32) {
   const int64_t nv = std::max<int64_t>(near.nnz, 1) * 2;
   f32.opvals_p.release();  // of an earlier mesh
   alloc(f64.vals, (size_t)nv * sizeof(double));
-  DevBuf d_quads, d_units;  // freed at the end, after the stream has run
+  DevBuf d_quads, d_units, d_colpos;  // freed at the end, after the stream has run
   if (near.nleaf > 0 && near.nnz > 0) {
     if (nq > 64 || dpc > 9) throw std::runtime_error("near assembly: more than 64 quad points or 9 DoFs per cell");
     // tiles of kAsmRows rows x kAsmCols columns of every leaf's block
@@ -2835,8 +2877,12 @@ void Engine::assemble_near(bool want_f32) {
     alloc(d_quads, (size_t)npts * 64);
     hipLaunchKernelGGL(k_pack_quads, dim3(nblk(npts, 256)), dim3(256), 0, stream, npts, f64.qx.as<double>(),
                        f64.qn.as<double>(), f64.qw.as<double>(), d_quads.as<double2>());
+    alloc(d_colpos, near.ent_cell.size() * dpc * sizeof(int));
+    hipLaunchKernelGGL(k_entry_cols, dim3(near.nleaf, 4), dim3(256), 0, stream, d_ent_beg.as<int>(),
+                       d_ent_cell.as<int>(), d_cdofs.as<int>(), dpc, d_col_beg.as<int>(), d_cols.as<int>(),
+                       d_colpos.as<int>());
     AsmArgs a{d_row_beg.as<int>(), d_rows.as<int>(), d_col_beg.as<int>(), d_cols.as<int>(), d_ent_beg.as<int>(),
-              d_ent_cell.as<int>(), d_ent_mask.as<uint64_t>(), d_ent_near.as<uint8_t>(), d_ent_colpos.as<int>(),
+              d_ent_cell.as<int>(), d_ent_mask.as<uint64_t>(), d_ent_near.as<uint8_t>(), d_colpos.as<int>(),
               d_val_beg.as<int64_t>(), nq, d_dbl_ptr.as<int>(), d_dbl_idx.as<int>(), d_xyz.as<double>(),
               d_quads.as<double2>(), f64.qsh.as<double>(), d_geom.as<double>(), d_sing.as<double>(),
               d_scnt.as<int>(), maxq * ps, f64.vals.as<double>()};

@@ -13,13 +13,13 @@ namespace pbfmm {
 
 namespace {
 
-template <typename T>
-void append_off(std::vector<T> &dst, const std::vector<T> &src, T off, bool keep_negative = false) {
+template <typename T, typename A>
+void append_off(std::vector<T, A> &dst, const std::vector<T, A> &src, T off, bool keep_negative = false) {
   dst.reserve(dst.size() + src.size());
   for (const T &v : src) dst.push_back(keep_negative && v < 0 ? v : v + off);
 }
-template <typename T>
-void append(std::vector<T> &dst, const std::vector<T> &src) {
+template <typename V>
+void append(V &dst, const V &src) {
   dst.insert(dst.end(), src.begin(), src.end());
 }
 // prefix array (n+1 entries starting at 0) of a part appended to a merged one
@@ -135,7 +135,7 @@ void merge_forest(const std::vector<const Engine *> &parts, Engine &e, std::vect
     append(e.qd.x, q.qd.x);
     append(e.qd.n, q.qd.n);
     append(e.qd.jxw, q.qd.jxw);
-    append(e.qd.sh, q.qd.sh);
+    if (e.qd.sh.empty()) e.qd.sh = q.qd.sh;
     // octree arrays the device reads
     append(t.level, q.tree.level);
     append_off(t.parent, q.tree.parent, bo, true);
@@ -164,20 +164,16 @@ void merge_forest(const std::vector<const Engine *> &parts, Engine &e, std::vect
     append_off(np.ent_cell, q.near.ent_cell, coff);
     append(np.ent_mask, q.near.ent_mask);
     append(np.ent_near, q.near.ent_near);
-    append(np.ent_colpos, q.near.ent_colpos);
-    append_prefix(np.work_beg, q.near.work_beg);
     append_off(np.row_leaf, q.near.row_leaf, leaf_off);
     np.nleaf += q.near.nleaf;
     np.nnz += q.near.nnz;
     // far field
     const int32_t p2m_leaf_off = (int32_t)fp.p2m_leaf.size();
-    const int32_t col_off = (int32_t)fp.p2m_col_dof.size();
     append_off(fp.p2m_leaf, q.far.p2m_leaf, bo);
     append_prefix(fp.p2m_col_beg, q.far.p2m_col_beg);
     append_off(fp.p2m_col_dof, q.far.p2m_col_dof, doff);
     append_off(fp.p2m_qpt, q.far.p2m_qpt, qoff);
     append_off(fp.p2m_qleaf, q.far.p2m_qleaf, p2m_leaf_off);
-    append_off(fp.p2m_qcol, q.far.p2m_qcol, col_off);
     m2m_off[s] = (int32_t)(fp.m2m_ops.size() / ((size_t)fp.kp * fp.kp));
     // the single-level operators only: the batch runs M2M and L2L level by
     // level, without the parts' composite two-level ones (build_m2m_groups,
@@ -205,7 +201,6 @@ void merge_forest(const std::vector<const Engine *> &parts, Engine &e, std::vect
   if (np.row_beg.empty()) np.row_beg.push_back(0);
   if (np.col_beg.empty()) np.col_beg.push_back(0);
   if (np.ent_beg.empty()) np.ent_beg.push_back(0);
-  if (np.work_beg.empty()) np.work_beg.push_back(0);
   if (fp.p2m_col_beg.empty()) fp.p2m_col_beg.push_back(0);
   if (fp.m2p_work_beg.empty()) fp.m2p_work_beg.push_back(0);
   // M2M and L2L operators are indexed level * 8 + octant within a part
@@ -270,7 +265,7 @@ void validate_plans(const Engine &e) {
   size_is("quad points", e.qd.x.size(), 3 * NQ);
   size_is("quad normals", e.qd.n.size(), 3 * NQ);
   size_is("quad weights", e.qd.jxw.size(), NQ);
-  size_is("quad shapes", e.qd.sh.size(), NQ * dpc);
+  size_is("quad shapes", e.qd.sh.size(), nq * dpc);
   size_is("tree parent", t.parent.size(), nb);
   in_range("tree parent", t.parent, -1, nb, true);
   size_is("tree children", t.child.size(), (size_t)8 * nb);
@@ -300,8 +295,6 @@ void validate_plans(const Engine &e) {
   in_range("near cells", np.ent_cell, (int64_t)0, nc);
   size_is("near entry masks", np.ent_mask.size(), np.ent_cell.size());
   size_is("near entry flags", np.ent_near.size(), np.ent_cell.size());
-  size_is("near entry columns", np.ent_colpos.size(), np.ent_cell.size() * dpc);
-  size_is("near work", np.work_beg.size(), (size_t)nl + 1);
   size_is("near row leaf", np.row_leaf.size(), np.rows.size());
   in_range("near row leaf", np.row_leaf, 0, std::max(nl, 1));
   int64_t vend = 0;
@@ -309,10 +302,6 @@ void validate_plans(const Engine &e) {
     const int64_t R = np.row_beg[l + 1] - np.row_beg[l], C = np.col_beg[l + 1] - np.col_beg[l];
     if (np.val_beg[l] != vend) throw std::runtime_error("plan check: near value offsets malformed");
     vend += R * C;
-    for (int k = np.ent_beg[l] * dpc; k < np.ent_beg[l + 1] * dpc; ++k)
-      if (np.ent_colpos[k] < 0 || np.ent_colpos[k] >= C) throw std::runtime_error("plan check: near column position");
-    if (np.work_beg[l + 1] - np.work_beg[l] != R * (np.ent_beg[l + 1] - np.ent_beg[l]))
-      throw std::runtime_error("plan check: near work offsets malformed");
   }
   if (vend != np.nnz) throw std::runtime_error("plan check: near value count");
   const FarPlan &fp = e.far;
@@ -322,15 +311,7 @@ void validate_plans(const Engine &e) {
   in_range("p2m columns", fp.p2m_col_dof, (int64_t)0, n);
   in_range("p2m quad points", fp.p2m_qpt, (int64_t)0, NQ);
   size_is("p2m quad leaves", fp.p2m_qleaf.size(), fp.p2m_qpt.size());
-  size_is("p2m quad columns", fp.p2m_qcol.size(), fp.p2m_qpt.size() * dpc);
-  for (size_t i = 0; i < fp.p2m_qpt.size(); ++i) {
-    const int li = fp.p2m_qleaf[i];
-    if (li < 0 || li >= npl) throw std::runtime_error("plan check: p2m quad leaf");
-    for (int j = 0; j < dpc; ++j) {
-      const int c = fp.p2m_qcol[i * dpc + j];
-      if (c < fp.p2m_col_beg[li] || c >= fp.p2m_col_beg[li + 1]) throw std::runtime_error("plan check: p2m column");
-    }
-  }
+  in_range("p2m quad leaves", fp.p2m_qleaf, 0, std::max(npl, 1));
   const size_t op_sz = (size_t)kp * kp;
   if (fp.m2m_ops.size() % op_sz || fp.l2l_ops.size() % op_sz || fp.m2l_ops.size() != (size_t)fp.n_m2l_ops * op_sz)
     throw std::runtime_error("plan check: operator storage");

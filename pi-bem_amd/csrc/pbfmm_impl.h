@@ -6,6 +6,8 @@
 #include <cstdint>
 #include <functional>
 #include <string>
+#include <memory>
+#include <utility>
 #include <vector>
 
 #include "../../include/pbfmm.h"
@@ -20,6 +22,19 @@ inline int kt_of(int p) { return (p + 1) * (p + 2) / 2; }
 // Runs body(i) for i in [0, n) on up to 16 host threads, `grain` indices at
 // a time (dynamic); the caller's results must not depend on the order.
 void parallel_for(int64_t n, int64_t grain, const std::function<void(int64_t)> &body);
+// Vectors whose resize leaves new elements uninitialised: large plan arrays,
+// filled by several threads, whose pages are then touched by those.
+template <typename T>
+struct NoInit : std::allocator<T> {
+  template <typename U> struct rebind { using other = NoInit<U>; };
+  NoInit() = default;
+  template <typename U> NoInit(const NoInit<U> &) {}
+  template <typename U> void construct(U *) noexcept {}
+  template <typename U, typename A, typename... R> void construct(U *p, A &&a, R &&...r) {
+    ::new ((void *)p) U(std::forward<A>(a), std::forward<R>(r)...);
+  }
+};
+template <typename T> using RawVec = std::vector<T, NoInit<T>>;
 // Pairs per GEMM chunk of the batched translations (64 GEMM columns): 32 pairs
 // when both kernels' expansions travel (2 columns per pair), 64 pairs when
 // one combined expansion does.
@@ -66,7 +81,8 @@ void unit_support_point(int dpc, int j, double &xi, double &eta);
 
 struct QuadData {
   int nq = 0;
-  std::vector<double> x, n, jxw, sh;  // per global quad id g = cell*nq+q
+  std::vector<double> x, n, jxw;  // per global quad id g = cell*nq+q
+  std::vector<double> sh;         // shape values of the rule, [nq][dpc], the same for every cell
 };
 void compute_quad_data(const HostMesh &m, const Quadrature2D &rule, QuadData &qd);
 
@@ -83,7 +99,7 @@ struct Tree {
   std::vector<std::vector<int32_t>> dofs_filled;              // per level
   std::vector<int32_t> nperm, node_beg, node_cnt;
   std::vector<int32_t> qperm, quad_beg, quad_cnt;
-  std::vector<int32_t> qblock;  // (L+1) x nquad
+  RawVec<int32_t> qblock;       // (L+1) x nquad
   std::vector<int32_t> nsub, sub_beg;
   std::vector<std::vector<int32_t>> nn, il, nil;  // index sub_beg[b]+s
   void center(int b, double c[3]) const {
@@ -101,14 +117,13 @@ struct NearPlan {
   int nleaf = 0;                    // leaves holding nodes
   std::vector<int32_t> leaf_block;  // block id
   std::vector<int32_t> row_beg, rows;   // rows (node ids) per leaf
-  std::vector<int32_t> col_beg, cols;   // columns per leaf
+  std::vector<int32_t> col_beg;
+  RawVec<int32_t> cols;                 // columns per leaf
   std::vector<int64_t> val_beg;         // offset of the rows x cols block
   std::vector<int32_t> ent_beg;         // entries per leaf
-  std::vector<int32_t> ent_cell;
-  std::vector<uint64_t> ent_mask;       // quad points of the cell in this entry
-  std::vector<uint8_t> ent_near;        // 1: leaf near list (may be singular)
-  std::vector<int32_t> ent_colpos;      // dpc per entry
-  std::vector<int64_t> work_beg;        // prefix of rows*entries per leaf
+  RawVec<int32_t> ent_cell;
+  RawVec<uint64_t> ent_mask;            // quad points of the cell in this entry
+  RawVec<uint8_t> ent_near;             // 1: leaf near list (may be singular)
   std::vector<int32_t> row_leaf;        // leaf-ordered row -> leaf
   int64_t nnz = 0;
 };
@@ -134,9 +149,9 @@ struct FarPlan {
   // P2M as a product with unit multipoles: per leaf (index into p2m_leaf) the
   // sorted DoFs of the cells that have quad points in the leaf (columns
   // p2m_col_beg[li] .. p2m_col_beg[li+1]); per quad point of the leaves, in
-  // leaf order, its id, its leaf and the column of each of its cell's DoFs.
+  // leaf order, its id and its leaf.
   std::vector<int32_t> p2m_col_beg, p2m_col_dof;
-  std::vector<int32_t> p2m_qpt, p2m_qleaf, p2m_qcol;
+  std::vector<int32_t> p2m_qpt, p2m_qleaf;
   ChunkList m2m;                  // tgt = parent, src = child; op = level*8 + octant
   ChunkList m2l;                  // op = offset class (all levels)
   ChunkList l2l;                  // tgt = child, src = parent; op = level*8 + octant

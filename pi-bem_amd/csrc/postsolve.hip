@@ -536,30 +536,40 @@ void Engine::ps_setup(int quad_order) {
         dloc[fill[d]++] = (int8_t)j;
       }
   }
-  // scalar mass-matrix pattern: the DoFs sharing a cell
+  // scalar mass-matrix pattern: the DoFs sharing a cell, rows on host threads
+  // (the columns counted, then stored)
   std::vector<int32_t> mptr(n + 1, 0), mcol;
-  {
+  auto row_cols = [&](int64_t r, std::vector<int32_t> &row) {
+    row.clear();
+    for (int32_t t = dptr[r]; t < dptr[r + 1]; ++t)
+      for (int j = 0; j < D; ++j) row.push_back(mesh.cdofs[(int64_t)dcell[t] * D + j]);
+    std::sort(row.begin(), row.end());
+    row.erase(std::unique(row.begin(), row.end()), row.end());
+  };
+  constexpr int64_t kRows = 1024;
+  const int64_t nruns = (n + kRows - 1) / kRows;
+  std::vector<std::vector<int32_t>> runs(nruns);
+  parallel_for(nruns, 1, [&](int64_t b) {
     std::vector<int32_t> row;
-    for (int64_t r = 0; r < n; ++r) {
-      row.clear();
-      for (int32_t t = dptr[r]; t < dptr[r + 1]; ++t)
-        for (int j = 0; j < D; ++j) row.push_back(mesh.cdofs[(int64_t)dcell[t] * D + j]);
-      std::sort(row.begin(), row.end());
-      row.erase(std::unique(row.begin(), row.end()), row.end());
-      mcol.insert(mcol.end(), row.begin(), row.end());
-      mptr[r + 1] = (int32_t)mcol.size();
+    for (int64_t r = b * kRows; r < std::min(n, (b + 1) * kRows); ++r) {
+      row_cols(r, row);
+      runs[b].insert(runs[b].end(), row.begin(), row.end());
+      mptr[r + 1] = (int32_t)row.size();
     }
-  }
+  });
+  for (int64_t r = 0; r < n; ++r) mptr[r + 1] += mptr[r];
+  mcol.resize(mptr[n]);
   std::vector<int32_t> pos((size_t)nc * D * D);
-  for (int64_t c = 0; c < nc; ++c)
-    for (int i = 0; i < D; ++i) {
-      const int32_t r = mesh.cdofs[c * D + i];
-      for (int j = 0; j < D; ++j) {
-        const int32_t col = mesh.cdofs[c * D + j];
-        const auto b = mcol.begin() + mptr[r], e = mcol.begin() + mptr[r + 1];
-        pos[((size_t)c * D + i) * D + j] = (int32_t)(std::lower_bound(b, e, col) - mcol.begin());
+  parallel_for(nruns, 1, [&](int64_t b) {
+    std::copy(runs[b].begin(), runs[b].end(), mcol.begin() + mptr[b * kRows]);
+    for (int64_t r = b * kRows; r < std::min(n, (b + 1) * kRows); ++r)
+      for (int32_t t = dptr[r]; t < dptr[r + 1]; ++t) {
+        const int32_t *cd = &mesh.cdofs[(int64_t)dcell[t] * D];
+        const auto rb = mcol.begin() + mptr[r], re = mcol.begin() + mptr[r + 1];
+        for (int j = 0; j < D; ++j)
+          pos[((size_t)dcell[t] * D + dloc[t]) * D + j] = (int32_t)(std::lower_bound(rb, re, cd[j]) - mcol.begin());
       }
-    }
+  });
   ps.nnz = (int64_t)mcol.size();
   ps_up(ps.d2c_ptr, dptr);
   ps_up(ps.d2c_cell, dcell);

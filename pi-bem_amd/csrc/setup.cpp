@@ -147,11 +147,12 @@ void compute_quad_data(const HostMesh &m, const Quadrature2D &rule, QuadData &qd
   qd.x.resize(3 * NQ);
   qd.n.resize(3 * NQ);
   qd.jxw.resize(NQ);
-  qd.sh.resize(NQ * dpc);
-  std::vector<double> N(nq * dpc), dx(nq * dpc), dy(nq * dpc);
+  qd.sh.resize(nq * dpc);
+  std::vector<double> &N = qd.sh;
+  std::vector<double> dx(nq * dpc), dy(nq * dpc);
   for (int q = 0; q < nq; ++q)
     lagrange_q(dpc, rule.pts[2 * q], rule.pts[2 * q + 1], &N[q * dpc], &dx[q * dpc], &dy[q * dpc]);
-  for (int64_t c = 0; c < m.ncells; ++c) {
+  parallel_for(m.ncells, 1024, [&](int64_t c) {
     const double *G = &m.geom[c * dpc * 3];
     for (int q = 0; q < nq; ++q) {
       double x[3] = {0, 0, 0}, a[3] = {0, 0, 0}, b[3] = {0, 0, 0};
@@ -169,9 +170,8 @@ void compute_quad_data(const HostMesh &m, const Quadrature2D &rule, QuadData &qd
         qd.n[3 * g + k] = cr[k] / J;
       }
       qd.jxw[g] = J * rule.w[q];
-      for (int j = 0; j < dpc; ++j) qd.sh[g * dpc + j] = N[q * dpc + j];
     }
-  }
+  });
 }
 
 // ---------------------------------------------------------------------------
@@ -220,7 +220,8 @@ void build_tree(const HostMesh &m, const QuadData &qd, int L, int max_nodes, Tre
   std::iota(t.nperm.begin(), t.nperm.end(), 0);
   t.qperm.resize(NQ);
   std::iota(t.qperm.begin(), t.qperm.end(), 0);
-  t.qblock.assign((size_t)(L + 1) * NQ, 0);
+  t.qblock.resize((size_t)(L + 1) * NQ);  // every level's entries are written below, level 0's are the root
+  std::fill(t.qblock.begin(), t.qblock.begin() + NQ, 0);
   t.startL.assign(L + 1, 0);
   t.endL.assign(L + 1, 0);
   t.dofs_filled.assign(L + 1, {});
@@ -244,15 +245,22 @@ void build_tree(const HostMesh &m, const QuadData &qd, int L, int max_nodes, Tre
   const double rootp[3] = {-1.1 * maxc, -1.1 * maxc, -1.1 * maxc};
   add_block(0, 0, rootp, delta, 0, (int)N, 0, (int)NQ);
 
-  std::vector<int32_t> parents = {0}, tmp;
-  std::vector<uint8_t> cls;
+  std::vector<int32_t> parents = {0};
+  struct Counts {
+    int n[8], q[8];
+  };
   for (int level = 1; level <= L; ++level) {
     delta /= 2.;
-    for (int P : parents) {
+    // stable partition of every parent's node and quad ranges into octants,
+    // the parents on host threads
+    std::vector<Counts> cnts(parents.size());
+    parallel_for((int64_t)parents.size(), 4, [&](int64_t ip) {
+      const int P = parents[ip];
       const double pm[3] = {t.pmin[3 * P], t.pmin[3 * P + 1], t.pmin[3 * P + 2]};
-      int cn[8] = {0}, cq[8] = {0};
-      // stable partition of the parent's node and quad ranges into octants
+      std::vector<int32_t> tmp;
+      std::vector<uint8_t> cls;
       auto part = [&](std::vector<int32_t> &perm, int beg, int cnt, const double *X, int *counts) {
+        std::fill(counts, counts + 8, 0);
         cls.resize(cnt);
         for (int i = 0; i < cnt; ++i) {
           cls[i] = (uint8_t)child_index(pm, delta, X + 3 * (int64_t)perm[beg + i]);
@@ -265,8 +273,13 @@ void build_tree(const HostMesh &m, const QuadData &qd, int L, int max_nodes, Tre
         for (int i = 0; i < cnt; ++i) tmp[off[cls[i]]++] = perm[beg + i];
         std::copy(tmp.begin(), tmp.begin() + cnt, perm.begin() + beg);
       };
-      part(t.nperm, t.node_beg[P], t.node_cnt[P], m.xyz.data(), cn);
-      part(t.qperm, t.quad_beg[P], t.quad_cnt[P], qd.x.data(), cq);
+      part(t.nperm, t.node_beg[P], t.node_cnt[P], m.xyz.data(), cnts[ip].n);
+      part(t.qperm, t.quad_beg[P], t.quad_cnt[P], qd.x.data(), cnts[ip].q);
+    });
+    for (size_t ip = 0; ip < parents.size(); ++ip) {
+      const int P = parents[ip];
+      const double pm[3] = {t.pmin[3 * P], t.pmin[3 * P + 1], t.pmin[3 * P + 2]};
+      const int *cn = cnts[ip].n, *cq = cnts[ip].q;
       int nb0 = t.node_beg[P], qb0 = t.quad_beg[P];
       for (int c = 0; c < 8; ++c) {
         if (cn[c] + cq[c] > 0) {
@@ -275,7 +288,6 @@ void build_tree(const HostMesh &m, const QuadData &qd, int L, int max_nodes, Tre
           const int id = add_block(level, P, cp, delta, nb0, cn[c], qb0, cq[c]);
           t.child[8 * P + t.nchild[P]++] = id;
           t.octant[id] = c;
-          for (int i = 0; i < cq[c]; ++i) t.qblock[(size_t)level * NQ + t.qperm[qb0 + i]] = id;
         }
         nb0 += cn[c];
         qb0 += cq[c];
@@ -292,13 +304,18 @@ void build_tree(const HostMesh &m, const QuadData &qd, int L, int max_nodes, Tre
       }
       if (std::round(bn) <= max_nodes) {
         t.leaves.push_back(b);
-        for (int i = 0; i < t.quad_cnt[b]; ++i)
-          for (int k = level + 1; k <= L; ++k) t.qblock[(size_t)k * NQ + t.qperm[t.quad_beg[b] + i]] = b;
       } else {
         next.push_back(b);
       }
       if (bn > 0) t.dofs_filled[level].push_back(b);
     }
+    // the block of each quad point at this level, and a leaf's at all deeper ones
+    parallel_for(t.endL[level] - t.startL[level] + 1, 16, [&](int64_t kb) {
+      const int b = t.startL[level] + (int)kb;
+      const int last = std::binary_search(next.begin(), next.end(), b) ? level : L;
+      for (int i = 0; i < t.quad_cnt[b]; ++i)
+        for (int k = level; k <= last; ++k) t.qblock[(size_t)k * NQ + t.qperm[t.quad_beg[b] + i]] = b;
+    });
     parents.swap(next);
   }
   for (int b : parents) t.leaves.push_back(b);
@@ -357,12 +374,25 @@ void build_tree(const HostMesh &m, const QuadData &qd, int L, int max_nodes, Tre
         }
       }
       sort_unique(cells);
+      // the blocks that hold those cells' quad points at each level; childless
+      // ones stay the same at all deeper levels
+      std::vector<int32_t> holders;
+      bool final_ = false;
       for (int s = 0; s < t.nsub[b]; ++s) {
         std::vector<int32_t> &il = t.il[t.sub_beg[b] + s];
         il = t.nn[t.sub_beg[b] + s];
-        const size_t lev = level + s;
-        for (int c : cells)
-          for (int q = 0; q < qd.nq; ++q) il.push_back(t.qblock[lev * NQ + (int64_t)c * qd.nq + q]);
+        if (!final_) {
+          const size_t lev = level + s;
+          holders.clear();
+          for (int c : cells)
+            for (int q = 0; q < qd.nq; ++q) {
+              const int x = t.qblock[lev * NQ + (int64_t)c * qd.nq + q];
+              if (holders.empty() || holders.back() != x) holders.push_back(x);
+            }
+          sort_unique(holders);
+          final_ = std::all_of(holders.begin(), holders.end(), [&](int x) { return t.nchild[x] == 0; });
+        }
+        il.insert(il.end(), holders.begin(), holders.end());
         sort_unique(il);
       }
       for (int s = 0; s < t.nsub[b]; ++s) {
@@ -415,109 +445,174 @@ void parallel_for(int64_t n, int64_t grain, const std::function<void(int64_t)> &
 }
 
 // The near field of one leaf: its entries (cell, quad-point mask, near
-// flag), the column of each entry's DoFs and its sorted rows and columns.
+// flag) and its sorted rows and columns.
 namespace {
 struct LeafNear {
-  std::vector<int32_t> ent_cell, ent_colpos, rows, cols;
+  std::vector<int32_t> ent_cell, rows, cols;
   std::vector<uint64_t> ent_mask;
   std::vector<uint8_t> ent_near;
 };
 
-void leaf_near(const HostMesh &m, const QuadData &qd, const Tree &t, int leaf, LeafNear &o) {
+// The quad points of every childless block as (cell, mask) runs, cells
+// ascending (a block's points keep their ascending order in qperm): what the
+// near lists are made of, so that a leaf merges cells and not points.
+struct BlockCells {
+  std::vector<int64_t> beg;
+  std::vector<int32_t> cell;
+  std::vector<uint64_t> mask;
+};
+BlockCells block_cells(const QuadData &qd, const Tree &t) {
+  BlockCells o;
+  o.beg.assign(t.nb + 1, 0);
+  for (int b = 0; b < t.nb; ++b) {
+    int last = -1;
+    for (int i = 0; t.nchild[b] == 0 && i < t.quad_cnt[b]; ++i) {
+      const int g = t.qperm[t.quad_beg[b] + i], c = g / qd.nq;
+      if (c != last) {
+        o.cell.push_back(c);
+        o.mask.push_back(0);
+        last = c;
+      }
+      o.mask.back() |= (uint64_t)1 << (g - c * qd.nq);
+    }
+    o.beg[b + 1] = (int64_t)o.cell.size();
+  }
+  return o;
+}
+
+// One worker's marks: the mask gathered per cell, and the leaf that last
+// marked a DoF.
+struct NearScratch {
+  std::vector<uint64_t> mask;
+  std::vector<int32_t> dof, cells;
+};
+
+// Sorts v, distinct numbers below n: by looking has(i) up for every i where v
+// holds a good part of them.
+template <typename Has>
+void sort_marked(std::vector<int32_t> &v, int64_t n, const Has &has) {
+  if ((int64_t)v.size() * 16 < n) {
+    std::sort(v.begin(), v.end());
+    return;
+  }
+  size_t k = 0;
+  for (int32_t i = 0; k < v.size() && i < n; ++i)
+    if (has(i)) v[k++] = i;
+}
+
+void leaf_near(const HostMesh &m, const QuadData &qd, const Tree &t, const BlockCells &bc, int leaf, int stamp,
+               NearScratch &s, LeafNear &o) {
   const int dpc = m.dpc;
-  std::vector<int32_t> qs;
-  auto add_entries = [&](std::vector<int32_t> &q, uint8_t near) {
-    sort_unique(q);
-    size_t i = 0;
-    while (i < q.size()) {
-      const int cell = q[i] / qd.nq;
-      uint64_t mask = 0;
-      while (i < q.size() && q[i] / qd.nq == cell) mask |= (uint64_t)1 << (q[i++] % qd.nq);
-      o.ent_cell.push_back(cell);
-      o.ent_mask.push_back(mask);
-      o.ent_near.push_back(near && cell < m.ncells_real);  // mirror images are never singular
+  auto add_block = [&](int b) {
+    auto add = [&](int c, uint64_t mask) {
+      if (!s.mask[c]) s.cells.push_back(c);
+      s.mask[c] |= mask;
+    };
+    if (t.nchild[b] == 0) {
+      for (int64_t i = bc.beg[b]; i < bc.beg[b + 1]; ++i) add(bc.cell[i], bc.mask[i]);
+    } else {
+      for (int i = 0; i < t.quad_cnt[b]; ++i) {
+        const int g = t.qperm[t.quad_beg[b] + i], c = g / qd.nq;
+        add(c, (uint64_t)1 << (g - c * qd.nq));
+      }
     }
   };
-  auto quads_of = [&](int b, std::vector<int32_t> &q) {
-    for (int i = 0; i < t.quad_cnt[b]; ++i) q.push_back(t.qperm[t.quad_beg[b] + i]);
+  auto add_entries = [&](uint8_t near) {
+    sort_marked(s.cells, m.ncells, [&](int c) { return s.mask[c] != 0; });
+    for (int c : s.cells) {
+      o.ent_cell.push_back(c);
+      o.ent_mask.push_back(s.mask[c]);
+      o.ent_near.push_back(near && c < m.ncells_real);  // mirror images are never singular
+      s.mask[c] = 0;
+    }
+    s.cells.clear();
   };
   // near quad points: blocks of the deepest intList
-  for (int b : t.il[t.sub_beg[leaf] + t.nsub[leaf] - 1]) quads_of(b, qs);
-  add_entries(qs, 1);
+  for (int b : t.il[t.sub_beg[leaf] + t.nsub[leaf] - 1]) add_block(b);
+  add_entries(1);
   // bigger far blocks in the nonIntLists of the leaf and of every ancestor
   for (int a = leaf; a != 0; a = t.parent[a]) {
     const int lev = t.level[a];
-    qs.clear();
-    for (int s = 0; s < t.nsub[a]; ++s)
-      for (int b : t.nil[t.sub_beg[a] + s])
-        if (b < t.startL[lev]) quads_of(b, qs);
-    if (!qs.empty()) add_entries(qs, 0);
+    for (int q = 0; q < t.nsub[a]; ++q)
+      for (int b : t.nil[t.sub_beg[a] + q])
+        if (b < t.startL[lev]) add_block(b);
+    add_entries(0);
   }
-  const size_t ne = o.ent_cell.size();
-  for (size_t e = 0; e < ne; ++e)
-    for (int j = 0; j < dpc; ++j) o.cols.push_back(m.cdofs[(int64_t)o.ent_cell[e] * dpc + j]);
-  sort_unique(o.cols);
-  o.ent_colpos.reserve(ne * dpc);
-  for (size_t e = 0; e < ne; ++e)
+  for (int c : o.ent_cell)
     for (int j = 0; j < dpc; ++j) {
-      const int d = m.cdofs[(int64_t)o.ent_cell[e] * dpc + j];
-      o.ent_colpos.push_back((int32_t)(std::lower_bound(o.cols.begin(), o.cols.end(), d) - o.cols.begin()));
+      const int d = m.cdofs[(int64_t)c * dpc + j];
+      if (s.dof[d] != stamp) {
+        s.dof[d] = stamp;
+        o.cols.push_back(d);
+      }
     }
+  sort_marked(o.cols, m.n, [&](int d) { return s.dof[d] == stamp; });
   o.rows.assign(t.nperm.begin() + t.node_beg[leaf], t.nperm.begin() + t.node_beg[leaf] + t.node_cnt[leaf]);
   std::sort(o.rows.begin(), o.rows.end());
 }
 }  // namespace
 
 // Leaves are independent: each is built on a host thread, then they are
-// concatenated in leaf order, so the plan does not depend on the threads.
+// copied into place in leaf order, so the plan does not depend on the threads.
+// Merging the blocks' cells by marks instead of sorting quad points, and
+// leaving the entries' column positions to the GPU (k_entry_cols): a
+// 12,376-DoF hull mirrored at its waterline (20.8 M entries; the whole of
+// pbfmm_direct_integrals) 800 -> 70 ms, 98,306 DoFs (Q2, leaf 80) 64 -> 24 ms.
 void build_near_plan(const HostMesh &m, const QuadData &qd, const Tree &t, NearPlan &np) {
   np = NearPlan();
   if (qd.nq > 64) throw std::runtime_error("quadrature order above 8 is not supported");
   std::vector<int> leaves;
   for (int leaf : t.leaves)
     if (t.node_cnt[leaf] > 0) leaves.push_back(leaf);
-  std::vector<LeafNear> part(leaves.size());
-  parallel_for((int64_t)leaves.size(), 64, [&](int64_t k) { leaf_near(m, qd, t, leaves[k], part[k]); });
-  size_t ne = 0, nr = 0, nc = 0;
-  for (const auto &o : part) {
-    ne += o.ent_cell.size();
-    nr += o.rows.size();
-    nc += o.cols.size();
+  const int64_t nl = (int64_t)leaves.size();
+  std::vector<LeafNear> part(nl);
+  {
+    const BlockCells bc = block_cells(qd, t);
+    std::atomic<int64_t> next{0};
+    constexpr int64_t kTake = 8;
+    parallel_for(std::min<int64_t>(16, (nl + 63) / 64), 1, [&](int64_t) {  // one call per worker
+      NearScratch s;
+      s.mask.assign(m.ncells, 0);
+      s.dof.assign(m.n, -1);
+      for (int64_t k0; (k0 = next.fetch_add(kTake)) < nl;)
+        for (int64_t k = k0; k < std::min(nl, k0 + kTake); ++k) leaf_near(m, qd, t, bc, leaves[k], (int)k, s, part[k]);
+    });
   }
-  np.ent_cell.reserve(ne);
-  np.ent_mask.reserve(ne);
-  np.ent_near.reserve(ne);
-  np.ent_colpos.reserve(ne * m.dpc);
-  np.rows.reserve(nr);
-  np.row_leaf.reserve(nr);
-  np.cols.reserve(nc);
-  np.row_beg.push_back(0);
-  np.col_beg.push_back(0);
-  np.ent_beg.push_back(0);
-  np.work_beg.push_back(0);
-  for (size_t k = 0; k < leaves.size(); ++k) {
-    LeafNear &o = part[k];
-    const int64_t e0 = (int64_t)np.ent_cell.size();
-    np.ent_cell.insert(np.ent_cell.end(), o.ent_cell.begin(), o.ent_cell.end());
-    np.ent_mask.insert(np.ent_mask.end(), o.ent_mask.begin(), o.ent_mask.end());
-    np.ent_near.insert(np.ent_near.end(), o.ent_near.begin(), o.ent_near.end());
-    np.ent_colpos.insert(np.ent_colpos.end(), o.ent_colpos.begin(), o.ent_colpos.end());
-    const int64_t e1 = (int64_t)np.ent_cell.size();
+  np.row_beg.assign(1, 0);
+  np.col_beg.assign(1, 0);
+  np.ent_beg.assign(1, 0);
+  int64_t ne = 0, nr = 0, nc = 0;
+  for (int64_t k = 0; k < nl; ++k) {
+    const LeafNear &o = part[k];
+    ne += (int64_t)o.ent_cell.size();
+    nr += (int64_t)o.rows.size();
+    nc += (int64_t)o.cols.size();
+    if (ne >= (int64_t(1) << 31) || nc >= (int64_t(1) << 31))
+      throw std::runtime_error("near field: more than 2^31 entries or leaf columns");
     np.val_beg.push_back(np.nnz);
     np.nnz += (int64_t)o.rows.size() * (int64_t)o.cols.size();
-    for (int r : o.rows) {
-      np.rows.push_back(r);
-      np.row_leaf.push_back(np.nleaf);
-    }
-    np.cols.insert(np.cols.end(), o.cols.begin(), o.cols.end());
     np.leaf_block.push_back(leaves[k]);
-    np.row_beg.push_back((int32_t)np.rows.size());
-    np.col_beg.push_back((int32_t)np.cols.size());
-    np.ent_beg.push_back((int32_t)e1);
-    np.work_beg.push_back(np.work_beg.back() + (int64_t)o.rows.size() * (e1 - e0));
+    np.row_beg.push_back((int32_t)nr);
+    np.col_beg.push_back((int32_t)nc);
+    np.ent_beg.push_back((int32_t)ne);
     np.nleaf++;
-    o = LeafNear();  // free as we go
   }
+  np.ent_cell.resize(ne);
+  np.ent_mask.resize(ne);
+  np.ent_near.resize(ne);
+  np.cols.resize(nc);
+  np.rows.resize(nr);
+  np.row_leaf.resize(nr);
+  parallel_for(nl, 16, [&](int64_t k) {
+    LeafNear &o = part[k];
+    std::copy(o.ent_cell.begin(), o.ent_cell.end(), np.ent_cell.begin() + np.ent_beg[k]);
+    std::copy(o.ent_mask.begin(), o.ent_mask.end(), np.ent_mask.begin() + np.ent_beg[k]);
+    std::copy(o.ent_near.begin(), o.ent_near.end(), np.ent_near.begin() + np.ent_beg[k]);
+    std::copy(o.cols.begin(), o.cols.end(), np.cols.begin() + np.col_beg[k]);
+    std::copy(o.rows.begin(), o.rows.end(), np.rows.begin() + np.row_beg[k]);
+    std::fill(np.row_leaf.begin() + np.row_beg[k], np.row_leaf.begin() + np.row_beg[k + 1], (int32_t)k);
+    o = LeafNear();  // free as we go
+  });
 }
 
 // ---------------------------------------------------------------------------
@@ -551,6 +646,26 @@ double Anm(int n, int m) {
   for (int i = n + m; i > 0; --i) f2 *= i;
   return ((n & 1) ? -1.0 : 1.0) / std::sqrt(f1 * f2);
 }
+// its values for degrees up to 2 p, p <= 10
+struct AnmTable {
+  double a[21][21];
+  AnmTable() {
+    for (int n = 0; n <= 20; ++n)
+      for (int m = 0; m <= n; ++m) a[n][m] = Anm(n, m);
+  }
+  double operator()(int n, int m) const { return a[n][std::abs(m)]; }
+};
+const AnmTable kA;
+// cos and sin of k beta and powers of rho, for |k| up to 2 p
+struct Angles {
+  double c[41], s[41], pw[22], ipw[22];
+  Angles(double beta, double rho) {
+    for (int k = -20; k <= 20; ++k) c[k + 20] = std::cos(k * beta), s[k + 20] = std::sin(k * beta);
+    for (int k = 0; k <= 21; ++k) pw[k] = std::pow(rho, double(k)), ipw[k] = std::pow(rho, double(-k));
+  }
+  double cos(int k) const { return c[k + 20]; }
+  double sin(int k) const { return s[k + 20]; }
+};
 double ire(int k) {  // Re(i^k), k even
   const int r = ((k % 4) + 4) % 4;
   return r == 0 ? 1.0 : (r == 2 ? -1.0 : 0.0);
@@ -579,15 +694,15 @@ void op_m2m(int p, const double d[3], double *opT) {
   double rho, ca, beta;
   sph(d, rho, ca, beta);
   Leg P(p, ca);
+  const Angles an(beta, rho);
   for (int n = 0; n <= p; ++n)
     for (int m = 0; m <= n; ++m)
       for (int nn = 0; nn <= n; ++nn)
         for (int mm = -nn; mm <= nn; ++mm) {
           if (std::abs(m - mm) > n - nn) continue;
-          double rf = P(nn, std::abs(mm)) * std::pow(rho, double(nn)) * Anm(nn, mm) * Anm(n - nn, m - mm) / Anm(n, m);
+          double rf = P(nn, std::abs(mm)) * an.pw[nn] * kA(nn, mm) * kA(n - nn, m - mm) / kA(n, m);
           rf *= ire(std::abs(m) - std::abs(mm) - std::abs(m - mm));
-          put(opT, kt, kp, tri(n, m), tri(n - nn, std::abs(m - mm)), rf * std::cos(mm * beta),
-              -rf * std::sin(mm * beta), sgn(m - mm));
+          put(opT, kt, kp, tri(n, m), tri(n - nn, std::abs(m - mm)), rf * an.cos(mm), -rf * an.sin(mm), sgn(m - mm));
         }
 }
 
@@ -598,17 +713,17 @@ void op_l2l(int p, const double d[3], double *opT) {
   double rho, ca, beta;
   sph(d, rho, ca, beta);
   Leg P(p, ca);
+  const Angles an(beta, rho);
   for (int n = 0; n <= p; ++n)
     for (int m = 0; m <= n; ++m)
       for (int nn = n; nn <= p; ++nn) {
-        const double rf0 = std::pow(rho, double(nn - n));
+        const double rf0 = an.pw[nn - n];
         for (int mm = -nn; mm <= nn; ++mm) {
           if (std::abs(mm - m) > nn - n) continue;
-          double c = Anm(nn - n, mm - m) / Anm(nn, mm) * Anm(n, m) * ire(std::abs(mm) - std::abs(mm - m) - std::abs(m)) *
+          double c = kA(nn - n, mm - m) / kA(nn, mm) * kA(n, m) * ire(std::abs(mm) - std::abs(mm - m) - std::abs(m)) *
                      (((nn + n) & 1) ? -1.0 : 1.0);
           const double rf = P(nn - n, std::abs(mm - m)) * rf0 * c;
-          put(opT, kt, kp, tri(n, m), tri(nn, std::abs(mm)), rf * std::cos((mm - m) * beta),
-              rf * std::sin((mm - m) * beta), sgn(mm));
+          put(opT, kt, kp, tri(n, m), tri(nn, std::abs(mm)), rf * an.cos(mm - m), rf * an.sin(mm - m), sgn(mm));
         }
       }
 }
@@ -620,16 +735,16 @@ void op_m2l(int p, const double d[3], double *opT) {
   double rho, ca, beta;
   sph(d, rho, ca, beta);
   Leg P(2 * p, ca);
+  const Angles an(beta, rho);
   for (int n = 0; n <= p; ++n)
     for (int m = 0; m <= n; ++m)
       for (int nn = 0; nn <= p; ++nn) {
-        const double rf0 = std::pow(rho, double(-n - nn - 1));
+        const double rf0 = an.ipw[n + nn + 1];
         for (int mm = -nn; mm <= nn; ++mm) {
-          double c = Anm(nn, mm) / Anm(n + nn, m - mm) * Anm(n, m) * ire(std::abs(m - mm) - std::abs(m) - std::abs(mm)) /
+          double c = kA(nn, mm) / kA(n + nn, m - mm) * kA(n, m) * ire(std::abs(m - mm) - std::abs(m) - std::abs(mm)) /
                      ((nn & 1) ? -1.0 : 1.0);
           const double rf = P(n + nn, std::abs(mm - m)) * rf0 * c;
-          put(opT, kt, kp, tri(n, m), tri(nn, std::abs(mm)), rf * std::cos((mm - m) * beta),
-              rf * std::sin((mm - m) * beta), mm < 0 ? -1 : 1);
+          put(opT, kt, kp, tri(n, m), tri(nn, std::abs(mm)), rf * an.cos(mm - m), rf * an.sin(mm - m), mm < 0 ? -1 : 1);
         }
       }
 }
@@ -670,8 +785,10 @@ static std::vector<int> row_degrees(int p, int kp) {
 
 // opT[k*kp + row] *= in_scale^deg(k) * out_scale^deg(row)
 static void scale_op(double *opT, int kp, const std::vector<int> &deg, double in_scale, double out_scale) {
+  double in[21], out[21];
+  for (int n = 0; n <= 20; ++n) in[n] = std::pow(in_scale, n), out[n] = std::pow(out_scale, n);
   for (int k = 0; k < kp; ++k)
-    for (int r = 0; r < kp; ++r) opT[(size_t)k * kp + r] *= std::pow(in_scale, deg[k]) * std::pow(out_scale, deg[r]);
+    for (int r = 0; r < kp; ++r) opT[(size_t)k * kp + r] *= in[deg[k]] * out[deg[r]];
 }
 
 void build_far_plan(const Tree &t, int p, FarPlan &fp) {
@@ -685,23 +802,28 @@ void build_far_plan(const Tree &t, int p, FarPlan &fp) {
   for (int b : t.leaves)
     if (t.node_cnt[b] > 0) fp.l2p_leaf.push_back(b);
 
-  // M2M / L2L operators per level and octant
-  fp.m2m_ops.assign((size_t)(L + 1) * 8 * kp * kp, 0.0);
-  fp.l2l_ops.assign((size_t)(L + 1) * 8 * kp * kp, 0.0);
-  for (int l = 1; l <= L; ++l) {
-    const double dl = t.delta[0] / std::pow(2.0, l);
-    for (int o = 0; o < 8; ++o) {
-      double d[3];
-      for (int k = 0; k < 3; ++k) d[k] = (kOffs[o][k] != 0 ? 0.5 : -0.5) * dl;
-      op_m2m(p, d, &fp.m2m_ops[((size_t)l * 8 + o) * kp * kp]);
+  // M2M / L2L operators per level and octant.  On level-scaled expansions
+  // (child ME/delta_l^n -> parent ME/delta_{l-1}^n, parent LE.delta_{l-1}^(n+1)
+  // -> child LE.delta_l^(n+1)) they are the same at every level: built once
+  // per octant for a child box of size 1 and copied.
+  const size_t op_sz = (size_t)kp * kp;
+  fp.m2m_ops.assign((size_t)(L + 1) * 8 * op_sz, 0.0);
+  fp.l2l_ops.assign((size_t)(L + 1) * 8 * op_sz, 0.0);
+  if (L >= 1) {
+    parallel_for(8, 1, [&](int64_t o) {
+      double d[3], *mm = &fp.m2m_ops[(8 + o) * op_sz], *ll = &fp.l2l_ops[(8 + o) * op_sz];
+      for (int k = 0; k < 3; ++k) d[k] = kOffs[o][k] != 0 ? 0.5 : -0.5;
+      op_m2m(p, d, mm);
       const double dn[3] = {-d[0], -d[1], -d[2]};
-      op_l2l(p, dn, &fp.l2l_ops[((size_t)l * 8 + o) * kp * kp]);
-      // level-scaled expansions: child ME/delta_l^n -> parent ME/delta_{l-1}^n,
-      // parent LE.delta_{l-1}^(n+1) -> child LE.delta_l^(n+1)
-      scale_op(&fp.m2m_ops[((size_t)l * 8 + o) * kp * kp], kp, deg, dl, 1.0 / (2.0 * dl));
-      scale_op(&fp.l2l_ops[((size_t)l * 8 + o) * kp * kp], kp, deg, 1.0 / (2.0 * dl), dl);
+      op_l2l(p, dn, ll);
+      scale_op(mm, kp, deg, 1.0, 0.5);
+      scale_op(ll, kp, deg, 0.5, 1.0);
       // the extra power of the box size: child delta / parent delta
-      for (size_t i = 0; i < (size_t)kp * kp; ++i) fp.l2l_ops[((size_t)l * 8 + o) * kp * kp + i] *= 0.5;
+      for (size_t i = 0; i < op_sz; ++i) ll[i] *= 0.5;
+    });
+    for (int l = 2; l <= L; ++l) {
+      std::copy_n(&fp.m2m_ops[8 * op_sz], 8 * op_sz, &fp.m2m_ops[(size_t)l * 8 * op_sz]);
+      std::copy_n(&fp.l2l_ops[8 * op_sz], 8 * op_sz, &fp.l2l_ops[(size_t)l * 8 * op_sz]);
     }
   }
   // M2M pairs (bem_fma.cc:2318-2339: every block of level l into its parent)
@@ -747,6 +869,8 @@ void build_far_plan(const Tree &t, int p, FarPlan &fp) {
     fp.m2l.level_off[l] = (int)fp.m2l.op.size();
     fp.m2l.level_off1[l] = (int)fp.m2l.op1.size();
     std::map<std::array<int, 3>, std::vector<std::pair<int, int>>> cls;
+    // the class of an offset within +-4 boxes (all but augmented lists' ones) without a search
+    std::vector<std::pair<int, int>> *near_cls[9][9][9] = {};
     const double dl = t.delta[0] / std::pow(2.0, l);
     for (int b : t.dofs_filled[l]) {
       double cb[3];
@@ -758,7 +882,13 @@ void build_far_plan(const Tree &t, int p, FarPlan &fp) {
             t.center(src, cs);
             std::array<int, 3> key;
             for (int k = 0; k < 3; ++k) key[k] = (int)std::lround((cs[k] - cb[k]) / dl);
-            cls[key].push_back({b, src});
+            if (std::abs(key[0]) <= 4 && std::abs(key[1]) <= 4 && std::abs(key[2]) <= 4) {
+              std::vector<std::pair<int, int>> *&v = near_cls[key[0] + 4][key[1] + 4][key[2] + 4];
+              if (!v) v = &cls[key];
+              v->push_back({b, src});
+            } else {
+              cls[key].push_back({b, src});
+            }
           } else if (src > t.endL[l]) {
             fp.m2p_tgt.push_back(b);
             fp.m2p_src.push_back(src);
@@ -834,6 +964,33 @@ static void compose_ops(const double *A, const double *B, int kp, double *C) {
     }
 }
 
+// Composite two-level operators by (octant, octant of the child), the same
+// for every pair of levels as the single ones are, numbered on first use.
+struct Composites {
+  int ids[64], n = 0;
+  std::vector<int> keys;
+  Composites() { std::fill(ids, ids + 64, -1); }
+  int id(int o, int go) {
+    int &v = ids[o * 8 + go];
+    if (v < 0) {
+      v = n++;
+      keys.push_back(o * 8 + go);
+    }
+    return v;
+  }
+  // appends them to the single operators; order gives the octants of the
+  // operator that acts last and of the one that acts first
+  template <typename Order>
+  void append(std::vector<double> &ops, int kp, const Order &order) const {
+    const size_t sz = (size_t)kp * kp, at = ops.size();
+    ops.resize(at + n * sz);
+    parallel_for(n, 1, [&](int64_t k) {
+      const std::pair<int, int> q = order(keys[k] / 8, keys[k] % 8);
+      compose_ops(&ops[(8 + q.first) * sz], &ops[(8 + q.second) * sz], kp, &ops[at + k * sz]);
+    });
+  }
+};
+
 // The upward pass in half the launches: M2M child levels a and a - 1 in one
 // launch.  The targets at level a - 1 take their children at level a as
 // usual; the targets at level a - 2 take their leaf children at level a - 1
@@ -852,15 +1009,12 @@ void build_m2m_groups(const Tree &t, FarPlan &fp) {
   for (int l = 1; l <= L; ++l)
     if (fp.m2l_per_level[l] > 0) me_lo = std::min(me_lo, l);
   for (int b : fp.m2p_src) me_lo = std::min(me_lo, (int)t.level[b]);
-  const size_t base = fp.m2m_ops.size() / ((size_t)kp * kp);
-  std::vector<double> comp;  // appended composite operators
-  int ncomp = 0;
+  const int base = (int)(fp.m2m_ops.size() / ((size_t)kp * kp));
+  Composites comp;
   for (int a = L; a > me_lo; a -= 2) {
     std::map<int, std::vector<std::pair<int, int>>> cls;
     for (int b = t.startL[a]; b <= t.endL[a]; ++b) cls[a * 8 + t.octant[b]].push_back({t.parent[b], b});
     if (a - 1 > me_lo) {
-      // composite operators of this level pair, on first use
-      std::vector<int> cop(64, -1);
       for (int c = t.startL[a - 1]; c <= t.endL[a - 1]; ++c) {
         if (t.nchild[c] == 0) {
           cls[(a - 1) * 8 + t.octant[c]].push_back({t.parent[c], c});
@@ -868,15 +1022,7 @@ void build_m2m_groups(const Tree &t, FarPlan &fp) {
         }
         for (int q = 0; q < t.nchild[c]; ++q) {
           const int gc = t.child[8 * c + q];
-          const int key = t.octant[c] * 8 + t.octant[gc];
-          if (cop[key] < 0) {
-            cop[key] = ncomp++;
-            comp.resize(comp.size() + (size_t)kp * kp);
-            compose_ops(&fp.m2m_ops[((size_t)(a - 1) * 8 + t.octant[c]) * kp * kp],
-                        &fp.m2m_ops[((size_t)a * 8 + t.octant[gc]) * kp * kp], kp,
-                        &comp[comp.size() - (size_t)kp * kp]);
-          }
-          cls[-1 - (int)(base + cop[key])].push_back({t.parent[c], gc});
+          cls[-1 - (base + comp.id(t.octant[c], t.octant[gc]))].push_back({t.parent[c], gc});
         }
       }
     }
@@ -884,7 +1030,8 @@ void build_m2m_groups(const Tree &t, FarPlan &fp) {
     fp.m2m_g.level_off1.push_back((int)fp.m2m_g.op1.size());
     fp.m2m_g.level_off.push_back((int)fp.m2m_g.op.size());
   }
-  fp.m2m_ops.insert(fp.m2m_ops.end(), comp.begin(), comp.end());
+  // T_{a-1}(octant c) T_a(octant gc): the child's operator acts first
+  comp.append(fp.m2m_ops, kp, [](int o, int go) { return std::make_pair(o, go); });
 }
 
 // The downward pass in half the launches: L2L into target levels l and
@@ -905,16 +1052,14 @@ void build_l2l_groups(const Tree &t, FarPlan &fp) {
   int le_lo = L + 1;
   for (int l = 1; l <= L; ++l)
     if (fp.m2l_per_level[l] > 0) le_lo = std::min(le_lo, l);
-  const size_t base = fp.l2l_ops.size() / ((size_t)kp * kp);
+  const int base = (int)(fp.l2l_ops.size() / ((size_t)kp * kp));
   std::vector<char> filled(t.level.size(), 0);
   for (int l = 0; l <= L; ++l)
     for (int b : t.dofs_filled[l]) filled[b] = 1;
-  std::vector<double> comp;
-  int ncomp = 0;
+  Composites comp;
   for (int l = std::max(2, le_lo + 1); l <= L; l += 2) {
     std::map<int, std::vector<std::pair<int, int>>> cls;
     const bool pair = l + 1 <= L;
-    std::vector<int> cop(64, -1);
     for (int b : t.dofs_filled[l]) {
       if (!pair || t.nchild[b] == 0) {
         cls[l * 8 + t.octant[b]].push_back({b, t.parent[b]});
@@ -924,21 +1069,15 @@ void build_l2l_groups(const Tree &t, FarPlan &fp) {
         const int gc = t.child[8 * b + q];
         if (!filled[gc]) continue;
         cls[(l + 1) * 8 + t.octant[gc]].push_back({gc, b});
-        const int key = t.octant[b] * 8 + t.octant[gc];
-        if (cop[key] < 0) {
-          cop[key] = ncomp++;
-          comp.resize(comp.size() + (size_t)kp * kp);
-          compose_ops(&fp.l2l_ops[((size_t)(l + 1) * 8 + t.octant[gc]) * kp * kp],
-                      &fp.l2l_ops[((size_t)l * 8 + t.octant[b]) * kp * kp], kp, &comp[comp.size() - (size_t)kp * kp]);
-        }
-        cls[-1 - (int)(base + cop[key])].push_back({gc, t.parent[b]});
+        cls[-1 - (base + comp.id(t.octant[b], t.octant[gc]))].push_back({gc, t.parent[b]});
       }
     }
     for (auto &kv : cls) add_class(fp.l2l_g, kv.first >= 0 ? kv.first : -1 - kv.first, kv.second);
     fp.l2l_g.level_off1.push_back((int)fp.l2l_g.op1.size());
     fp.l2l_g.level_off.push_back((int)fp.l2l_g.op.size());
   }
-  fp.l2l_ops.insert(fp.l2l_ops.end(), comp.begin(), comp.end());
+  // T_{l+1}(octant gc) T_l(octant b): the parent's operator acts first
+  comp.append(fp.l2l_ops, kp, [](int o, int go) { return std::make_pair(go, o); });
 }
 
 // The image of cell c is the reflection x -> (x, y, 2 z0 - z) of its mapping
@@ -981,9 +1120,11 @@ void build_p2m_plan(const HostMesh &m, const QuadData &qd, const Tree &t, FarPla
     const int b = fp.p2m_leaf[li];
     const int beg = t.quad_beg[b], cnt = t.quad_cnt[b];
     std::vector<int32_t> &c = cols[li];
-    c.reserve((size_t)cnt * dpc);
+    int64_t last = -1;  // a block's points come cell by cell
     for (int i = 0; i < cnt; ++i) {
       const int64_t cell = t.qperm[beg + i] / nq;
+      if (cell == last) continue;
+      last = cell;
       for (int j = 0; j < dpc; ++j) c.push_back(m.cdofs[cell * dpc + j]);
     }
     std::sort(c.begin(), c.end());
@@ -998,7 +1139,6 @@ void build_p2m_plan(const HostMesh &m, const QuadData &qd, const Tree &t, FarPla
   fp.p2m_col_dof.assign(fp.p2m_col_beg[nleaf], 0);
   fp.p2m_qpt.assign(qbeg[nleaf], 0);
   fp.p2m_qleaf.assign(qbeg[nleaf], 0);
-  fp.p2m_qcol.assign((size_t)qbeg[nleaf] * dpc, 0);
   parallel_for(nleaf, 64, [&](int64_t li) {
     const int b = fp.p2m_leaf[li];
     const int beg = t.quad_beg[b], cnt = t.quad_cnt[b];
@@ -1007,14 +1147,8 @@ void build_p2m_plan(const HostMesh &m, const QuadData &qd, const Tree &t, FarPla
     std::copy(c.begin(), c.end(), fp.p2m_col_dof.begin() + c0);
     for (int i = 0; i < cnt; ++i) {
       const int64_t q = qbeg[li] + i;
-      const int g = t.qperm[beg + i];
-      const int64_t cell = g / nq;
-      fp.p2m_qpt[q] = g;
+      fp.p2m_qpt[q] = t.qperm[beg + i];
       fp.p2m_qleaf[q] = (int32_t)li;
-      for (int j = 0; j < dpc; ++j) {
-        const int d = m.cdofs[cell * dpc + j];
-        fp.p2m_qcol[q * dpc + j] = c0 + (int)(std::lower_bound(c.begin(), c.end(), d) - c.begin());
-      }
     }
   });
 }
