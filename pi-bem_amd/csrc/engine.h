@@ -229,6 +229,7 @@ struct Engine {
   std::vector<int64_t> graph_key(int precision) const;
   void drop_graphs();
   int use_side_fusion(bool f32);
+  int first_plan(bool f32) const;
   // near-field SpMV kernel per precision ([0] FP64, [1] FP32) and storage
   // (pairs, single values): 0 workgroup per leaf with an LDS copy of the
   // columns, 1 wavefront per leaf with 2 rows in flight, 2 with 4 rows, 3 (6

@@ -3151,8 +3151,10 @@ static void launch_spmm(Engine &e, const double *x, double *out, int R) {
 // problems of 602 to 393,218 DoFs and leaf sizes 20 to 96).  Single values:
 // column vectors, and the wavefront per leaf, which is faster for many narrow
 // leaves (393,218 DoFs, leaf 20: 0.158 against 0.253 ms FP32, 0.245 against
-// 0.303 ms FP64; leaf 80: 0.492 against 0.354, 0.929 against 0.674).  The
-// others stay for pbfmm_set_spmv_kernel.  A kernel whose first launch takes
+// 0.303 ms FP64; leaf 80: 0.492 against 0.354, 0.929 against 0.674); FP32 with
+// few values also the workgroup per leaf, row-major and in row pairs (24,578
+// DoFs, leaf 20: 16.4 and 14.7 us, column vectors 17.2 us).  The others stay
+// for pbfmm_set_spmv_kernel.  A kernel whose first launch takes
 // half as long again as the best time so far is not timed further.
 template <typename T, int NK>
 void Engine::tune_spmv() {
@@ -3173,8 +3175,19 @@ void Engine::tune_spmv() {
   const int first = NK == 2 ? 0 : kColsVariant<T>;
   int pick = first;
   (void)timed(first, 1);
-  const float best = timed(first, 2);
-  if (timed(1, 1) < 1.5f * best && timed(1, 2) < best) pick = 1;
+  float best = timed(first, 2);
+  auto against = [&](int v) {
+    if (timed(v, 1) >= 1.5f * best) return;
+    const float ms = timed(v, 2);
+    if (ms < best) best = ms, pick = v;
+  };
+  against(1);
+  if (kPairedF32<T, NK> && near.nnz <= 16000000) {
+    against(0);
+    ensure_row_pairs();
+    against(3);
+    if (pick != 3) f32.opvals_p.release();
+  }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   spmv_variant[sizeof(T) == 4 ? 1 : 0][NK - 1] = pick;
@@ -3584,13 +3597,34 @@ double Engine::norm2(const double *v) {
 // DoFs, orders 4 to 8, leaf sizes 20 to 96, both precisions).  A plan other
 // than 0 is kept only if it beats plan 0 by 2%.  Timing costs two dozen
 // applications and a plan gains a tenth of one as a rule, so one solve does not
-// pay for it: the first kPlanAfter applications of a precision run plan 0
+// pay for it: the first kPlanAfter applications of a precision run first_plan
 // (98,306 DoFs, Q2, one mixed solve on a new handle: 75 ms of timing before a
 // solve of 16 ms).
+//
+// first_plan: the plan that the sizes suggest.  Measured at those problems,
+// us per application of plan 0 against the plan chosen, FP32 unless stated:
+//   few values (at most 3 M: the level launches wait on latency, the SpMV and
+//   M2P fit beside them): plan 3.  1,538 DoFs 27.4 / 24.5, 9,602 (leaf 20)
+//   68.4 / 59.3; FP64 32.6 / 27.0, 88.9 / 77.0; without M2P plan 0 (602 DoFs
+//   16.0, plan 3 16.4; 6,146 DoFs at leaf 64 33.0, plan 3 35.6).
+//   many M2L pairs beside them (24,578 DoFs, leaf 20, 7 M values): plan 5,
+//   100.1 / 84.5; FP64 133.4 / 114.6.
+//   larger, FP64 from 8 M and FP32 from 25 M values: the SpMV on the second
+//   stream, plan 24 (FP64 24,578 DoFs at leaf 96 89.7 / 85.2, 98,306 at leaf
+//   80 428 / 407; FP32 98,306 261 / 228, 393,218 775 / 641), with slots where
+//   M2L pairs are many for the values, FP32: plan 92 (38,402 DoFs at leaf 20
+//   136 / 114, 98,306 at leaf 32 236 / 202).
+int Engine::first_plan(bool f32) const {
+  const int64_t nnz = near.nnz, m2l = (int64_t)far.m2l.tgt.size(), m2p = (int64_t)far.m2p_item_node.size();
+  if (nnz <= 3000000) return m2p > nnz / 1000 ? 3 : 0;
+  if (nnz <= 10000000 && m2l >= 100000) return 5;
+  if (f32 && nnz >= 10000000 && m2l > nnz / 200) return 92;
+  return nnz >= (f32 ? 25000000 : 8000000) ? 24 : 0;
+}
 int Engine::use_side_fusion(bool f32) {
   int &mode = side_fusion[f32 ? 1 : 0];
   if (mode >= 0) return mode;
-  if (plan_apps[f32 ? 1 : 0]++ < kPlanAfter) return 0;
+  if (plan_apps[f32 ? 1 : 0]++ < kPlanAfter) return first_plan(f32);
   const unsigned g = nblk(n, 256);
   if (d_cost.bytes < (size_t)2 * n * 8) alloc(d_cost, (size_t)2 * n * 8);
   double *u = d_cost.as<double>(), *v = d_cost.as<double>() + n;
