@@ -902,9 +902,10 @@ int pbfmm_get_expansions(pbfmm_handle *h, int32_t which, double *k1, double *k2)
         for (int m = 0; m <= nn; ++m) {
           const int i = nn * (nn + 1) / 2 + m;
           k1[(size_t)b * 2 * kt + 2 * i] = v[(size_t)b * 2 * kp + i] * sc;
-          k1[(size_t)b * 2 * kt + 2 * i + 1] = v[(size_t)b * 2 * kp + kt + i] * sc;
+          const size_t im = (size_t)b * 2 * kp + (m > 0 ? im_row(kt, nn, m) : 0);
+          k1[(size_t)b * 2 * kt + 2 * i + 1] = m > 0 ? v[im] * sc : 0.0;
           k2[(size_t)b * 2 * kt + 2 * i] = v[(size_t)b * 2 * kp + kp + i] * sc;
-          k2[(size_t)b * 2 * kt + 2 * i + 1] = v[(size_t)b * 2 * kp + kp + kt + i] * sc;
+          k2[(size_t)b * 2 * kt + 2 * i + 1] = m > 0 ? v[kp + im] * sc : 0.0;
         }
       }
     return PBFMM_OK;

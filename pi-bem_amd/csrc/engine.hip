@@ -1002,6 +1002,9 @@ __device__ __forceinline__ T wave_allsum(T v) {
   return v;
 }
 
+// im_row on the device
+__device__ __forceinline__ int im_row_d(int kt, int n, int m) { return kt + n * (n - 1) / 2 + m - 1; }
+
 // Set-up, FP64: one thread per quad point of the leaves, atomics into U
 // (for leaves whose unit multipoles do not fit in LDS).
 __global__ void __launch_bounds__(256) k_p2m_unit(
@@ -1027,15 +1030,18 @@ __global__ void __launch_bounds__(256) k_p2m_unit(
   }
   // level-scaled multipoles: coefficient of degree n divided by delta^n
   const double inv_delta = 1.0 / delta[b];
-  auto emit = [&](int k, int n, double Rr, double Ri, double Gr, double Gi) {
+  auto emit = [&](int n, int m, double Rr, double Ri, double Gr, double Gi) {
     double sc = 1.0;
     for (int q = 0; q < n; ++q) sc *= inv_delta;
     Rr *= sc; Ri *= sc; Gr *= sc; Gi *= sc;
+    const int k = n * (n + 1) / 2 + m, ki = im_row_d(kt, n, m);
     for (int j = 0; j < dpc; ++j) {
       atomicAdd(col[j] + k, wj[j] * Gr);
-      atomicAdd(col[j] + kt + k, wj[j] * Gi);
       atomicAdd(col[j] + kp + k, wj[j] * Rr);
-      atomicAdd(col[j] + kp + kt + k, wj[j] * Ri);
+      if (m > 0) {
+        atomicAdd(col[j] + ki, wj[j] * Gi);
+        atomicAdd(col[j] + kp + ki, wj[j] * Ri);
+      }
     }
   };
   double Rmr = 1, Rmi = 0, Gmr = 0, Gmi = 0;  // R_m^m, D R_m^m
@@ -1048,13 +1054,13 @@ __global__ void __launch_bounds__(256) k_p2m_unit(
       Rmr = nr; Rmi = ni; Gmr = gr; Gmi = gi;
     }
     double Rcr = Rmr, Rci = Rmi, Gcr = Gmr, Gci = Gmi, Rpr = 0, Rpi = 0, Gpr = 0, Gpi = 0;
-    emit(m * (m + 1) / 2 + m, m, Rcr, Rci, Gcr, Gci);
+    emit(m, m, Rcr, Rci, Gcr, Gci);
     for (int n = m + 1; n <= p; ++n) {
       const double a = RA<double>(n, m), bb = RB<double>(n, m);
       const double Rnr = a * z * Rcr - bb * r2 * Rpr, Rni = a * z * Rci - bb * r2 * Rpi;
       const double Gnr = a * (nz * Rcr + z * Gcr) - bb * (dn2 * Rpr + r2 * Gpr);
       const double Gni = a * (nz * Rci + z * Gci) - bb * (dn2 * Rpi + r2 * Gpi);
-      emit(n * (n + 1) / 2 + m, n, Rnr, Rni, Gnr, Gni);
+      emit(n, m, Rnr, Rni, Gnr, Gni);
       Rpr = Rcr; Rpi = Rci; Gpr = Gcr; Gpi = Gci;
       Rcr = Rnr; Rci = Rni; Gcr = Gnr; Gci = Gni;
     }
@@ -1127,32 +1133,33 @@ __global__ void __launch_bounds__(256) k_p2m_unit_leaf(
       Rmr = nr; Rmi = ni; Gmr = gr; Gmi = gi;
       sc *= inv_delta;
     }
-    auto emit = [&](int k, double s, double Rr, double Ri, double Gr, double Gi) {
+    auto emit = [&](int n, double s, double Rr, double Ri, double Gr, double Gi) {
       Rr *= s; Ri *= s; Gr *= s; Gi *= s;
+      const int k = n * (n + 1) / 2 + m, ki = im_row_d(kt, n, m);
       for (int j = 0; j < dpc; ++j) {
         double *col = sU + cj[j];
         if (half <= 0) {
           atomicAdd(col + k, wj[j] * Gr);
-          atomicAdd(col + kt + k, wj[j] * Gi);
+          if (m > 0) atomicAdd(col + ki, wj[j] * Gi);
         }
         if (half < 0) {
           atomicAdd(col + kp + k, wj[j] * Rr);
-          atomicAdd(col + kp + kt + k, wj[j] * Ri);
+          if (m > 0) atomicAdd(col + kp + ki, wj[j] * Ri);
         } else if (half == 1) {
           atomicAdd(col + k, wj[j] * Rr);
-          atomicAdd(col + kt + k, wj[j] * Ri);
+          if (m > 0) atomicAdd(col + ki, wj[j] * Ri);
         }
       }
     };
     double Rcr = Rmr, Rci = Rmi, Gcr = Gmr, Gci = Gmi, Rpr = 0, Rpi = 0, Gpr = 0, Gpi = 0;
-    emit(m * (m + 1) / 2 + m, sc, Rcr, Rci, Gcr, Gci);
+    emit(m, sc, Rcr, Rci, Gcr, Gci);
     for (int n = m + 1; n <= p; ++n) {
       const double a = RA<double>(n, m), bb = RB<double>(n, m);
       const double Rnr = a * z * Rcr - bb * r2 * Rpr, Rni = a * z * Rci - bb * r2 * Rpi;
       const double Gnr = a * (nz * Rcr + z * Gcr) - bb * (dn2 * Rpr + r2 * Gpr);
       const double Gni = a * (nz * Rci + z * Gci) - bb * (dn2 * Rpi + r2 * Gpi);
       sc *= inv_delta;
-      emit(n * (n + 1) / 2 + m, sc, Rnr, Rni, Gnr, Gni);
+      emit(n, sc, Rnr, Rni, Gnr, Gni);
       Rpr = Rcr; Rpi = Rci; Gpr = Gcr; Gpi = Gci;
       Rcr = Rnr; Rci = Rni; Gcr = Gnr; Gci = Gni;
     }
@@ -1214,15 +1221,12 @@ struct P2mClear {
   double *acc = nullptr;
   int64_t ne = 0, na = 0;  // expansion values (blocks x kp), accumulator length
 };
-// NK = 1 reads the compact unit multipoles: kpc values per column, compact
-// row c holding full row cmap[c] (-1: padding), without the imaginary parts
-// of the m = 0 coefficients (zero for real sources) and without the
-// expansion's padding; the leaf's ME is expanded to kp rows in LDS.
-constexpr int kMaxKp = 144;  // kp at order 10
+// NK = 1 reads kpc values per column, without most of the expansion's padding
+// to kp rows, and stores zeros there.
 template <typename T, int NK>
 __global__ void __launch_bounds__(256) k_p2m(int nleaf, const int *__restrict__ leaves,
                                              const int *__restrict__ col_beg, const int *__restrict__ col_dof,
-                                             const T *__restrict__ U, int kp, int kpc, const int *__restrict__ cmap,
+                                             const T *__restrict__ U, int kp, int kpc,
                                              const double *__restrict__ phi, const double *__restrict__ dphi,
                                              T *__restrict__ ME, int64_t vs, int64_t es,
                                              P2mClear<T> cl = P2mClear<T>()) {
@@ -1276,31 +1280,14 @@ __global__ void __launch_bounds__(256) k_p2m(int nleaf, const int *__restrict__ 
   }
   part[t] = acc;
   __syncthreads();
-  if constexpr (NK == 2) {
+  const int K = NK * kp / VW;  // vectors of the leaf's expansion, zeros from NOV on
+  if (t < K) {
+    TV a{};
     if (t < NOV) {
-      TV a = part[t];
+      a = part[t];
       for (int q = 1; q < nph; ++q) add16(a, part[q * NOV + t]);
-      reinterpret_cast<TV *>(ME + (int64_t)leaves[li] * NO)[t] = a;
     }
-  } else {
-    // the compact sums into their rows of the leaf's kp-row ME (zeros
-    // elsewhere), then stored whole
-    __shared__ T sme[kMaxKp];
-    for (int i = t; i < kp; i += 256) sme[i] = T(0);
-    __syncthreads();
-    if (t < NOV) {
-      TV a = part[t];
-      for (int q = 1; q < nph; ++q) add16(a, part[q * NOV + t]);
-      const T *av = reinterpret_cast<const T *>(&a);
-#pragma unroll
-      for (int k = 0; k < VW; ++k) {
-        const int r = cmap[t * VW + k];
-        if (r >= 0) sme[r] = av[k];
-      }
-    }
-    __syncthreads();
-    T *me = ME + (int64_t)leaves[li] * kp;
-    for (int i = t; i < kp; i += 256) me[i] = sme[i];
+    reinterpret_cast<TV *>(ME + (int64_t)leaves[li] * NK * kp)[t] = a;
   }
 }
 
@@ -1321,23 +1308,23 @@ __global__ void k_op_near(int nleaf, const int *__restrict__ row_beg, const int 
     op[vb + i] = d ? -vals[2 * (vb + i) + 1] : vals[2 * (vb + i)];
   }
 }
-// (compact: kpc values per column, value o of row cmap[o], zero for padding)
-__global__ void k_op_unit(int64_t ncol, int kp, int kpc, const int *__restrict__ cmap,
-                          const int *__restrict__ col_dof, const uint8_t *__restrict__ dir,
+// (the first kpc of the kp values per column)
+__global__ void k_op_unit(int64_t ncol, int kp, int kpc, const int *__restrict__ col_dof, const uint8_t *__restrict__ dir,
                           const double *__restrict__ U, double *__restrict__ op) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < ncol * kpc;
        i += (int64_t)gridDim.x * blockDim.x) {
     const int64_t c = i / kpc;
-    const int r = cmap[(int)(i - c * kpc)];
-    op[i] = r < 0 ? 0.0 : (dir[col_dof[c]] ? -U[c * 2 * kp + kp + r] : U[c * 2 * kp + r]);
+    const int r = (int)(i - c * kpc);
+    op[i] = dir[col_dof[c]] ? -U[c * 2 * kp + kp + r] : U[c * 2 * kp + r];
   }
 }
 
 // Padded length of one real expansion vector at order P.
 template <int P>
 struct Kp {
-  static constexpr int kt = (P + 1) * (P + 2) / 2;
-  static constexpr int value = ((2 * kt + 15) / 16) * 16;
+  static constexpr int rows = (P + 1) * (P + 1);     // of one expansion
+  static constexpr int cols = (rows + 3) / 4 * 4;    // summed over by the translations: 4 per MFMA
+  static constexpr int value = (rows + 15) / 16 * 16;
 };
 
 // ---------------------------------------------------------------------------
@@ -1349,10 +1336,10 @@ struct Kp {
 // bem_fma.cc:2600-2602) are all OUT[tgt] += T_class . IN[src] with one R-linear
 // KP x KP operator per class (M2M / L2L: level and child octant; M2L:
 // integer offset, all levels).  Pairs are grouped by class into chunks of 32; a block
-// computes C (KP x 64) = A (KP x KP) . B (KP x 64 source columns, both
-// kernels) with 16x16x4 MFMA tiles (KP/16 wavefronts, wave w: row tile w,
-// all 64 columns), stages C through LDS and adds it to the targets with
-// coalesced atomics (targets are distinct within a chunk, not across chunks).
+// computes C (KP x 64) = A (KP x KC) . B (KC x 64 source columns, both
+// kernels; KC the expansion's rows padded to 4) with 16x16x4 MFMA tiles,
+// stages C through LDS and adds it to the targets with coalesced atomics
+// (targets are distinct within a chunk, not across chunks).
 //   f32 (v_mfma_f32_16x16x4f32): lane l holds A[l%16][l/16], B[l/16][l%16],
 //       D[4(l/16)+j][l%16], j < 4
 //   f64 (v_mfma_f64_16x16x4f64): same inputs, D[l/16+4j][l%16]
@@ -1380,29 +1367,38 @@ static_assert(kM2LChunk == 32 && kChunk1 == 64, "k_translate maps 2 x 32 or 1 x 
 
 // LDS tile (elements of T).  B is [64 columns][BS] (one source vector per
 // column), C is [64 columns][CS], both column-major, sharing one buffer.
-//   FP32: BS = KP + 2, so that the MFMA reads (16 columns x 2 k-rows per half
+//   FP32: BS = KC + 2, so that the MFMA reads (16 columns x 2 k-rows per half
 //   wavefront) hit 32 distinct banks; filled with 8-byte stores.  CS = KP + 4:
 //   an FP32 MFMA lane holds 4 consecutive rows of one column, stored as one
 //   16-byte write, and 8 such writes cover the 32 banks once.
-//   FP64: BS = KP + 2 (16-byte fill stores), CS = KP + 1.
-template <int P, typename T>
+//   FP64: BS = KC + 2 (16-byte fill stores), CS = KP + 1.
+// A workgroup's KP/16 row tiles x 4 groups of 16 columns are dealt to NR x CW
+// wavefronts: wave w takes row tile w % NR and 4 / CW column groups, so that
+// a lane's operator value feeds 4 / CW MFMAs.  A workgroup whose wavefronts
+// are no multiple of the 4 SIMDs leaves the matrix cores of some of them
+// idle (the first waves of every workgroup go to the same SIMDs).  M2L of
+// 579,952 pairs at order 8, FP64 / FP32: 6 wavefronts, K = 96 372 / 233 us
+// (without gather and output 259, matrix cores 57% busy), 12 wavefronts,
+// K = 84 307 / 190, near what its atomic adds take alone (305 / 177);
+// 211,368 pairs at order 7: 5 wavefronts of 80 rows 122 / 75, 8 of 64 rows
+// 92 / 54, into slots 109 / 45 and 56 / 31.
+template <int P, typename T, int KIND>
 struct TrLayout {
-  static constexpr int KP = Kp<P>::value;
-  static constexpr int BS = KP + 2;
+  static constexpr int KP = Kp<P>::value, KC = Kp<P>::cols;
+  static constexpr int BS = KC + 2;
   static constexpr int CS = sizeof(T) == 4 ? KP + 4 : KP + 1;
-  static constexpr int NR = KP / 16;        // 16-row tiles = wavefronts per block
-  static constexpr int NT = 64 * NR;        // threads per block
+  static constexpr int NR = KP / 16;        // 16-row tiles
+  static constexpr int CW = NR % 2 == 0 || NR > 4 ? 2 : 4;
+  static constexpr int NT = 64 * NR * CW;   // threads per block
   static constexpr int elems = 64 * (BS > CS ? BS : CS);
   static constexpr size_t bytes = (size_t)elems * sizeof(T);
 };
 
-// Wavefront w owns output rows 16w..16w+15 for all 64 columns (4 column
-// groups), so each operator fragment it loads from L2 feeds 4 MFMAs.  The
-// source vectors of the chunk (NK kp contiguous values per pair) are gathered
+// The source vectors of the chunk (NK expansions per pair) are gathered
 // with 16-byte loads, all issued before the LDS stores.  NK = 2: both
 // kernels' expansions, 32 pairs x 2 columns; NK = 1: one combined expansion,
 // 64 pairs.
-// KIND (0 M2M, 1 M2L, 2 L2L) only names the instantiation, so that traces and
+// KIND (0 M2M, 1 M2L, 2 L2L) names the instantiation, so that traces and
 // profiles tell the three passes apart; KIND 3 is M2L that stores each pair's
 // result into its own slot instead of adding it to the target (summed per
 // target by k_m2l_reduce).
@@ -1424,19 +1420,19 @@ __device__ __forceinline__ void translate_chunk(int c, T *__restrict__ sB, int *
   const T *__restrict__ ops = args.ops;
   const T *__restrict__ IN = args.IN;
   T *__restrict__ OUT = args.OUT;
-  using Lay = TrLayout<P, T>;
-  constexpr int KP = Lay::KP, K2 = NK * KP, BS = Lay::BS, CS = Lay::CS, NT = Lay::NT;
+  using Lay = TrLayout<P, T, KIND>;
+  constexpr int KP = Lay::KP, KC = Lay::KC, K2 = NK * KP, BS = Lay::BS, CS = Lay::CS, NT = Lay::NT;
   constexpr int PC = 64 / NK;                // pairs per chunk
-  static_assert(NT == 4 * KP, "launch bound");
+  constexpr int G = 4 / Lay::CW;             // column groups of a wavefront
+  static_assert(NT <= 1024 && PC <= NT, "threads per block");
   static_assert(sizeof(T) == 8 || (BS % 2 == 0 && CS % 4 == 0), "LDS vector alignment");
   using M = Mfma<T>;
   using TV = typename Vec16<T>::type;
   constexpr int V = 16 / sizeof(T);          // elements per 16-byte vector
-  constexpr int NVP = K2 / V;                // vectors per pair (both kernels)
-  constexpr int NV = PC * NVP;               // vectors per chunk
+  constexpr int NVC = KC / V;                // vectors per column (KC is a multiple of 4)
+  constexpr int NV = 64 * NVC;               // vectors per chunk
   constexpr int PER = (NV + NT - 1) / NT;    // vectors per thread
-  constexpr int KT2 = 2 * Kp<P>::kt;
-  const int t = threadIdx.x, w = t >> 6, l = t & 63;
+  const int t = threadIdx.x, w = (t >> 6) % Lay::NR, g0 = (t >> 6) / Lay::NR * G, l = t & 63;
   const T *A = ops + (int64_t)chunk_op[c] * KP * KP;  // column-major, read from L2
   const int beg = chunk_beg[c], cnt = chunk_cnt[c];
   if (t < PC) {
@@ -1448,10 +1444,10 @@ __device__ __forceinline__ void translate_chunk(int c, T *__restrict__ sB, int *
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     const int i = t + j * NT;
-    const int pr = i / NVP;
+    const int col = i / NVC, pr = col / NK;
     buf[j] = TV{};
     if (i < NV && pr < cnt)
-      buf[j] = *reinterpret_cast<const TV *>(IN + (int64_t)sS[pr] * K2 + (i - pr * NVP) * V);
+      buf[j] = *reinterpret_cast<const TV *>(IN + (int64_t)sS[pr] * K2 + (col % NK) * KP + (i - col * NVC) * V);
   }
   // M2M and L2L launches hold few chunks per level and wait on latency: each
   // lane loads its operator values for the whole K loop at once after the
@@ -1459,7 +1455,7 @@ __device__ __forceinline__ void translate_chunk(int c, T *__restrict__ sB, int *
   // M2L has tens of thousands of chunks in flight and keeps its registers
   // for occupancy, loading operator values inside the K loop.
   constexpr bool PRE = KIND != 1;
-  constexpr int NA = PRE ? KP / 4 : 1;
+  constexpr int NA = PRE ? KC / 4 : 1;
   T areg[NA];
   const T *ak = A + (l >> 4) * KP + 16 * w + (l & 15);
   if constexpr (PRE) {
@@ -1470,9 +1466,8 @@ __device__ __forceinline__ void translate_chunk(int c, T *__restrict__ sB, int *
   for (int j = 0; j < PER; ++j) {
     const int i = t + j * NT;
     if (i < NV) {
-      const int pr = i / NVP, off = (i - pr * NVP) * V;
-      const int col = NK * pr + (off >= KP), k = off >= KP ? off - KP : off;
-      T *d = sB + col * BS + k;
+      const int col = i / NVC;
+      T *d = sB + col * BS + (i - col * NVC) * V;
       if constexpr (sizeof(T) == 4) {  // 8-byte aligned: two 8-byte stores
         reinterpret_cast<float2 *>(d)[0] = float2{buf[j].x, buf[j].y};
         reinterpret_cast<float2 *>(d)[1] = float2{buf[j].z, buf[j].w};
@@ -1482,35 +1477,35 @@ __device__ __forceinline__ void translate_chunk(int c, T *__restrict__ sB, int *
     }
   }
   __syncthreads();
-  typename M::acc acc[4];
+  typename M::acc acc[G];
 #pragma unroll
-  for (int g = 0; g < 4; ++g) acc[g] = typename M::acc{0, 0, 0, 0};
-  const T *bk = sB + (l & 15) * BS + (l >> 4);
+  for (int g = 0; g < G; ++g) acc[g] = typename M::acc{0, 0, 0, 0};
+  const T *bk = sB + (g0 * 16 + (l & 15)) * BS + (l >> 4);
   if constexpr (PRE) {
 #pragma unroll
-    for (int k0 = 0; k0 < KP; k0 += 4) {
+    for (int k0 = 0; k0 < KC; k0 += 4) {
       const T a = areg[k0 / 4];
 #pragma unroll
-      for (int g = 0; g < 4; ++g) acc[g] = M::mac(a, bk[g * 16 * BS + k0], acc[g]);
+      for (int g = 0; g < G; ++g) acc[g] = M::mac(a, bk[g * 16 * BS + k0], acc[g]);
     }
   } else {
 #pragma unroll 4
-    for (int k0 = 0; k0 < KP; k0 += 4) {
+    for (int k0 = 0; k0 < KC; k0 += 4) {
       const T a = ak[k0 * KP];
 #pragma unroll
-      for (int g = 0; g < 4; ++g) acc[g] = M::mac(a, bk[g * 16 * BS + k0], acc[g]);
+      for (int g = 0; g < G; ++g) acc[g] = M::mac(a, bk[g * 16 * BS + k0], acc[g]);
     }
   }
   __syncthreads();  // B tile no longer needed: reuse the buffer for C
-  T *sC = sB;
+  T *sC = sB + g0 * 16 * CS;
   if constexpr (sizeof(T) == 4) {
 #pragma unroll
-    for (int g = 0; g < 4; ++g)
+    for (int g = 0; g < G; ++g)
       *reinterpret_cast<float4 *>(sC + (16 * g + (l & 15)) * CS + 16 * w + 4 * (l >> 4)) =
           float4{acc[g][0], acc[g][1], acc[g][2], acc[g][3]};
   } else {
 #pragma unroll
-    for (int g = 0; g < 4; ++g)
+    for (int g = 0; g < G; ++g)
 #pragma unroll
       for (int j = 0; j < 4; ++j) sC[(16 * g + (l & 15)) * CS + 16 * w + M::row(l, j)] = acc[g][j];
   }
@@ -1523,15 +1518,17 @@ __device__ __forceinline__ void translate_chunk(int c, T *__restrict__ sB, int *
     static_assert(NK == 1, "slot M2L is the single-expansion operator's");
     for (int i = t; i < cnt * KP; i += NT) {
       const int cc = i / KP, row = i - cc * KP;
-      OUT[(int64_t)sT[cc] * KP + row] = sC[cc * CS + row];
+      OUT[(int64_t)sT[cc] * KP + row] = sB[cc * CS + row];
     }
   } else {
     // coalesced accumulation: consecutive lanes add consecutive rows of one
-    // target (the Im rows of m = 0, zero for real densities, included:
-    // skipping them scatters the lanes and measured slower)
-    for (int i = t; i < NK * cnt * KT2; i += NT) {
-      const int cc = i / KT2, row = i - cc * KT2;
-      atomicAdd(OUT + (int64_t)sT[cc / NK] * K2 + (cc % NK) * KP + row, sC[cc * CS + row]);
+    // target; the lanes of the padding rows stay idle, so that a wavefront's
+    // rows start on a cache line (in-bounds probe, 580,000 targets of 96 rows:
+    // FP64 90 rows added by 64 consecutive lanes 332 us, 96 by aligned lanes
+    // 305 us, FP32 210 and 177 us: the adds are bound by the lines they touch)
+    for (int i = t; i < NK * cnt * KP; i += NT) {
+      const int cc = i / KP, row = i - cc * KP;
+      if (row < Kp<P>::rows) atomicAdd(OUT + (int64_t)sT[cc / NK] * K2 + (cc % NK) * KP + row, sB[cc * CS + row]);
     }
   }
 }
@@ -1584,15 +1581,31 @@ __device__ __forceinline__ int xcd_chunk(int w, int nch) {
   const int per = (nch + kXcd - 1) / kXcd;
   return (w % kXcd) * per + w / kXcd;
 }
-static inline int xcd_blocks(int nch) { return kXcdChunks ? (nch + kXcd - 1) / kXcd * kXcd : nch; }
+__host__ __device__ __forceinline__ int xcd_blocks(int nch) { return kXcdChunks ? (nch + kXcd - 1) / kXcd * kXcd : nch; }
 
 template <typename T, int P, int KIND, int NK>
-__global__ void __launch_bounds__(4 * Kp<P>::value) k_translate(TrArgs<T> a, int nch) {
-  __shared__ __align__(16) T sB[TrLayout<P, T>::elems];
+__global__ void __launch_bounds__((TrLayout<P, T, KIND>::NT)) k_translate(TrArgs<T> a, int nch) {
+  __shared__ __align__(16) T sB[TrLayout<P, T, KIND>::elems];
   __shared__ int sT[64 / NK], sS[64 / NK];
   const int c = xcd_chunk(blockIdx.x, nch);
   if (c >= nch) return;
   translate_chunk<T, P, KIND, NK>(c, sB, sT, sS, a);
+}
+
+// M2L of one combined expansion by fewer workgroups than chunks (a multiple
+// of 8, see kM2LBeside): each takes every (gridDim.x / 8)th chunk of its XCD's
+// run.  A kernel of its own, since the loop's registers cost the others
+// occupancy (order 8 FP64 M2L into slots 272 -> 358 us).
+template <typename T, int P>
+__global__ void __launch_bounds__((TrLayout<P, T, 1>::NT)) k_translate_few(TrArgs<T> a, int nch) {
+  __shared__ __align__(16) T sB[TrLayout<P, T, 1>::elems];
+  __shared__ int sT[64], sS[64];
+  for (int w = blockIdx.x; w < xcd_blocks(nch); w += gridDim.x) {
+    const int c = xcd_chunk(w, nch);
+    if (c >= nch) return;
+    if (w != (int)blockIdx.x) __syncthreads();  // the tile of the chunk before is read
+    translate_chunk<T, P, 1, 1>(c, sB, sT, sS, a);
+  }
 }
 
 // Evaluation of both kernels' expansions at a point: M2P
@@ -1643,8 +1656,9 @@ __device__ __forceinline__ void eval2(const T *__restrict__ E, int p_rt, int kt_
       }
       const int idx = n * (n + 1) / 2 + m;
       const T f = pc * r * f2;
-      v1 += (E[idx] * cm - E[kt + idx] * sm) * f;
-      if constexpr (NK == 2) v2 += (E[kp + idx] * cm - E[kp + kt + idx] * sm) * f;
+      const int im = kt + idx - n - 1;  // im_row: m = 0 has none
+      v1 += (m ? E[idx] * cm - E[im] * sm : E[idx]) * f;
+      if constexpr (NK == 2) v2 += (m ? E[kp + idx] * cm - E[kp + im] * sm : E[kp + idx]) * f;
     }
   }
 }
@@ -1784,10 +1798,10 @@ struct SideArgs {
 // launches would pay that latency once per launch.  One LDS buffer serves
 // every role.
 template <typename T, int P, int KIND, int SPMV, bool M2P>
-__global__ void __launch_bounds__(4 * Kp<P>::value) k_translate_side(int nch, TrArgs<T> tr, SideArgs<T> sd) {
-  constexpr int NT = 4 * Kp<P>::value;
+__global__ void __launch_bounds__((TrLayout<P, T, KIND>::NT)) k_translate_side(int nch, TrArgs<T> tr, SideArgs<T> sd) {
+  constexpr int NT = TrLayout<P, T, KIND>::NT;
   using E = typename NearEntry<T, 1>::type;
-  constexpr size_t TB = TrLayout<P, T>::bytes;
+  constexpr size_t TB = TrLayout<P, T, KIND>::bytes;
   constexpr size_t SB = SPMV == 0 ? kSpmvTile * sizeof(E) : 0;
   __shared__ __align__(16) unsigned char smem[TB > SB ? TB : SB];
   __shared__ int sT[64], sS[64];
@@ -2788,23 +2802,13 @@ void Engine::build_unit_multipoles(bool want_f32) {
     }
     sync();  // qpt, qleaf, qcol, dqbeg, dfit, dfit_half are freed on return
   }
-  // the operator's unit multipoles (U1 on Neumann, -U2 on Dirichlet DoFs),
-  // compact: the real parts, then the imaginary parts of m >= 1 (those of
-  // m = 0 vanish for real sources), padded to a multiple of 4
-  {
-    std::vector<int32_t> cmap;
-    for (int i = 0; i < kt; ++i) cmap.push_back(i);
-    for (int nn = 0; nn <= p; ++nn)
-      for (int m = 1; m <= nn; ++m) cmap.push_back(kt + nn * (nn + 1) / 2 + m);
-    while (cmap.size() % 4) cmap.push_back(-1);
-    kpc = (int)cmap.size();
-    up(d_cmap, cmap);
-  }
+  // the operator's unit multipoles (U1 on Neumann, -U2 on Dirichlet DoFs)
+  kpc = ((p + 1) * (p + 1) + 3) / 4 * 4;
   const int64_t nou = std::max<int64_t>(ncol, 1) * kpc;
   alloc(f64.opunit, (size_t)nou * sizeof(double));
   if (ncol > 0) {
     hipLaunchKernelGGL(k_op_unit, dim3((unsigned)std::min<int64_t>(nblk(ncol * kpc, 256), 8192)), dim3(256), 0,
-                       stream, ncol, kp, kpc, d_cmap.as<int>(), d_p2m_col_dof.as<int>(), d_dir.as<uint8_t>(),
+                       stream, ncol, kp, kpc, d_p2m_col_dof.as<int>(), d_dir.as<uint8_t>(),
                        f64.unit.as<double>(), f64.opunit.as<double>());
     HIPCHK(hipGetLastError());
   }
@@ -2983,12 +2987,14 @@ FarDev<float> &far_of<float>(Engine &e) { return e.f32; }
   }
 
 // OUT[tgt] += ops[class] . IN[src] for the chunks [c0, c1) of a chunk list
-// (chunks of 32 pairs for NK = 2, of 64 pairs for NK = 1).
+// (chunks of 32 pairs for NK = 2, of 64 pairs for NK = 1); M2L of one
+// expansion by at most max_wg workgroups (0: one per chunk).
 template <typename T, int KIND, int NK>
 static void launch_translate(Engine &e, hipStream_t st, const ChunkDev &cl, int c0, int c1, const T *ops,
-                             const T *IN, T *OUT, const int *slot_pos = nullptr) {
+                             const T *IN, T *OUT, const int *slot_pos = nullptr, int max_wg = 0) {
   const int n = c1 - c0;
   if (n <= 0) return;
+  const bool few = KIND == 1 && NK == 1 && max_wg > 0 && max_wg < xcd_blocks(n);
   const DevBuf &op = NK == 2 ? cl.op : cl.op1, &beg = NK == 2 ? cl.beg : cl.beg1, &cnt = NK == 2 ? cl.cnt : cl.cnt1;
   // the slot M2L (KIND 3) reads each pair's slot where the others read its target
   const int *tgt = KIND == 3 ? slot_pos : cl.tgt.as<int>();
@@ -2997,8 +3003,13 @@ static void launch_translate(Engine &e, hipStream_t st, const ChunkDev &cl, int 
                      ops, IN, OUT};
 #define PBFMM_TR(PP)                                                                                         \
   case PP:                                                                                                   \
-    hipLaunchKernelGGL((k_translate<T, PP, KIND, NK>), dim3(xcd_blocks(n)), dim3(TrLayout<PP, T>::NT), 0, st, tr, \
-                       n);                                                                                   \
+    if constexpr (KIND == 1 && NK == 1)                                                                      \
+      if (few) {                                                                                             \
+        hipLaunchKernelGGL((k_translate_few<T, PP>), dim3(max_wg), dim3(TrLayout<PP, T, KIND>::NT), 0, st, tr, n); \
+        break;                                                                                               \
+      }                                                                                                      \
+    hipLaunchKernelGGL((k_translate<T, PP, KIND, NK>), dim3(xcd_blocks(n)), dim3(TrLayout<PP, T, KIND>::NT), 0, st, \
+                       tr, n);                                                                               \
     break;
   switch (e.p) {
     PBFMM_TR(1) PBFMM_TR(2) PBFMM_TR(3) PBFMM_TR(4) PBFMM_TR(5)
@@ -3029,7 +3040,7 @@ static void launch_translate_side(Engine &e, const ChunkDev &cl, int c0, int c1,
                    cl.src.as<int>(), ops, IN, OUT};
 #define PBFMM_TRS(PP)                                                                                         \
   case PP: {                                                                                                  \
-    constexpr int NT = TrLayout<PP, T>::NT;                                                                   \
+    constexpr int NT = TrLayout<PP, T, KIND>::NT;                                                             \
     sd.spmv_blocks = spmv_side_blocks<SPMV>(sd, NT);                                                          \
     const int64_t mb = M2P ? (sd.m2p_hi - sd.m2p_lo + NT - 1) / NT : 0;                                      \
     const int64_t nb = xcd_blocks(nch) + sd.spmv_blocks + mb;                                                 \
@@ -3214,7 +3225,7 @@ void Engine::generate(const double *phi, const double *dphi) {
   if (nleaf > 0)
     hipLaunchKernelGGL((k_p2m<T, NK>), dim3(nleaf), dim3(256), 0, stream, nleaf, d_p2m_leaf.as<int>(),
                        d_p2m_col_beg.as<int>(), d_p2m_col_dof.as<int>(),
-                       (NK == 2 ? F.unit : F.opunit).template as<T>(), kp, kpc, d_cmap.as<int>(), phi, dphi,
+                       (NK == 2 ? F.unit : F.opunit).template as<T>(), kp, kpc, phi, dphi,
                        F.me.template as<T>(), (int64_t)0, (int64_t)0);
   mark(1);
   for (int l = L; l >= 1; --l)
@@ -3285,8 +3296,8 @@ void Engine::matvec(const double *phi, const double *dphi, double *outN, double 
     cl.ne = ne;
     const unsigned nclear = (unsigned)std::min<int64_t>(nblk(2 * ne, 256), 1024);
     hipLaunchKernelGGL((k_p2m<T, 2>), dim3(nleaf + nclear), dim3(256), 0, stream, nleaf, d_p2m_leaf.as<int>(),
-                       d_p2m_col_beg.as<int>(), d_p2m_col_dof.as<int>(), F.unit.template as<T>(), kp, kpc,
-                       nullptr, phi, dphi, me, (int64_t)0, (int64_t)0, cl);
+                       d_p2m_col_beg.as<int>(), d_p2m_col_dof.as<int>(), F.unit.template as<T>(), kp, kpc, phi, dphi,
+                       me, (int64_t)0, (int64_t)0, cl);
   } else {
     hipLaunchKernelGGL(k_clear_operator<T>, dim3((unsigned)std::min<int64_t>(nblk(2 * ne, 256), 4096)), dim3(256),
                        0, stream, me, le, ne, nullptr, (int64_t)0);
@@ -3383,6 +3394,18 @@ void Engine::launch_m2l_slots(const T *ops, const T *IN, T *LE) {
   HIPCHK(hipGetLastError());
 }
 
+// Workgroups of an M2L launch beside the SpMV on the second stream: one per
+// CU.  A workgroup per chunk takes every wavefront slot it can (12 wavefronts
+// each) and holds the memory-bound SpMV back until it drains; one per CU
+// leaves the SpMV the room to stream.  Plan 24, us per application, a
+// workgroup per chunk / one per CU: 393,218 DoFs FP64 1,266 / 1,142, FP32
+// 716 / 627; 98,306 390 / 343, 239 / 208; 24,578 at leaf 96 (452 values per
+// M2L pair) 83.5 / 80.1, 64 / 59.  Where M2L is the longer of the two it wants
+// all of the chip: 40,346 DoFs, order 7, leaf 20 (62 values per pair) 190 / 201.
+// Streaming 256 FP64 values takes about what a pair of order 6 to 8 does.
+constexpr int kM2LBeside = 256;
+constexpr int64_t kBesideValues = 256;
+
 // The single-value pipeline in fewer launches, for vmult: P2M, whose extra
 // workgroups clear the other MEs, LE and the M2P accumulator; M2M levels
 // L..me_lo + 1; M2L; L2L
@@ -3422,7 +3445,7 @@ void Engine::matvec_fused(const double *x, double *out, double *dst, int side) {
     const unsigned nclear = (unsigned)std::min<int64_t>(nblk(2 * ne + n, 256), 1024);
     hipLaunchKernelGGL((k_p2m<T, 1>), dim3(nleaf + nclear), dim3(256), 0, stream, nleaf, d_p2m_leaf.as<int>(),
                        d_p2m_col_beg.as<int>(), d_p2m_col_dof.as<int>(), F.opunit.template as<T>(), kp, kpc,
-                       d_cmap.as<int>(), x, nullptr, me, (int64_t)0, (int64_t)0, cl);
+                       x, nullptr, me, (int64_t)0, (int64_t)0, cl);
   } else {
     hipLaunchKernelGGL(k_clear_operator<T>, dim3((unsigned)std::min<int64_t>(nblk(2 * ne + n, 256), 4096)),
                        dim3(256), 0, stream, me, le, ne, acc, n);
@@ -3509,6 +3532,7 @@ void Engine::matvec_fused(const double *x, double *out, double *dst, int side) {
     near_done = true;
   }
   if (fork_later) fork_spmv();
+  const int m2l_wg = fork_later && near.nnz > kBesideValues * (int64_t)far.m2l.tgt.size() ? kM2LBeside : 0;
   // M2L, carrying M2P (sides 2, 3) and the SpMV (side 3, or whatever no M2M
   // launch took)
   const int c1 = nchunks<1>(far.m2l);
@@ -3530,7 +3554,7 @@ void Engine::matvec_fused(const double *x, double *out, double *dst, int side) {
   else if (m2p_here)
     launch_translate_side<T, 1, -1, true>(*this, m2l_cl, 0, c1, mops, me, le, sd);
   else
-    launch_translate<T, 1, 1>(*this, stream, m2l_cl, 0, c1, mops, me, le);
+    launch_translate<T, 1, 1>(*this, stream, m2l_cl, 0, c1, mops, me, le, nullptr, m2l_wg);
   m2p_done = m2p_done || m2p_here;
   // L2L, the deepest launched level (or group of two levels) carrying M2P
   // (side 1)
@@ -4912,8 +4936,7 @@ void Engine::matvec_combined_multi(const double *x, double *out, int R) {
                      ne, T(0));
   if (nleaf > 0)  // every right-hand side in one launch (blockIdx.y)
     hipLaunchKernelGGL((k_p2m<T, 1>), dim3(nleaf, R), dim3(256), 0, stream, nleaf, d_p2m_leaf.as<int>(),
-                       d_p2m_col_beg.as<int>(), d_p2m_col_dof.as<int>(), F.opunit.template as<T>(), kp, kpc,
-                       d_cmap.as<int>(), x, nullptr, ME, (int64_t)n, sb);
+                       d_p2m_col_beg.as<int>(), d_p2m_col_dof.as<int>(), F.opunit.template as<T>(), kp, kpc, x, nullptr, ME, (int64_t)n, sb);
   if (me_lo < 0) consumer_levels();
   for (int l = L; l > me_lo; --l)
     launch_translate<T, 0, 1>(*this, stream, mr_m2m, lvl<1>(mr_m2m_h, l), lvl<1>(mr_m2m_h, l + 1),

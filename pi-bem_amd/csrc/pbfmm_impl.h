@@ -40,8 +40,14 @@ template <typename T> using RawVec = std::vector<T, NoInit<T>>;
 // one combined expansion does.
 constexpr int kM2LChunk = 32;
 constexpr int kChunk1 = 64;
-// padded length of one real expansion vector [Re(0..Kt-1), Im(0..Kt-1)]
-inline int kp_of(int p) { return ((2 * kt_of(p) + 15) / 16) * 16; }
+// One real expansion vector: the real parts of the kt coefficients (n, m) at
+// n(n+1)/2 + m, then the imaginary parts of those with m >= 1 in the same
+// order (at m = 0 they vanish for real sources and have no row): (p+1)^2
+// rows, padded with zeros to kp, a multiple of the matrix cores' 16 rows.
+// Before, with all 2 kt = (p+1)(p+2) rows, order 7 took 80 rows instead of 64
+// and the others as many as now, but every product ran over kp columns.
+inline int im_row(int kt, int n, int m) { return kt + n * (n - 1) / 2 + m - 1; }  // m >= 1
+inline int kp_of(int p) { return ((p + 1) * (p + 1) + 15) / 16 * 16; }
 
 // ---------------------------------------------------------------------------
 // Mesh and regular quadrature data (host, FP64)
@@ -185,7 +191,7 @@ void build_far_plan(const Tree &t, int p, FarPlan &fp);
 void build_m2m_groups(const Tree &t, FarPlan &fp);
 void build_l2l_groups(const Tree &t, FarPlan &fp);
 void build_p2m_plan(const HostMesh &m, const QuadData &qd, const Tree &t, FarPlan &fp);
-// R-linear translation operators on [Re, Im] vectors (padded to kp).
+// R-linear translation operators on real expansion vectors (padded to kp).
 void op_m2m(int p, const double d[3], double *opT);  // d = child - parent
 void op_l2l(int p, const double d[3], double *opT);  // d = parent - child
 void op_m2l(int p, const double d[3], double *opT);  // d = source - target

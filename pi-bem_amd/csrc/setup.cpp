@@ -673,12 +673,14 @@ double ire(int k) {  // Re(i^k), k even
 inline int tri(int n, int m) { return n * (n + 1) / 2 + m; }
 inline int sgn(int x) { return (x > 0) - (x < 0); }
 // out(n,m) += w * a~ where a~ = (x, sig*y) of input (nn, mi): adds the four real
-// entries of the R-linear map into the transposed operator opT[col*kp + row].
-inline void put(double *opT, int kt, int kp, int out, int in, double wr, double wi, int sig) {
+// entries of the R-linear map into the transposed operator opT[col*kp + row];
+// those of imaginary parts at m = 0 or mi = 0, zero for real sources, have no row.
+inline void put(double *opT, int kt, int kp, int n, int m, int nn, int mi, double wr, double wi, int sig) {
+  const int out = tri(n, m), in = tri(nn, mi);
   opT[(size_t)in * kp + out] += wr;
-  opT[(size_t)(kt + in) * kp + out] += -sig * wi;
-  opT[(size_t)in * kp + kt + out] += wi;
-  opT[(size_t)(kt + in) * kp + kt + out] += sig * wr;
+  if (mi > 0) opT[(size_t)im_row(kt, nn, mi) * kp + out] += -sig * wi;
+  if (m > 0) opT[(size_t)in * kp + im_row(kt, n, m)] += wi;
+  if (m > 0 && mi > 0) opT[(size_t)im_row(kt, nn, mi) * kp + im_row(kt, n, m)] += sig * wr;
 }
 void sph(const double d[3], double &rho, double &ca, double &beta) {
   rho = std::sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
@@ -702,7 +704,7 @@ void op_m2m(int p, const double d[3], double *opT) {
           if (std::abs(m - mm) > n - nn) continue;
           double rf = P(nn, std::abs(mm)) * an.pw[nn] * kA(nn, mm) * kA(n - nn, m - mm) / kA(n, m);
           rf *= ire(std::abs(m) - std::abs(mm) - std::abs(m - mm));
-          put(opT, kt, kp, tri(n, m), tri(n - nn, std::abs(m - mm)), rf * an.cos(mm), -rf * an.sin(mm), sgn(m - mm));
+          put(opT, kt, kp, n, m, n - nn, std::abs(m - mm), rf * an.cos(mm), -rf * an.sin(mm), sgn(m - mm));
         }
 }
 
@@ -723,7 +725,7 @@ void op_l2l(int p, const double d[3], double *opT) {
           double c = kA(nn - n, mm - m) / kA(nn, mm) * kA(n, m) * ire(std::abs(mm) - std::abs(mm - m) - std::abs(m)) *
                      (((nn + n) & 1) ? -1.0 : 1.0);
           const double rf = P(nn - n, std::abs(mm - m)) * rf0 * c;
-          put(opT, kt, kp, tri(n, m), tri(nn, std::abs(mm)), rf * an.cos(mm - m), rf * an.sin(mm - m), sgn(mm));
+          put(opT, kt, kp, n, m, nn, std::abs(mm), rf * an.cos(mm - m), rf * an.sin(mm - m), sgn(mm));
         }
       }
 }
@@ -744,7 +746,7 @@ void op_m2l(int p, const double d[3], double *opT) {
           double c = kA(nn, mm) / kA(n + nn, m - mm) * kA(n, m) * ire(std::abs(m - mm) - std::abs(m) - std::abs(mm)) /
                      ((nn & 1) ? -1.0 : 1.0);
           const double rf = P(n + nn, std::abs(mm - m)) * rf0 * c;
-          put(opT, kt, kp, tri(n, m), tri(nn, std::abs(mm)), rf * an.cos(mm - m), rf * an.sin(mm - m), mm < 0 ? -1 : 1);
+          put(opT, kt, kp, n, m, nn, std::abs(mm), rf * an.cos(mm - m), rf * an.sin(mm - m), mm < 0 ? -1 : 1);
         }
       }
 }
@@ -770,15 +772,14 @@ static void add_class(ChunkList &cl, int op, const std::vector<std::pair<int, in
   }
 }
 
-// Degree n of each row of a real expansion vector [Re(0..Kt-1), Im(0..Kt-1),
-// padding] (index n(n+1)/2 + m); padding rows get degree 0.
+// Degree n of each row of a real expansion vector; padding rows get degree 0.
 static std::vector<int> row_degrees(int p, int kp) {
   const int kt = kt_of(p);
   std::vector<int> deg(kp, 0);
   for (int n = 0; n <= p; ++n)
     for (int m = 0; m <= n; ++m) {
       deg[n * (n + 1) / 2 + m] = n;
-      deg[kt + n * (n + 1) / 2 + m] = n;
+      if (m > 0) deg[im_row(kt, n, m)] = n;
     }
   return deg;
 }
