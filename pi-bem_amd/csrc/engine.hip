@@ -3126,9 +3126,13 @@ void Engine::launch_spmv(int variant, const double *phi, const double *dphi, dou
 // together 83 / 92 / 112 / 166 us; 290 MB (38,402 DoFs, Q2, leaf 80) apart
 // 357 / 558 / 963 / 1762 us, together 347 / 459 / 700 / 1173 us.  2 MB (1,538
 // DoFs, leaf 20), 8 / 16 / 32: apart 62 / 90 / 144 us, together 64 / 92 / 143.
+// Two of them up to 1 GB stay apart: 310 MB in narrow leaves (a hull of 8,100
+// DoFs, leaf 20), the near field alone, FP32 124 us apart, 155 together, FP64
+// 236 and 272; 1.8 GB FP32 780 apart, 545 together.
 static bool use_spmm(const Engine &e, int R, size_t value_bytes) {
   const int64_t bytes = e.near.nnz * (int64_t)value_bytes;
-  return bytes >= ((int64_t)256 << 20) ? R >= 2 : R >= (bytes >= ((int64_t)8 << 20) ? 8 : 16);
+  if (bytes >= ((int64_t)256 << 20)) return R >= (bytes >= ((int64_t)1 << 30) ? 2 : 3);
+  return R >= (bytes >= ((int64_t)8 << 20) ? 8 : 16);
 }
 
 // The near field of R right-hand sides, n apart.  One (a single column of
