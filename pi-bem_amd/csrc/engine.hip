@@ -2474,7 +2474,10 @@ __global__ void k_seg_scale(int64_t n, const int *__restrict__ seg, const double
 
 // Segmented GMRES building blocks: every part of a forest runs its own
 // Arnoldi process inside shared basis vectors.  Dots over part-aligned chunks
-// (part[j * nch + c]) finished per (part, vector): out[s * ldo + j].
+// (part[j * nch + c]), which the kernels that use the sums finish themselves:
+// a launch of this size takes 3 to 4 us whatever it does, and with launches
+// for the sums and the norm a step took nine of them instead of five (twelve
+// spheroids of 1.5k to 5.4k DoFs, mixed solve 5.31 -> 4.77 ms).
 __global__ void __launch_bounds__(kRedThreads) k_mdot_seg(const int64_t *__restrict__ cbeg, int64_t ldv,
                                                           const double *__restrict__ V, const double *__restrict__ w,
                                                           double *__restrict__ part) {
@@ -2486,25 +2489,44 @@ __global__ void __launch_bounds__(kRedThreads) k_mdot_seg(const int64_t *__restr
   const double r = block_sum(acc, sh);
   if (threadIdx.x == 0) part[(int64_t)j * gridDim.x + blockIdx.x] = r;
 }
-__global__ void __launch_bounds__(kRedThreads) k_finish_seg(int nch, const int *__restrict__ sch_off, int ldo,
-                                                            const double *__restrict__ part, double *__restrict__ out) {
-  __shared__ double sh[kRedThreads / 64];
-  const int s = blockIdx.x, j = blockIdx.y;
-  double acc = 0;
-  for (int c = sch_off[s] + threadIdx.x; c < sch_off[s + 1]; c += kRedThreads) acc += part[(int64_t)j * nch + c];
-  const double r = block_sum(acc, sh);
-  if (threadIdx.x == 0) out[(int64_t)s * ldo + j] = r;
-}
-// w -= sum_j V_j h[part][j]
-__global__ void k_gemv_sub_seg(int64_t n, int64_t ldv, int nv, const double *__restrict__ V,
-                               const double *__restrict__ h, int ldh, const int *__restrict__ seg,
-                               double *__restrict__ w) {
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double *hs = h + (int64_t)seg[i] * ldh;
-  double acc = w[i];
-  for (int j = 0; j < nv; ++j) acc -= V[(int64_t)j * ldv + i] * hs[j];
-  w[i] = acc;
+// w -= sum_j V_j h[part][j], h[part][j] the sum of the part's chunks in
+// part[j * nch + c], by every workgroup of the part in the same order; the
+// first stores it in h_out[part * ldh + j].  Workgroup (c, y) takes rows
+// 256 y .. of chunk c, so that it has one part, and stores the sum of squares
+// of its new w in npart[c * gridDim.y + y] when npart is given.  nv <= 128.
+__global__ void __launch_bounds__(kRedThreads) k_gemv_sub_seg(const int64_t *__restrict__ cbeg,
+                                                              const int *__restrict__ seg,
+                                                              const int *__restrict__ sch_off, int64_t ldv, int nv,
+                                                              const double *__restrict__ V,
+                                                              const double *__restrict__ part, int ldh,
+                                                              double *__restrict__ h_out, double *__restrict__ w,
+                                                              double *__restrict__ npart) {
+  __shared__ double hs[kRedThreads], sh[kRedThreads / 64];
+  const int c = blockIdx.x, nch = gridDim.x, t = (int)threadIdx.x;
+  const int s = seg[cbeg[c]];
+  const int c0 = sch_off[s], c1 = sch_off[s + 1];
+  const int64_t i = cbeg[c] + (int64_t)blockIdx.y * kRedThreads + t;
+  const bool row = i < cbeg[c + 1];
+  double acc = row ? w[i] : 0.0;
+  for (int j0 = 0; j0 < nv; j0 += kRedThreads) {  // a batch's restart has no upper limit
+    const int nj = min(kRedThreads, nv - j0);
+    if (j0 > 0) __syncthreads();
+    if (t < nj) {
+      double h = 0;
+#pragma unroll 4
+      for (int q = c0; q < c1; ++q) h += part[(int64_t)(j0 + t) * nch + q];
+      hs[t] = h;
+      if (c == c0 && blockIdx.y == 0) h_out[(int64_t)s * ldh + j0 + t] = h;
+    }
+    __syncthreads();
+    if (row)
+      for (int j = 0; j < nj; ++j) acc -= V[(int64_t)(j0 + j) * ldv + i] * hs[j];
+  }
+  if (row) w[i] = acc;
+  if (npart) {  // the same for every workgroup
+    const double r = block_sum(acc * acc, sh);
+    if (t == 0) npart[c * gridDim.y + blockIdx.y] = r;
+  }
 }
 // x += sum_j V_j y[part][j]
 __global__ void k_gemv_add_seg(int64_t n, int64_t ldv, int nv, const double *__restrict__ V,
@@ -2517,15 +2539,30 @@ __global__ void k_gemv_add_seg(int64_t n, int64_t ldv, int nv, const double *__r
   for (int j = 0; j < nv; ++j) acc += V[(int64_t)j * ldv + i] * ys[j];
   x[i] = acc;
 }
-// Arnoldi normalisation per part (nrm2 holds squared norms); parts that are
-// no longer active get zero vectors, so they stay inert
-__global__ void k_scale_inv_seg(int64_t n, const int *__restrict__ seg, const double *__restrict__ nrm2,
-                                const uint8_t *__restrict__ active, double *__restrict__ v) {
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int s = seg[i];
-  const double q = nrm2[s];
-  v[i] = (active[s] && q > 0) ? v[i] / sqrt(q) : 0.0;
+// Arnoldi normalisation per part, its squared norm summed from npart by every
+// workgroup in the same order (the part's first stores it in nrm2); parts
+// that are no longer active get zero vectors, so they stay inert.  The
+// workgroups are k_gemv_sub_seg's.
+__global__ void __launch_bounds__(kRedThreads) k_scale_seg(const int64_t *__restrict__ cbeg,
+                                                           const int *__restrict__ seg,
+                                                           const int *__restrict__ sch_off,
+                                                           const double *__restrict__ npart,
+                                                           const uint8_t *__restrict__ active,
+                                                           double *__restrict__ nrm2, double *__restrict__ v) {
+  __shared__ double sh[kRedThreads / 64], qs;
+  const int c = blockIdx.x, t = (int)threadIdx.x, ny = gridDim.y;
+  const int s = seg[cbeg[c]];
+  double a = 0;
+  for (int q = sch_off[s] * ny + t; q < sch_off[s + 1] * ny; q += kRedThreads) a += npart[q];
+  const double r = block_sum(a, sh);
+  if (t == 0) {
+    qs = r;
+    if (c == sch_off[s] && blockIdx.y == 0) nrm2[s] = r;
+  }
+  __syncthreads();
+  const double q = qs;
+  const int64_t i = cbeg[c] + (int64_t)blockIdx.y * kRedThreads + t;
+  if (i < cbeg[c + 1]) v[i] = (active[s] && q > 0) ? v[i] / sqrt(q) : 0.0;
 }
 
 // ===========================================================================
@@ -4595,9 +4632,13 @@ static int gmres_core_seg(Engine &e, const SegCtx &c, const double *b, double *x
   std::vector<double> est(S), beta, y((size_t)S * m), hcol(m + 2), fsc(S);
   std::vector<int> ks(S);
   std::vector<uint8_t> active(S), done(S);
-  auto dots = [&](int nv, const double *Vs, const double *vec, double *out, int ldo) {
-    hipLaunchKernelGGL(k_mdot_seg, dim3(nch, nv), dim3(kRedThreads), 0, e.stream, rch, n, Vs, vec, part);
-    hipLaunchKernelGGL(k_finish_seg, dim3(S, nv), dim3(kRedThreads), 0, e.stream, nch, sch, ldo, part, out);
+  // the norm's partial sums follow the dots' in part
+  constexpr int kSubs = kRedChunk / kRedThreads;
+  double *npart = part + (size_t)nch * (m + 2);
+  auto project = [&](int nv, double *vec, double *h, double *np) {  // vec -= V h, h = V . vec
+    hipLaunchKernelGGL(k_mdot_seg, dim3(nch, nv), dim3(kRedThreads), 0, e.stream, rch, n, V, vec, part);
+    hipLaunchKernelGGL(k_gemv_sub_seg, dim3(nch, kSubs), dim3(kRedThreads), 0, e.stream, rch, seg, sch, n, nv, V,
+                       part, ldh, h, vec, np);
   };
   // relaxed mixed precision (sw given): the FP64 operator until every
   // active part's estimate is below its switch level sw[s], then the inner
@@ -4648,12 +4689,10 @@ static int gmres_core_seg(Engine &e, const SegCtx &c, const double *b, double *x
       ++it;
       double *slot = hd + (size_t)k * SL;
       double *h1 = slot, *h2 = slot + (size_t)S * ldh, *hn = slot + (size_t)2 * S * ldh;
-      dots(k + 1, V, vk1, h1, ldh);
-      hipLaunchKernelGGL(k_gemv_sub_seg, dim3(g), dim3(256), 0, e.stream, n, n, k + 1, V, h1, ldh, seg, vk1);
-      dots(k + 1, V, vk1, h2, ldh);
-      hipLaunchKernelGGL(k_gemv_sub_seg, dim3(g), dim3(256), 0, e.stream, n, n, k + 1, V, h2, ldh, seg, vk1);
-      dots(1, vk1, vk1, hn, 1);
-      hipLaunchKernelGGL(k_scale_inv_seg, dim3(g), dim3(256), 0, e.stream, n, seg, hn, act_d, vk1);
+      project(k + 1, vk1, h1, nullptr);
+      project(k + 1, vk1, h2, npart);
+      hipLaunchKernelGGL(k_scale_seg, dim3(nch, kSubs), dim3(kRedThreads), 0, e.stream, rch, seg, sch, npart, act_d,
+                         hn, vk1);
       if (k < k_sync && k + 1 < m && it < maxit) continue;
       HIPCHK(hipMemcpyAsync(hbuf.data() + (size_t)k_done * SL, hd + (size_t)k_done * SL,
                             (size_t)(k + 1 - k_done) * SL * 8, hipMemcpyDeviceToHost, e.stream));
@@ -4820,7 +4859,7 @@ int Engine::gmres_forest(const double *b, double *x, double tol, int restart, in
   const size_t SL = (size_t)2 * S * (restart + 2) + S;
   if (d_hs.bytes < SL * restart * 8) alloc(d_hs, SL * restart * 8);
   if (d_ys.bytes < (size_t)S * restart * 8) alloc(d_ys, (size_t)S * restart * 8);
-  const size_t red = (size_t)n_rch * (restart + 2) * 8;
+  const size_t red = (size_t)n_rch * (restart + 2 + kRedChunk / kRedThreads) * 8;
   if (d_red.bytes < red) alloc(d_red, red);
   if (!d_ptmp.p) alloc(d_ptmp, n * 8);
   if (!d_ptmp2.p) alloc(d_ptmp2, n * 8);
@@ -5008,7 +5047,7 @@ int Engine::gmres_multi(const double *b, double *x, int R, double tol, int resta
     const size_t SL = (size_t)2 * R * (restart + 2) + R;
     alloc(mr_hs, SL * restart * 8);
     alloc(mr_ys, (size_t)R * restart * 8);
-    alloc(mr_red, (size_t)mr_nch * (restart + 2) * 8);
+    alloc(mr_red, (size_t)mr_nch * (restart + 2 + kRedChunk / kRedThreads) * 8);
     mr_restart = restart;
   }
   struct MeanMode {  // linear pure-Neumann operator for the duration of the solve
