@@ -202,6 +202,9 @@ struct Engine {
   int plan_apps[2] = {0, 0}, graph_steps[2] = {0, 0};
   hipStream_t side_stream = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+  void make_side_stream();
+  void fork_side();
+  int m2l_beside() const;  // workgroups of an M2L launch beside the SpMV, 0: one per chunk
   // slot M2L: targets, their slot ranges (CSR) and each pair's slot, the
   // slots of one target consecutive (its pairs in ascending order)
   DevBuf d_red_tgt, d_red_beg, d_slot_pos;

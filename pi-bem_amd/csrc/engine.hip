@@ -1592,19 +1592,19 @@ __global__ void __launch_bounds__((TrLayout<P, T, KIND>::NT)) k_translate(TrArgs
   translate_chunk<T, P, KIND, NK>(c, sB, sT, sS, a);
 }
 
-// M2L of one combined expansion by fewer workgroups than chunks (a multiple
+// M2L by fewer workgroups than chunks (a multiple
 // of 8, see kM2LBeside): each takes every (gridDim.x / 8)th chunk of its XCD's
 // run.  A kernel of its own, since the loop's registers cost the others
 // occupancy (order 8 FP64 M2L into slots 272 -> 358 us).
-template <typename T, int P>
+template <typename T, int P, int NK>
 __global__ void __launch_bounds__((TrLayout<P, T, 1>::NT)) k_translate_few(TrArgs<T> a, int nch) {
   __shared__ __align__(16) T sB[TrLayout<P, T, 1>::elems];
-  __shared__ int sT[64], sS[64];
+  __shared__ int sT[64 / NK], sS[64 / NK];
   for (int w = blockIdx.x; w < xcd_blocks(nch); w += gridDim.x) {
     const int c = xcd_chunk(w, nch);
     if (c >= nch) return;
     if (w != (int)blockIdx.x) __syncthreads();  // the tile of the chunk before is read
-    translate_chunk<T, P, 1, 1>(c, sB, sT, sS, a);
+    translate_chunk<T, P, 1, NK>(c, sB, sT, sS, a);
   }
 }
 
@@ -2759,6 +2759,12 @@ void Engine::upload_far(bool want_f32) {
   if (want_f32) upload_far_t<float>(*this, f32);
 }
 
+// Both kernels' SpMV beside M2L and L2L on the second stream, from this many
+// values on; fork and join cost more than few values gain.  generate + products on host vectors, us, apart / beside: 1,538
+// DoFs (0.3 M values) 148 / 188, 6,146 (1.4 M) 235 / 213, 24,578 at leaf 20
+// (7 M) 380 / 345, 38,402 Q2 at leaf 20 (15 M) 533 / 473, 98,306 1,027 / 887.
+constexpr int64_t kPairsBeside = 1000000;
+
 // Unit multipoles of every leaf (FP64, rounded once for the FP32 operator).
 void Engine::build_unit_multipoles(bool want_f32) {
   const int64_t ncol = (int64_t)far.p2m_col_dof.size();
@@ -2837,6 +2843,8 @@ void Engine::build_unit_multipoles(bool want_f32) {
       HIPCHK(hipGetLastError());
       sync();  // the index copies are freed on return
     }
+    // the products' second stream is made (0.2 ms) while the GPU is busy here
+    if (near.nnz >= kPairsBeside) make_side_stream();
     sync();  // qpt, qleaf, qcol, dqbeg, dfit, dfit_half are freed on return
   }
   // the operator's unit multipoles (U1 on Neumann, -U2 on Dirichlet DoFs)
@@ -3024,14 +3032,14 @@ FarDev<float> &far_of<float>(Engine &e) { return e.f32; }
   }
 
 // OUT[tgt] += ops[class] . IN[src] for the chunks [c0, c1) of a chunk list
-// (chunks of 32 pairs for NK = 2, of 64 pairs for NK = 1); M2L of one
-// expansion by at most max_wg workgroups (0: one per chunk).
+// (chunks of 32 pairs for NK = 2, of 64 pairs for NK = 1); M2L by at most
+// max_wg workgroups (0: one per chunk).
 template <typename T, int KIND, int NK>
 static void launch_translate(Engine &e, hipStream_t st, const ChunkDev &cl, int c0, int c1, const T *ops,
                              const T *IN, T *OUT, const int *slot_pos = nullptr, int max_wg = 0) {
   const int n = c1 - c0;
   if (n <= 0) return;
-  const bool few = KIND == 1 && NK == 1 && max_wg > 0 && max_wg < xcd_blocks(n);
+  const bool few = KIND == 1 && max_wg > 0 && max_wg < xcd_blocks(n);
   const DevBuf &op = NK == 2 ? cl.op : cl.op1, &beg = NK == 2 ? cl.beg : cl.beg1, &cnt = NK == 2 ? cl.cnt : cl.cnt1;
   // the slot M2L (KIND 3) reads each pair's slot where the others read its target
   const int *tgt = KIND == 3 ? slot_pos : cl.tgt.as<int>();
@@ -3040,9 +3048,9 @@ static void launch_translate(Engine &e, hipStream_t st, const ChunkDev &cl, int 
                      ops, IN, OUT};
 #define PBFMM_TR(PP)                                                                                         \
   case PP:                                                                                                   \
-    if constexpr (KIND == 1 && NK == 1)                                                                      \
+    if constexpr (KIND == 1)                                                                                 \
       if (few) {                                                                                             \
-        hipLaunchKernelGGL((k_translate_few<T, PP>), dim3(max_wg), dim3(TrLayout<PP, T, KIND>::NT), 0, st, tr, n); \
+        hipLaunchKernelGGL((k_translate_few<T, PP, NK>), dim3(max_wg), dim3(TrLayout<PP, T, KIND>::NT), 0, st, tr, n); \
         break;                                                                                               \
       }                                                                                                      \
     hipLaunchKernelGGL((k_translate<T, PP, KIND, NK>), dim3(xcd_blocks(n)), dim3(TrLayout<PP, T, KIND>::NT), 0, st, \
@@ -3276,6 +3284,36 @@ void Engine::generate(const double *phi, const double *dphi) {
   HIPCHK(hipGetLastError());
 }
 
+void Engine::make_side_stream() {
+  if (side_stream) return;
+  HIPCHK(hipEventCreateWithFlags(&ev_fork, hipEventDisableTiming));
+  HIPCHK(hipEventCreateWithFlags(&ev_join, hipEventDisableTiming));
+  HIPCHK(hipStreamCreateWithFlags(&side_stream, hipStreamNonBlocking));
+}
+
+// The second stream, ordered after what the handle's stream holds.
+void Engine::fork_side() {
+  make_side_stream();
+  HIPCHK(hipEventRecord(ev_fork, stream));
+  HIPCHK(hipStreamWaitEvent(side_stream, ev_fork, 0));
+}
+
+// Workgroups of an M2L launch beside the SpMV on the second stream: one per
+// CU.  A workgroup per chunk takes every wavefront slot it can (12 wavefronts
+// each) and holds the memory-bound SpMV back until it drains; one per CU
+// leaves the SpMV the room to stream.  Plan 24, us per application, a
+// workgroup per chunk / one per CU: 393,218 DoFs FP64 1,266 / 1,142, FP32
+// 716 / 627; 98,306 390 / 343, 239 / 208.  Both kernels' products of 98,306
+// DoFs (host vectors) 1,026 / 887.  Where M2L is the longer of the two it
+// wants all of the chip: 40,346 DoFs, order 7, leaf 20 (62 values per pair)
+// 190 / 201; both kernels' products of 38,402 DoFs, leaf 80 (481 per pair)
+// 439 / 493.  The line lies between there and 98,306 DoFs at leaf 80 (643).
+constexpr int kM2LBeside = 256;
+constexpr int64_t kBesideValues = 512;
+int Engine::m2l_beside() const {
+  return near.nnz > kBesideValues * (int64_t)far.m2l.tgt.size() ? kM2LBeside : 0;
+}
+
 // Downward pass and near field.  NK = 2: outN = N.phi, outD = D.dphi;
 // NK = 1: outN = N.phi - D.dphi (outD unused).
 template <typename T, int NK>
@@ -3283,7 +3321,15 @@ void Engine::products(const double *phi, const double *dphi, double *outN, doubl
   FarDev<T> &F = far_of<T>(*this);
   const int nrows = (int)near.rows.size();
   mark(3);
-  if (near.nleaf > 0) launch_spmv<T, NK>(spmv_variant[sizeof(T) == 4 ? 1 : 0][NK - 1], phi, dphi, outN, outD);
+  const int var = spmv_variant[sizeof(T) == 4 ? 1 : 0][NK - 1];
+  const bool beside = NK == 2 && !time_phases && near.nnz >= kPairsBeside;
+  if (beside) {
+    fork_side();
+    launch_spmv<T, NK>(var, phi, dphi, outN, outD, 1, side_stream);
+    HIPCHK(hipEventRecord(ev_join, side_stream));
+  } else if (near.nleaf > 0) {
+    launch_spmv<T, NK>(var, phi, dphi, outN, outD);
+  }
   mark(4);
   const int64_t nle = (int64_t)tree.nb * NK * kp;
   hipLaunchKernelGGL(k_fill<T>, dim3((unsigned)std::min<int64_t>(nblk(nle, 256), 4096)), dim3(256), 0, stream,
@@ -3293,17 +3339,25 @@ void Engine::products(const double *phi, const double *dphi, double *outN, doubl
     launch_m2l_slots<T>(F.m2l.template as<T>(), F.me.template as<T>(), F.le.template as<T>());
   else
     launch_translate<T, 1, NK>(*this, stream, m2l_cl, 0, nchunks<NK>(far.m2l), F.m2l.template as<T>(),
-                               F.me.template as<T>(), F.le.template as<T>());
+                               F.me.template as<T>(), F.le.template as<T>(), nullptr, beside ? m2l_beside() : 0);
   mark(6);
   const int64_t nitems = (int64_t)far.m2p_item_node.size();
-  if (nitems > 0)
-    PBFMM_BY_ORDER(p, hipLaunchKernelGGL((k_m2p<T, NK, PP>), dim3((unsigned)nblk(nitems, 256)), dim3(256), 0, stream, nitems,
-                       d_m2p_node.as<int>(), d_m2p_isrc.as<int>(), d_xyz.as<double>(), d_pmin.as<double>(),
-                       d_delta.as<double>(), p, kt, kp, F.me.template as<T>(), outN, outD, (int64_t)0, (int64_t)0));
+  auto m2p = [&]() {  // adds to the SpMV's rows
+    if (nitems == 0) return;
+    PBFMM_BY_ORDER(p, hipLaunchKernelGGL((k_m2p<T, NK, PP>), dim3((unsigned)nblk(nitems, 256)), dim3(256), 0, stream,
+                                         nitems, d_m2p_node.as<int>(), d_m2p_isrc.as<int>(), d_xyz.as<double>(),
+                                         d_pmin.as<double>(), d_delta.as<double>(), p, kt, kp,
+                                         F.me.template as<T>(), outN, outD, (int64_t)0, (int64_t)0));
+  };
+  if (!beside) m2p();
   mark(7);
   for (int l = 2; l <= L; ++l)
     launch_translate<T, 2, NK>(*this, stream, l2l_cl, lvl<NK>(far.l2l, l), lvl<NK>(far.l2l, l + 1),
                                F.l2l.template as<T>(), F.le.template as<T>(), F.le.template as<T>());
+  if (beside) {
+    HIPCHK(hipStreamWaitEvent(stream, ev_join, 0));
+    m2p();
+  }
   mark(8);
   if (nrows > 0)
     PBFMM_BY_ORDER(p, hipLaunchKernelGGL((k_l2p<T, NK, PP>), dim3(nblk(nrows, 256)), dim3(256), 0, stream, nrows, d_rows.as<int>(),
@@ -3435,18 +3489,6 @@ void Engine::launch_m2l_slots(const T *ops, const T *IN, T *LE) {
   HIPCHK(hipGetLastError());
 }
 
-// Workgroups of an M2L launch beside the SpMV on the second stream: one per
-// CU.  A workgroup per chunk takes every wavefront slot it can (12 wavefronts
-// each) and holds the memory-bound SpMV back until it drains; one per CU
-// leaves the SpMV the room to stream.  Plan 24, us per application, a
-// workgroup per chunk / one per CU: 393,218 DoFs FP64 1,266 / 1,142, FP32
-// 716 / 627; 98,306 390 / 343, 239 / 208; 24,578 at leaf 96 (452 values per
-// M2L pair) 83.5 / 80.1, 64 / 59.  Where M2L is the longer of the two it wants
-// all of the chip: 40,346 DoFs, order 7, leaf 20 (62 values per pair) 190 / 201.
-// Streaming 256 FP64 values takes about what a pair of order 6 to 8 does.
-constexpr int kM2LBeside = 256;
-constexpr int64_t kBesideValues = 256;
-
 // The single-value pipeline in fewer launches, for vmult: P2M, whose extra
 // workgroups clear the other MEs, LE and the M2P accumulator; M2M levels
 // L..me_lo + 1; M2L; L2L
@@ -3528,13 +3570,7 @@ void Engine::matvec_fused(const double *x, double *out, double *dst, int side) {
   // the FMM, from the start or (late) from M2L on, leaving the M2M levels'
   // latency-bound launches the whole chip
   auto fork_spmv = [&]() {
-    if (!side_stream) {
-      HIPCHK(hipStreamCreateWithFlags(&side_stream, hipStreamNonBlocking));
-      HIPCHK(hipEventCreateWithFlags(&ev_fork, hipEventDisableTiming));
-      HIPCHK(hipEventCreateWithFlags(&ev_join, hipEventDisableTiming));
-    }
-    HIPCHK(hipEventRecord(ev_fork, stream));
-    HIPCHK(hipStreamWaitEvent(side_stream, ev_fork, 0));
+    fork_side();
     // M2P first (plans 88, 92): compute-bound, beside the M2L's atomics
     if (late && m2p_first && !m2p_done) launch_m2p(side_stream);
     launch_spmv<T, 1>(var_full, x, nullptr, out, nullptr, 1, side_stream);
@@ -3573,7 +3609,7 @@ void Engine::matvec_fused(const double *x, double *out, double *dst, int side) {
     near_done = true;
   }
   if (fork_later) fork_spmv();
-  const int m2l_wg = fork_later && near.nnz > kBesideValues * (int64_t)far.m2l.tgt.size() ? kM2LBeside : 0;
+  const int m2l_wg = fork_later ? m2l_beside() : 0;
   // M2L, carrying M2P (sides 2, 3) and the SpMV (side 3, or whatever no M2M
   // launch took)
   const int c1 = nchunks<1>(far.m2l);
