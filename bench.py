@@ -74,9 +74,9 @@ def kernel_name(phase, prec, p, nk, tuning):
     choices (SpMV variant, M2L plan: bit 4 = slots, bit 1 = M2P/L2P side
     fusion; the operator's L2P is fused with the post-processing)."""
     t = "float" if prec == "fp32" else "double"
-    plan = int(tuning.get(f"side_fusion_{prec}", 0)) if nk == 1 else 0
+    plan = max(0, int(tuning.get(f"side_fusion_{prec}", 0))) if nk == 1 else 0  # -1: not timed yet
     if phase == "spmv":
-        v = int(tuning.get(f"spmv_kernel_{prec}", 0))
+        v = max(0, int(tuning.get(f"spmv_kernel_{prec}", 0)))
         fmt = (((SPMV_KERNEL_FP64 if prec == "fp64" and v > 2 else SPMV_KERNEL)[v]) if nk == 1
                else "k_spmv_lds/k_spmv_wave<{t}, {k}> (variant timed for the matvec)")
     elif phase == "l2p":

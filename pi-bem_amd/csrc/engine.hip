@@ -3726,6 +3726,10 @@ int Engine::use_side_fusion(bool f32) {
   int &mode = side_fusion[f32 ? 1 : 0];
   if (mode >= 0) return mode;
   if (plan_apps[f32 ? 1 : 0]++ < kPlanAfter) return first_plan(f32);
+  // timing synchronises: not while the caller captures the stream
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  HIPCHK(hipStreamIsCapturing(stream, &capturing));
+  if (capturing != hipStreamCaptureStatusNone) return first_plan(f32);
   const unsigned g = nblk(n, 256);
   if (d_cost.bytes < (size_t)2 * n * 8) alloc(d_cost, (size_t)2 * n * 8);
   double *u = d_cost.as<double>(), *v = d_cost.as<double>() + n;

@@ -44,8 +44,8 @@ constexpr int kChunk1 = 64;
 // n(n+1)/2 + m, then the imaginary parts of those with m >= 1 in the same
 // order (at m = 0 they vanish for real sources and have no row): (p+1)^2
 // rows, padded with zeros to kp, a multiple of the matrix cores' 16 rows.
-// Before, with all 2 kt = (p+1)(p+2) rows, order 7 took 80 rows instead of 64
-// and the others as many as now, but every product ran over kp columns.
+// With all 2 kt = (p+1)(p+2) rows, orders 3, 7 and 10 took a tile of 16 rows
+// more, and every product ran over kp columns instead of (p+1)^2.
 inline int im_row(int kt, int n, int m) { return kt + n * (n - 1) / 2 + m - 1; }  // m >= 1
 inline int kp_of(int p) { return ((p + 1) * (p + 1) + 15) / 16 * 16; }
 

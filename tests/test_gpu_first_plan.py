@@ -43,3 +43,52 @@ def test_first_applications_equal_plan_0(n, order, leaf):
             print(f"  {name}: {e:.1e}", flush=True)
             assert e <= tol
     f.close()
+
+
+def test_capture_where_the_plan_would_be_timed():
+    """The 65th application, which times the plan, inside a caller's capture:
+    it runs first_plan instead and the capture replays; the next eager one
+    times the plan."""
+    import ctypes as C
+    from pibem_amd import hip
+    rt = hip.hip()
+
+    def ok(rc):
+        assert rc == 0, rc
+
+    pr = M.config_sphere(16, 4)
+    stream, graph, run = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    ok(rt.hipStreamCreate(C.byref(stream)))
+    f = P.BEMFMA(trunc_order=pr.p, num_octree_levels=pr.levels, max_nodes_per_leaf=pr.max_nodes_per_leaf,
+                 quad_order=pr.quad_order, sing_quad_order=pr.sing_quad_order, stream=stream.value)
+    f.init_fma(pr.mesh, pr.dirichlet)
+    f.generate_octree_blocking()
+    f.direct_integrals()
+    f.multipole_integrals()
+    bp = P.BEMProblem(f)
+    bp.compute_alpha()
+    src = np.linspace(-1, 1, f.n)
+    x, y = hip.DeviceArray.from_numpy(src), hip.DeviceArray(f.n)
+    for _ in range(64):
+        bp.vmult_dev(x.value, y.value, P.PBFMM_FP64)
+    hip.synchronize()
+    ok(rt.hipStreamBeginCapture(stream, C.c_int(1)))  # thread-local mode
+    bp.vmult_dev(x.value, y.value, P.PBFMM_FP64)
+    ok(rt.hipStreamEndCapture(stream, C.byref(graph)))
+    ok(rt.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)))
+    assert f.tuning_state()["side_fusion_fp64"] == -1
+    for k in range(3):
+        x.upload(src * 0.5 ** k)
+        y.upload(np.zeros(f.n))
+        hip.synchronize()
+        ok(rt.hipGraphLaunch(run, stream))
+        hip.synchronize()
+        got = y.numpy()
+        bp.vmult_dev(x.value, y.value, P.PBFMM_FP64)
+        hip.synchronize()
+        assert np.linalg.norm(got - y.numpy()) <= 1e-13 * np.linalg.norm(got), k
+    assert f.tuning_state()["side_fusion_fp64"] >= 0
+    ok(rt.hipGraphExecDestroy(run))
+    ok(rt.hipGraphDestroy(graph))
+    f.close()
+    ok(rt.hipStreamDestroy(stream))
