@@ -352,9 +352,10 @@ int pbfmm_set_spmv_kernel(pbfmm_handle *h, int32_t precision, int32_t kernel);
  * second stream forked after the M2M levels, beside M2L onwards; 56 and 60:
  * plans 24 and 28 with M2P following the SpMV on the second stream; 88 and
  * 92: with M2P before the SpMV there; -1 times plans 0, 3, 5, 8, 24, 56 and
- * 92 on the next application).  Without a call the first 64 applications run
- * a plan chosen by sizes, and the plan is timed after them.  For tests and
- * tuning.  No counterpart in the reference. */
+ * 92 on the next application).  Without a call the first 16 applications run
+ * a plan chosen by sizes, the next 21 each run one of those plans, timed, and
+ * the fastest is kept.  For tests and tuning.  No counterpart in the
+ * reference. */
 int pbfmm_set_side_fusion(pbfmm_handle *h, int32_t precision, int32_t mode);
 
 /* The choices this handle's timings made so far (-1 = not timed yet):
@@ -378,7 +379,7 @@ int pbfmm_tuning_state(pbfmm_handle *h, int32_t *state);
  * reference): the preconditioner and the operator application of one Arnoldi
  * step of pbfmm_gmres_dev / pbfmm_solve_system run from a fixed input into a
  * fixed output, so the launches can be captured once and replayed.  -1
- * (default): 16 steps after the launch plan is timed (in the next steps after
+ * (default): 512 steps after the launch plan is chosen (in the next steps after
  * a call with -1) the graph is captured and three replays are timed against
  * three direct runs, and the faster is kept; 0 direct launches only; 1 graph
  * replays.  A graph is captured again whenever a choice or buffer it holds

@@ -197,9 +197,14 @@ struct Engine {
     return false;
   }
   static constexpr int kTimedPlans[] = {3, 5, 8, 24, 56, 92};  // besides 0 (use_side_fusion)
-  // applications before the plan is timed, and steps after that before the graph is
-  static constexpr int kPlanAfter = 64, kGraphAfter = 16;
-  int plan_apps[2] = {0, 0}, graph_steps[2] = {0, 0};
+  // applications of a precision before its plans are timed, applications of
+  // each plan (one of them untimed), and GMRES steps on the chosen plan
+  // before the graph is timed: a capture and seven steps, paid back by
+  // hundreds of steps if at all
+  static constexpr int kPlanAfter = 16, kPlanSamples = 3, kGraphAfter = 512;
+  int plan_apps[2] = {0, 0}, graph_steps[2] = {0, 0};  // plan_apps -1: time on the next application
+  std::vector<hipEvent_t> plan_ev[2];
+  hipEvent_t plan_end = nullptr;  // recorded after the application under way
   hipStream_t side_stream = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   void make_side_stream();
@@ -232,6 +237,8 @@ struct Engine {
   void drop_graphs();
   int use_side_fusion(bool f32);
   int first_plan(bool f32) const;
+  int explore_plan(bool f32);
+  void drop_plan_events();
   // near-field SpMV kernel per precision ([0] FP64, [1] FP32) and storage
   // (pairs, single values): 0 workgroup per leaf with an LDS copy of the
   // columns, 1 wavefront per leaf with 2 rows in flight, 2 with 4 rows, 3 (6

@@ -2621,6 +2621,7 @@ Engine::~Engine() {
   if (ev_fork) (void)hipEventDestroy(ev_fork);
   if (ev_join) (void)hipEventDestroy(ev_join);
   if (side_stream) (void)hipStreamDestroy(side_stream);
+  drop_plan_events();
 }
 
 void Engine::drop_graphs() {
@@ -3693,14 +3694,14 @@ double Engine::norm2(const double *v) {
 // The launch plan of the operator (matvec_fused).  Which is the fastest
 // depends on the problem (level launches that wait on latency, SpMV and M2L
 // that share the chip or crowd each other), by up to 1.7x, so it is timed, per
-// precision, on scratch vectors: kTimedPlans, of which one was within 2% of
+// precision: kTimedPlans, of which one was within 2% of
 // the best of all fourteen at every one of twenty problems (602 to 393,218
 // DoFs, orders 4 to 8, leaf sizes 20 to 96, both precisions).  A plan other
-// than 0 is kept only if it beats plan 0 by 2%.  Timing costs two dozen
-// applications and a plan gains a tenth of one as a rule, so one solve does not
-// pay for it: the first kPlanAfter applications of a precision run first_plan
-// (98,306 DoFs, Q2, one mixed solve on a new handle: 75 ms of timing before a
-// solve of 16 ms).
+// than 0 is kept only if it beats plan 0 by 2%.  Timing on scratch vectors
+// costs two dozen applications (98,306 DoFs, Q2, one mixed solve on a new
+// handle: 75 ms of timing before a solve of 16 ms), so the solves' own
+// applications are timed (explore_plan), after the first kPlanAfter of a
+// precision, which run first_plan.
 //
 // first_plan: the plan that the sizes suggest.  Measured at those problems,
 // us per application of plan 0 against the plan chosen, FP32 unless stated:
@@ -3722,14 +3723,70 @@ int Engine::first_plan(bool f32) const {
   if (f32 && nnz >= 10000000 && m2l > nnz / 200) return 92;
   return nnz >= (f32 ? 25000000 : 8000000) ? 24 : 0;
 }
+// Applications kPlanAfter .. of a precision, kPlanSamples for each of plan 0
+// and kTimedPlans: the first one (which may allocate) is not timed.  Every
+// plan computes the operator, so they are the solve's own; the events are
+// read once the last of them has passed, and first_plan runs until then.
+int Engine::explore_plan(bool f32) {
+  constexpr int np = 1 + (int)(sizeof(kTimedPlans) / sizeof(*kTimedPlans)), ns = kPlanSamples;
+  const int f = f32 ? 1 : 0, k = plan_apps[f] - kPlanAfter;
+  std::vector<hipEvent_t> &ev = plan_ev[f];
+  if (k < 0) {
+    ++plan_apps[f];
+    return first_plan(f32);
+  }
+  if (k < np * ns) {
+    ++plan_apps[f];
+    const int q = k / ns, j = k % ns;
+    if (j > 0) {
+      for (int e = 0; e < 2; ++e) {
+        hipEvent_t one;
+        HIPCHK(hipEventCreate(&one));
+        ev.push_back(one);
+      }
+      HIPCHK(hipEventRecord(ev[ev.size() - 2], stream));
+      plan_end = ev.back();
+    }
+    return q == 0 ? 0 : kTimedPlans[q - 1];
+  }
+  const hipError_t ready = hipEventQuery(ev.back());
+  if (ready == hipErrorNotReady) return first_plan(f32);
+  HIPCHK(ready);
+  float best = 0;
+  int pick = 0;
+  for (int q = 0; q < np; ++q) {
+    float ms = 0;
+    for (int j = 0; j < ns - 1; ++j) {
+      float one = 0;
+      const size_t at = 2 * (size_t)(q * (ns - 1) + j);
+      HIPCHK(hipEventElapsedTime(&one, ev[at], ev[at + 1]));
+      ms = j == 0 ? one : std::min(ms, one);
+    }
+    if (q == 0) best = 0.98f * ms;
+    else if (ms < best) best = ms, pick = kTimedPlans[q - 1];
+  }
+  for (hipEvent_t e : ev) (void)hipEventDestroy(e);
+  ev.clear();
+  return side_fusion[f] = pick;
+}
+
+void Engine::drop_plan_events() {
+  for (auto &v : plan_ev) {
+    for (hipEvent_t e : v) (void)hipEventDestroy(e);
+    v.clear();
+  }
+}
+
 int Engine::use_side_fusion(bool f32) {
   int &mode = side_fusion[f32 ? 1 : 0];
   if (mode >= 0) return mode;
-  if (plan_apps[f32 ? 1 : 0]++ < kPlanAfter) return first_plan(f32);
-  // timing synchronises: not while the caller captures the stream
+  const int f = f32 ? 1 : 0;
+  // a caller's capture takes neither synchronisation nor timing
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
   HIPCHK(hipStreamIsCapturing(stream, &capturing));
   if (capturing != hipStreamCaptureStatusNone) return first_plan(f32);
+  if (plan_apps[f] >= 0) return explore_plan(f32);
+  // pbfmm_set_side_fusion -1: timed now
   const unsigned g = nblk(n, 256);
   if (d_cost.bytes < (size_t)2 * n * 8) alloc(d_cost, (size_t)2 * n * 8);
   double *u = d_cost.as<double>(), *v = d_cost.as<double>() + n;
@@ -3800,6 +3857,10 @@ void Engine::vmult(const double *src, double *dst, int precision) {
       matvec_fused<float>(xin, d_outN.as<double>(), dst, side);
     else
       matvec_fused<double>(xin, d_outN.as<double>(), dst, side);
+    if (plan_end) {
+      HIPCHK(hipEventRecord(plan_end, stream));
+      plan_end = nullptr;
+    }
   } else {
     if (f32)
       matvec_combined<float>(xin, d_outN.as<double>());
