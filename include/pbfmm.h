@@ -352,9 +352,9 @@ int pbfmm_set_spmv_kernel(pbfmm_handle *h, int32_t precision, int32_t kernel);
  * second stream forked after the M2M levels, beside M2L onwards; 56 and 60:
  * plans 24 and 28 with M2P following the SpMV on the second stream; 88 and
  * 92: with M2P before the SpMV there; -1 times plans 0, 3, 5, 8, 24, 56 and
- * 92 on the next application).  Without a call the first 16 applications run
- * a plan chosen by sizes, the next 21 each run one of those plans, timed, and
- * the fastest is kept.  For tests and tuning.  No counterpart in the
+ * 92 on the next application).  Without a call the first 8 applications run
+ * a plan chosen by sizes, the next 35 each run one of those plans, timed, and
+ * a faster one is kept.  For tests and tuning.  No counterpart in the
  * reference. */
 int pbfmm_set_side_fusion(pbfmm_handle *h, int32_t precision, int32_t mode);
 

@@ -201,7 +201,7 @@ struct Engine {
   // each plan (one of them untimed), and GMRES steps on the chosen plan
   // before the graph is timed: a capture and seven steps, paid back by
   // hundreds of steps if at all
-  static constexpr int kPlanAfter = 16, kPlanSamples = 3, kGraphAfter = 512;
+  static constexpr int kPlanAfter = 8, kPlanSamples = 5, kGraphAfter = 512;
   int plan_apps[2] = {0, 0}, graph_steps[2] = {0, 0};  // plan_apps -1: time on the next application
   std::vector<hipEvent_t> plan_ev[2];
   hipEvent_t plan_end = nullptr;  // recorded after the application under way
