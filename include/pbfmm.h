@@ -352,10 +352,11 @@ int pbfmm_set_spmv_kernel(pbfmm_handle *h, int32_t precision, int32_t kernel);
  * second stream forked after the M2M levels, beside M2L onwards; 56 and 60:
  * plans 24 and 28 with M2P following the SpMV on the second stream; 88 and
  * 92: with M2P before the SpMV there; -1 times plans 0, 3, 5, 8, 24, 56 and
- * 92 on the next application).  Without a call the first 8 applications run
- * a plan chosen by sizes, the next 35 each run one of those plans, timed, and
- * a faster one is kept.  For tests and tuning.  No counterpart in the
- * reference. */
+ * 92 before the next application or solve).  Without a call a plan chosen by
+ * sizes runs; the plans are timed, once, before the 49th single application
+ * of a precision or before a solve on a handle that has made 256 applications
+ * in it.  A solve keeps one plan from its start to its end.  For tests and
+ * tuning.  No counterpart in the reference. */
 int pbfmm_set_side_fusion(pbfmm_handle *h, int32_t precision, int32_t mode);
 
 /* The choices this handle's timings made so far (-1 = not timed yet):
@@ -379,12 +380,11 @@ int pbfmm_tuning_state(pbfmm_handle *h, int32_t *state);
  * reference): the preconditioner and the operator application of one Arnoldi
  * step of pbfmm_gmres_dev / pbfmm_solve_system run from a fixed input into a
  * fixed output, so the launches can be captured once and replayed.  -1
- * (default): 512 steps after the launch plan is chosen (in the next steps after
- * a call with -1) the graph is captured and three replays are timed against
- * three direct runs, and the faster is kept; 0 direct launches only; 1 graph
+ * (default): after 512 steps of a precision (in the next steps after a call
+ * with -1) the graph is captured and three replays are timed against three
+ * direct runs, and the faster is kept; 0 direct launches only; 1 graph
  * replays.  A graph is captured again whenever a choice or buffer it holds
- * changes.  Batch handles and many right-hand
- * sides launch directly. */
+ * changes.  Batch handles and many right-hand sides launch directly. */
 int pbfmm_set_graph_mode(pbfmm_handle *h, int32_t mode);
 /* The timing behind the graph choice, ms per step: [0] [1] FP64 direct /
  * graph, [2] [3] FP32 direct / graph (0 until timed). */

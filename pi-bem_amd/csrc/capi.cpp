@@ -1069,7 +1069,7 @@ int pbfmm_set_side_fusion(pbfmm_handle *h, int32_t precision, int32_t mode) {
     return fail(h, PBFMM_ERR_ARG, "set_side_fusion: unknown precision");
   const int pi = precision == PBFMM_MIXED ? 1 : 0;
   h->eng.side_fusion[pi] = mode;
-  if (mode == -1) h->eng.plan_apps[pi] = -1;  // timed on the next application
+  if (mode == -1) h->eng.plan_apps[pi] = -1;  // timed before the next application or solve
   return PBFMM_OK;
 }
 

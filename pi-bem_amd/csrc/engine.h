@@ -196,15 +196,25 @@ struct Engine {
       if (v == m) return true;
     return false;
   }
-  static constexpr int kTimedPlans[] = {3, 5, 8, 24, 56, 92};  // besides 0 (use_side_fusion)
-  // applications of a precision before its plans are timed, applications of
-  // each plan (one of them untimed), and GMRES steps on the chosen plan
-  // before the graph is timed: a capture and seven steps, paid back by
-  // hundreds of steps if at all
-  static constexpr int kPlanAfter = 8, kPlanSamples = 5, kGraphAfter = 512;
-  int plan_apps[2] = {0, 0}, graph_steps[2] = {0, 0};  // plan_apps -1: time on the next application
-  std::vector<hipEvent_t> plan_ev[2];
-  hipEvent_t plan_end = nullptr;  // recorded after the application under way
+  static constexpr int kTimedPlans[] = {3, 5, 8, 24, 56, 92};  // besides 0 (time_plans)
+  // Applications of a precision before its plans are timed: single ones
+  // (pbfmm_vmult), and those a handle has run when a solve starts.  Timing
+  // takes about 25 applications (time_plans), half of a solve, so a handle
+  // that solves a few times keeps first_plan; single applications are timed
+  // once a caller has made as many as a solve makes.  kGraphAfter: GMRES
+  // steps before the graph is timed (a capture and seven steps, paid back by
+  // hundreds of steps if at all).
+  static constexpr int kPlanAfter = 48, kSolvePlanAfter = 256, kGraphAfter = 512;
+  int plan_apps[2] = {0, 0}, graph_steps[2] = {0, 0};  // plan_apps -1: time before the next application or solve
+  // A solve keeps one launch plan from its first application to its last
+  // (plans differ in the order of FP32 sums), so nothing is timed inside one.
+  struct Solving {
+    int &depth;
+    explicit Solving(int &d) : depth(++d) {}
+    ~Solving() { --depth; }
+  };
+  int solving = 0;
+  void settle_plan(int precision);
   hipStream_t side_stream = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   void make_side_stream();
@@ -237,8 +247,7 @@ struct Engine {
   void drop_graphs();
   int use_side_fusion(bool f32);
   int first_plan(bool f32) const;
-  int explore_plan(bool f32);
-  void drop_plan_events();
+  int time_plans(bool f32);
   // near-field SpMV kernel per precision ([0] FP64, [1] FP32) and storage
   // (pairs, single values): 0 workgroup per leaf with an LDS copy of the
   // columns, 1 wavefront per leaf with 2 rows in flight, 2 with 4 rows, 3 (6

@@ -2621,7 +2621,6 @@ Engine::~Engine() {
   if (ev_fork) (void)hipEventDestroy(ev_fork);
   if (ev_join) (void)hipEventDestroy(ev_join);
   if (side_stream) (void)hipStreamDestroy(side_stream);
-  drop_plan_events();
 }
 
 void Engine::drop_graphs() {
@@ -3693,14 +3692,12 @@ double Engine::norm2(const double *v) {
 
 // The launch plan of the operator (matvec_fused).  Which is the fastest
 // depends on the problem (level launches that wait on latency, SpMV and M2L
-// that share the chip or crowd each other), by up to 1.7x, so it is timed, per
-// precision: kTimedPlans, of which one was within 2% of
-// the best of all fourteen at every one of twenty problems (602 to 393,218
-// DoFs, orders 4 to 8, leaf sizes 20 to 96, both precisions).  Timing on scratch vectors
-// costs two dozen applications (98,306 DoFs, Q2, one mixed solve on a new
-// handle: 75 ms of timing before a solve of 16 ms), so the solves' own
-// applications are timed (explore_plan), after the first kPlanAfter of a
-// precision, which run first_plan.
+// that share the chip or crowd each other), by up to 1.7x.  New handles run
+// first_plan; handles in longer use time plan 0 and kTimedPlans, per
+// precision, on scratch vectors (time_plans), between solves and never in
+// one.  One of the timed plans was within 2% of the best of all fourteen at
+// every one of twenty problems (602 to 393,218 DoFs, orders 4 to 8, leaf
+// sizes 20 to 96, both precisions).
 //
 // first_plan: the plan that the sizes suggest.  Measured at those problems,
 // us per application of plan 0 against the plan chosen, FP32 unless stated:
@@ -3722,110 +3719,83 @@ int Engine::first_plan(bool f32) const {
   if (f32 && nnz >= 10000000 && m2l > nnz / 200) return 92;
   return nnz >= (f32 ? 25000000 : 8000000) ? 24 : 0;
 }
-// Applications kPlanAfter .. of a precision, kPlanSamples for each of plan 0
-// and kTimedPlans: the first one (which may allocate) is not timed.  Every
-// plan computes the operator, so they are the solve's own; the events are
-// read once the last of them has passed, and first_plan runs until then.
-int Engine::explore_plan(bool f32) {
-  constexpr int np = 1 + (int)(sizeof(kTimedPlans) / sizeof(*kTimedPlans)), ns = kPlanSamples;
-  const int f = f32 ? 1 : 0, k = plan_apps[f] - kPlanAfter;
-  std::vector<hipEvent_t> &ev = plan_ev[f];
-  if (k < 0) {
-    ++plan_apps[f];
-    return first_plan(f32);
-  }
-  if (k < np * ns) {
-    ++plan_apps[f];
-    const int q = k / ns, j = k % ns;
-    if (j > 0) {
-      for (int e = 0; e < 2; ++e) {
-        hipEvent_t one;
-        HIPCHK(hipEventCreate(&one));
-        ev.push_back(one);
-      }
-      HIPCHK(hipEventRecord(ev[ev.size() - 2], stream));
-      plan_end = ev.back();
+// Times the plans on scratch vectors and keeps the fastest for the handle.
+// A plan's time is the best of three runs of a few applications (other
+// streams' work and host pauses only add), after one that may allocate.
+// first_plan stays unless another beats it by 1%, what repeated timings of
+// one plan differ by; a plan whose first run is 10% behind is not timed
+// further.
+int Engine::time_plans(bool f32) {
+  const unsigned g = nblk(n, 256);
+  alloc(d_cost, (size_t)2 * n * 8);
+  double *u = d_cost.as<double>(), *v = d_cost.as<double>() + n;
+  hipLaunchKernelGGL(k_fill<double>, dim3(g), dim3(256), 0, stream, u, n, 1.0);
+  hipEvent_t ev[4] = {};
+  for (hipEvent_t &e : ev) HIPCHK(hipEventCreate(&e));
+  auto apply = [&](int plan) {
+    if (f32)
+      matvec_fused<float>(u, d_outN.as<double>(), v, plan);
+    else
+      matvec_fused<double>(u, d_outN.as<double>(), v, plan);
+  };
+  int reps = 1;
+  auto timed = [&](int plan, int runs) {  // ms per application, the best of the runs
+    HIPCHK(hipEventRecord(ev[0], stream));
+    for (int r = 0; r < runs; ++r) {
+      for (int k = 0; k < reps; ++k) apply(plan);
+      HIPCHK(hipEventRecord(ev[r + 1], stream));
     }
-    return q == 0 ? 0 : kTimedPlans[q - 1];
-  }
-  const hipError_t ready = hipEventQuery(ev.back());
-  if (ready == hipErrorNotReady) return first_plan(f32);
-  HIPCHK(ready);
-  // first_plan (one of those timed) stays unless another beats it by 3%: what
-  // other streams ran meanwhile is in the times
+    HIPCHK(hipEventSynchronize(ev[runs]));
+    float best = 0;
+    for (int r = 0; r < runs; ++r) {
+      float ms = 0;
+      HIPCHK(hipEventElapsedTime(&ms, ev[r], ev[r + 1]));
+      best = r == 0 ? ms : std::min(best, ms);
+    }
+    return best / reps;
+  };
   const int usual = first_plan(f32);
-  float best = 0, stay = 0;
-  int pick = 0;
-  for (int q = 0; q < np; ++q) {
-    const int plan = q == 0 ? 0 : kTimedPlans[q - 1];
-    float ms = 0;
-    for (int j = 0; j < ns - 1; ++j) {
-      float one = 0;
-      const size_t at = 2 * (size_t)(q * (ns - 1) + j);
-      HIPCHK(hipEventElapsedTime(&one, ev[at], ev[at + 1]));
-      ms = j == 0 ? one : std::min(ms, one);
-    }
-    if (plan == usual) stay = ms;
-    if (q == 0 || ms < best) best = ms, pick = plan;
-  }
-  if (stay <= 1.03f * best) pick = usual;
+  apply(usual);
+  float best = timed(usual, 2);
+  reps = (int)std::max(1.0f, std::min(4.0f, 0.1f / std::max(best, 1e-3f)));  // short applications several to a run
+  best = 0.99f * std::min(best, timed(usual, 3));
+  int pick = usual;
+  auto against = [&](int plan) {
+    if (plan == usual) return;
+    apply(plan);
+    float ms = timed(plan, 1);
+    if (ms > 1.1f * best) return;
+    ms = std::min(ms, timed(plan, 2));
+    if (ms < best) best = ms, pick = plan;
+  };
+  against(0);
+  for (int plan : kTimedPlans) against(plan);
   for (hipEvent_t e : ev) (void)hipEventDestroy(e);
-  ev.clear();
-  return side_fusion[f] = pick;
+  d_cost.release();
+  if (pick != usual) op_cost_ratio = 0;  // the precisions' cost ratio was another plan's
+  return side_fusion[f32 ? 1 : 0] = pick;
 }
 
-void Engine::drop_plan_events() {
-  for (auto &v : plan_ev) {
-    for (hipEvent_t e : v) (void)hipEventDestroy(e);
-    v.clear();
-  }
+// Before a solve: the plans of the precisions that it applies are timed where
+// that is due (or asked for by pbfmm_set_side_fusion -1).
+void Engine::settle_plan(int precision) {
+  if (time_phases || (int64_t)near.rows.size() != n) return;  // vmult takes no plan then
+  for (int f = 0; f < (precision == PBFMM_MIXED && have_f32 ? 2 : 1); ++f)
+    if (side_fusion[f] < 0 && (plan_apps[f] < 0 || plan_apps[f] >= kSolvePlanAfter)) time_plans(f == 1);
 }
 
 int Engine::use_side_fusion(bool f32) {
-  int &mode = side_fusion[f32 ? 1 : 0];
-  if (mode >= 0) return mode;
   const int f = f32 ? 1 : 0;
-  // a caller's capture takes neither synchronisation nor timing
-  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-  HIPCHK(hipStreamIsCapturing(stream, &capturing));
-  if (capturing != hipStreamCaptureStatusNone) return first_plan(f32);
-  if (plan_apps[f] >= 0) return explore_plan(f32);
-  // pbfmm_set_side_fusion -1: timed now
-  const unsigned g = nblk(n, 256);
-  if (d_cost.bytes < (size_t)2 * n * 8) alloc(d_cost, (size_t)2 * n * 8);
-  double *u = d_cost.as<double>(), *v = d_cost.as<double>() + n;
-  hipLaunchKernelGGL(k_fill<double>, dim3(g), dim3(256), 0, stream, u, n, 1.0);
-  hipEvent_t t0, t1;
-  HIPCHK(hipEventCreate(&t0));
-  HIPCHK(hipEventCreate(&t1));
-  auto timed = [&](int plan, int reps) {  // ms per application, after one more
-    for (int rep = 0; rep <= reps; ++rep) {
-      if (rep == 1) HIPCHK(hipEventRecord(t0, stream));
-      if (f32)
-        matvec_fused<float>(u, d_outN.as<double>(), v, plan);
-      else
-        matvec_fused<double>(u, d_outN.as<double>(), v, plan);
-    }
-    HIPCHK(hipEventRecord(t1, stream));
-    HIPCHK(hipEventSynchronize(t1));
-    float ms = 0;
-    HIPCHK(hipEventElapsedTime(&ms, t0, t1));
-    return ms / reps;
-  };
-  float plain = timed(0, 2);
-  // short applications are repeated up to 0.4 ms a plan
-  const int reps = (int)std::max(2.0f, std::min(6.0f, 0.4f / std::max(plain, 1e-3f)));
-  if (reps > 2) plain = timed(0, reps);
-  float best = 0.98f * plain;
-  int pick = 0;
-  for (int plan : kTimedPlans) {
-    const float ms = timed(plan, reps);
-    if (ms < best) best = ms, pick = plan;
+  if (side_fusion[f] >= 0) return side_fusion[f];
+  if (solving == 0) {
+    // a caller's capture takes neither synchronisation nor timing
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    HIPCHK(hipStreamIsCapturing(stream, &capturing));
+    if (capturing != hipStreamCaptureStatusNone) return first_plan(f32);
+    if (plan_apps[f] < 0 || plan_apps[f] >= kPlanAfter) return time_plans(f32);
   }
-  (void)hipEventDestroy(t0);
-  (void)hipEventDestroy(t1);
-  mode = pick;
-  return mode;
+  if (plan_apps[f] >= 0) ++plan_apps[f];
+  return first_plan(f32);
 }
 
 // BEMProblem::vmult.  Without Dirichlet DoFs the reference shifts src and dst
@@ -3861,10 +3831,6 @@ void Engine::vmult(const double *src, double *dst, int precision) {
       matvec_fused<float>(xin, d_outN.as<double>(), dst, side);
     else
       matvec_fused<double>(xin, d_outN.as<double>(), dst, side);
-    if (plan_end) {
-      HIPCHK(hipEventRecord(plan_end, stream));
-      plan_end = nullptr;
-    }
   } else {
     if (f32)
       matvec_combined<float>(xin, d_outN.as<double>());
@@ -4082,16 +4048,15 @@ std::vector<int64_t> Engine::graph_key(int precision) const {
 }
 
 // step_op(d_vn -> d_wk) as a graph replay when that was measured faster.
-// The first steps per precision run directly, until kGraphAfter have run with
-// a timed launch plan (the choice costs eight steps and a capture and gains 3%
-// where it gains), the next captures the step after one more direct run (allocations on first use happen outside the
-// capture) and times three direct runs against three replays; from then on
-// the faster one runs, recaptured whenever graph_key changes.
+// The first kGraphAfter steps per precision run directly (the choice costs
+// eight steps and a capture and gains 3% where it gains), the next captures
+// the step after one more direct run (allocations on first use happen outside
+// the capture) and times three direct runs against three replays; from then
+// on the faster one runs, recaptured whenever graph_key changes.
 void Engine::step_op_graph(int precision) {
   const int f = precision == PBFMM_MIXED && have_f32 ? 1 : 0;
   double *vin = d_vn.as<double>(), *w = d_wk.as<double>();
-  if (!graph_enabled || graph_use[f] == 0 || side_fusion[f] < 0 ||
-      (graph_use[f] < 0 && graph_steps[f]++ < kGraphAfter)) {
+  if (!graph_enabled || graph_use[f] == 0 || (graph_use[f] < 0 && graph_steps[f]++ < kGraphAfter)) {
     step_op(vin, w, precision);
     return;
   }
@@ -4568,6 +4533,8 @@ bool Engine::mixed_relaxed() {
 
 int Engine::gmres(const double *b, double *x, double tol, int restart, int maxit, int precision, int *iters,
                   double *relres) {
+  settle_plan(precision);
+  Solving in_solve(solving);
   if (restart != gm_restart) {
     alloc(d_V, (size_t)(restart + 1) * n * 8);
     alloc(d_w, n * 8);
@@ -4952,6 +4919,8 @@ static int gmres_seg_outer(Engine &e, const SegCtx &c, const double *b, double *
 
 int Engine::gmres_forest(const double *b, double *x, double tol, int restart, int maxit, int precision,
                          int *iters, double *relres) {
+  settle_plan(precision);
+  Solving in_solve(solving);
   const int S = (int)seg_off.size() - 1;
   if (restart != gm_restart) {
     alloc(d_V, (size_t)(restart + 1) * n * 8);

@@ -1,0 +1,114 @@
+"""One launch plan for a whole solve.  Plans differ in the order of FP32 sums,
+so nothing is timed inside a solve: a handle's solves run the plan that the
+sizes suggest, and the plans are timed between solves once a handle has made
+as many applications as several solves make.
+
+Solutions of the same system by two solves to a true relative residual of
+1e-8 are compared with the bars of the graph tests: 1e-10 (FP64), 1e-7 (mixed)
+of the solution's norm.
+"""
+import numpy as np
+import pytest
+
+import pibem_amd as P
+from pibem_amd import hip
+from pibem_amd import mesh as M
+
+pytestmark = pytest.mark.gpu
+
+
+def rel(a, b):
+    return np.linalg.norm(np.asarray(a) - np.asarray(b)) / np.linalg.norm(b)
+
+
+def solve(f, rhs, precision):
+    x = hip.DeviceArray(f.n)
+    it, rr = f.gmres_dev(rhs.value, x.value, 1e-8, 100, 2000, precision)
+    hip.synchronize()
+    assert rr <= 1e-8
+    return x.numpy(), it
+
+
+def plans(f):
+    st = f.tuning_state()
+    return st["side_fusion_fp64"], st["side_fusion_fp32"]
+
+
+def test_no_timing_inside_a_solve():
+    """The spheroid's first mixed solve takes more FP32 applications than the
+    single ones after which plans are timed would, its second one as well;
+    neither ends on a timed plan, and two new handles solve alike."""
+    pr = M.config_spheroid(16, 6)
+    print(f"\n[case] {pr.mesh.name} N={pr.mesh.n_dofs}", flush=True)
+    got = []
+    for _ in range(2):
+        f = P.setup(pr, P.PBFMM_MIXED)
+        f.set_mixed_scheme(2)
+        bp = P.BEMProblem(f)
+        rhs = hip.DeviceArray.from_numpy(bp.compute_rhs(pr.tmp_rhs))
+        for _ in range(2):
+            got.append(solve(f, rhs, P.PBFMM_MIXED))
+            assert plans(f) == (-1, -1)
+        print(f"  steps {[it for _, it in got]}", flush=True)
+        f.close()
+    assert got[0][1] + got[1][1] > 48
+    for x, it in got[1:]:
+        assert abs(it - got[0][1]) <= 1 and rel(x, got[0][0]) <= 1e-7
+
+
+def test_plans_timed_between_solves():
+    """Both precisions in turn on two handles with streams of their own: the
+    plans are chosen before a later solve, and every solve, before and after,
+    equals plan 0's."""
+    pr = M.config_sphere(16, 4)
+    hs = [P.setup(pr, P.PBFMM_MIXED) for _ in range(2)]
+    bps = [P.BEMProblem(f) for f in hs]
+    rhs = [hip.DeviceArray.from_numpy(bp.compute_rhs(pr.tmp_rhs)) for bp in bps]
+    hs[0].set_mixed_scheme(2)
+    hs[1].set_mixed_scheme(2)
+    ref = P.setup(pr, P.PBFMM_MIXED)
+    ref.set_mixed_scheme(2)
+    want = {}
+    for prec in (P.PBFMM_FP64, P.PBFMM_MIXED):
+        ref.set_side_fusion(P.PBFMM_FP64, 0)
+        ref.set_side_fusion(P.PBFMM_MIXED, 0)
+        P.BEMProblem(ref).compute_alpha()
+        want[prec] = solve(ref, rhs[0], prec)[0]
+    applied = 0
+    for k in range(40):
+        for f, b in zip(hs, rhs):
+            before = plans(f)
+            for prec, bar in ((P.PBFMM_FP64, 1e-10), (P.PBFMM_MIXED, 1e-7)):
+                x, it = solve(f, b, prec)
+                assert rel(x, want[prec]) <= bar, (k, prec)
+            if applied < 200:  # a solve's FP64 applications: at most its steps and four residuals
+                assert before == (-1, -1)
+        applied += it + 4
+        if all(min(plans(f)) >= 0 for f in hs):
+            break
+    print(f"\n[case] plans {[plans(f) for f in hs]} after {k + 1} solves of each precision", flush=True)
+    assert all(min(plans(f)) >= 0 for f in hs)
+    for f in hs + [ref]:
+        f.close()
+
+
+@pytest.mark.parametrize("before", [0, 8, 20, 42])
+def test_cost_ratio_of_the_plans_in_use(before):
+    """The mixed scheme is chosen by the cost of the two operators as the solve
+    runs them, whatever single applications came before."""
+    pr = M.config_sphere(16, 4)
+    f = P.setup(pr, P.PBFMM_MIXED)
+    bp = P.BEMProblem(f)
+    rhs = hip.DeviceArray.from_numpy(bp.compute_rhs(pr.tmp_rhs))
+    y = hip.DeviceArray(f.n)
+    for _ in range(before):
+        bp.vmult_dev(rhs.value, y.value, P.PBFMM_FP64)
+    hip.synchronize()
+    solve(f, rhs, P.PBFMM_MIXED)
+    st = f.tuning_state()
+    assert plans(f) == (-1, -1)
+    assert st["mixed_scheme"] in (1, 2) and st["op_cost_ratio"] is not None
+    # both operators' launches are the same few; their costs differ by less than 8x either way
+    assert 0.125 < st["op_cost_ratio"] < 8
+    f.close()
+
