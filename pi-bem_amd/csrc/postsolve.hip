@@ -35,7 +35,8 @@ namespace {
 constexpr int kPsThreads = 256;
 constexpr double kPsTol = 1e-13;   // relative CG residual per component
 constexpr int kPsMaxIt = 4000;
-constexpr int kPsAhead = 12;       // steps enqueued before the host first reads the state, and between its reads
+constexpr int kPsCheck = 8;        // convergence is tested after every kPsCheck steps
+constexpr int kPsFirst = 32;       // steps before the host first reads the state (32 or 40 are usual)
 
 template <typename T>
 void ps_up(DevBuf &b, const std::vector<T> &v) {
@@ -198,13 +199,18 @@ __global__ void k_ps_gather_mass(int64_t n, const int32_t *__restrict__ d2c_ptr,
 // kPsParts), every workgroup in the same order, and workgroup 0 keeps the
 // scalars a later launch reads.  The product is taken of z instead of p:
 // with p = z + beta p_old, M p = M z + beta M p_old, so the new direction
-// needs no pass of its own before its product.  A step whose predecessor
-// converged (every component's |r|^2 <= kPsTol^2 |b|^2) does nothing, so the
-// host looks at the state only every few dozen steps.
+// needs no pass of its own before its product (the recurrence of q loses
+// nothing: after the same number of steps the error against extended
+// precision is a direct product's to two digits, 6,146 to 98,306 DoFs, axes
+// up to 10^4 apart).  Every kPsCheck steps the residual is tested (every
+// component's |r|^2 <= kPsTol^2 |b|^2), and the launches after a passed test
+// do nothing, so the host reads the state a few times per solve.  A test
+// after each step would save up to 7 steps and leave errors of 1e-13 to 3e-13,
+// where these end between 1e-15 and 7e-14.
 // Bound by latency: 98,306 DoFs (Q2, 1.6 M entries) stream 19 MB of matrix
 // per step.  Eight launches per step with one workgroup per 2048 rows took
 // 112 us a step, this form 25 us (a whole projection with pressure, force and
-// volume on host vectors 4.88 -> 1.80 ms).
+// volume on host vectors 4.88 -> 1.94 ms).
 // ---------------------------------------------------------------------------
 constexpr int kPsParts = 512;
 constexpr int kPsLanes = 4;  // per row of M: 9 to 25 entries (8 and 16 lanes: 3 and 8% slower solves)
@@ -274,17 +280,20 @@ __global__ void __launch_bounds__(kPsThreads)
                 const double *__restrict__ val, const double *__restrict__ z, double *__restrict__ p,
                 double *__restrict__ q, const double *__restrict__ rz_part, const double *__restrict__ rr_part,
                 double *__restrict__ pq_part, double *__restrict__ cg) {
-  __shared__ double sh[kPsThreads / 64][6];
-  if (cg[kDone] != 0.0) return;
+  __shared__ double sh[kPsThreads / 64][6], done;
+  // workgroup 0 of this launch may set the flag: one thread reads it for its
+  // whole workgroup, which returns below either way
+  if (threadIdx.x == 0) done = cg[kDone];
   const int P = (int)gridDim.x;
   // rz_k, and |r|^2 (|b|^2 in step 0: then rr_part is its array)
   double s[6];
   ps_part_sums(rz_part, P, s);
   ps_part_sums(rr_part, P, s + 3);
-  ps_block_sums<6>(s, sh);
+  ps_block_sums<6>(s, sh);  // its barriers order the flag too
+  if (done != 0.0) return;
   const double *rz_old = cg + kRZ + 3 * ((k + 1) & 1);
   double be[3];
-  bool conv = true;
+  bool conv = k % kPsCheck == 0;
   for (int d = 0; d < 3; ++d) {
     be[d] = k > 0 && rz_old[d] > 0.0 ? s[d] / rz_old[d] : 0.0;
     if (k > 0 ? s[3 + d] > kPsTol * kPsTol * cg[kBB + d] : s[3 + d] != 0.0) conv = false;
@@ -297,7 +306,7 @@ __global__ void __launch_bounds__(kPsThreads)
     cg[kSteps] = k;
   }
   if (conv) {
-    // the other workgroups decide the same from the same sums; the flag is for later launches
+    // the other workgroups decide the same from the same sums; the flag is for later tests
     if (blockIdx.x == 0 && threadIdx.x == 0) cg[kDone] = 1.0;
     return;
   }
@@ -647,7 +656,8 @@ void Engine::ps_project(int mode, const double *in1, const double *in2, double *
   double h[kCgLen];
   for (int it = 0; ; ) {
     if (it >= kPsMaxIt) throw std::runtime_error("mass-matrix CG did not converge");
-    for (int k = 0; k < kPsAhead; ++k, ++it) {
+    // up to and with the launch that tests after kPsFirst steps, then test by test
+    for (int k = it == 0 ? kPsFirst + 1 : kPsCheck; k > 0; --k, ++it) {
       hipLaunchKernelGGL(k_ps_cg_dir, dim3(G), dim3(kPsThreads), 0, stream, n, it, ps.m_ptr.as<int32_t>(),
                          ps.m_col.as<int32_t>(), ps.m_val.as<double>(), z, p, q, rz_part[it & 1], rr_part, pq_part, cg);
       hipLaunchKernelGGL(k_ps_cg_update, dim3(G), dim3(kPsThreads), 0, stream, n, it, diag, p, q, x, r, z, pq_part,
