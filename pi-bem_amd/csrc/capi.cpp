@@ -5,8 +5,10 @@
 #include <cstring>
 #include <atomic>
 #include <exception>
+#include <new>
 #include <string>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "engine.h"
@@ -78,6 +80,31 @@ void ensure_alpha(pbfmm_handle *h) {
     h->alpha_ready = true;
     h->eng.have_prec = false;
   }
+}
+void configure(Engine &e, const pbfmm_params &p) {
+  e.p = p.trunc_order;
+  e.kt = kt_of(p.trunc_order);
+  e.kp = kp_of(p.trunc_order);
+  e.L = p.num_octree_levels;
+  e.sing_order = p.sing_quad_order;
+  e.sing_rule = p.sing_rule;
+}
+// A new engine for a handle that takes another mesh: buffers, plans, graphs
+// and timed choices are kept under keys (a restart length, a number of
+// right-hand sides) that say nothing of the mesh, so none of them stays.
+void renew_engine(pbfmm_handle *h) {
+  Engine &e = h->eng, choices;
+  choices.take_choices(e);
+  if (h->device_ready) {
+    if (hipSetDevice(h->prm.device) != hipSuccess) throw HipError("hipSetDevice failed");
+    e.sync();
+  }
+  static_assert(std::is_nothrow_default_constructible<Engine>::value, "nothing can fail between the two");
+  e.~Engine();
+  new (&e) Engine();
+  h->device_ready = false;
+  configure(e, h->prm);
+  e.take_choices(choices);
 }
 // device staging buffer of at least `bytes`, grown on demand
 void *stage(DevBuf &b, size_t bytes) {
@@ -156,12 +183,7 @@ int pbfmm_create(const pbfmm_params *p, pbfmm_handle **out) {
   try {
     h = new pbfmm_handle();
     h->prm = *p;
-    h->eng.p = p->trunc_order;
-    h->eng.kt = kt_of(p->trunc_order);
-    h->eng.kp = kp_of(p->trunc_order);
-    h->eng.L = p->num_octree_levels;
-    h->eng.sing_order = p->sing_quad_order;
-    h->eng.sing_rule = p->sing_rule;
+    configure(h->eng, *p);
   } catch (...) {
     delete h;
     return PBFMM_ERR_HIP;
@@ -190,9 +212,7 @@ int pbfmm_init_fma(pbfmm_handle *h, int64_t n_dofs, const double *xyz, int64_t n
       return fail(h, PBFMM_ERR_ARG, "init_fma: sizes exceed the 32-bit index range of this build");
     if ((dbl_ptr == nullptr) != (dbl_idx == nullptr))
       return fail(h, PBFMM_ERR_ARG, "init_fma: dbl_ptr and dbl_idx must both be given or both be null");
-    Engine &e = h->eng;
-    HostMesh &m = e.mesh;
-    m = HostMesh();
+    HostMesh m;
     m.n = n_dofs;
     m.ncells = n_cells;
     m.ncells_real = n_cells;
@@ -229,9 +249,6 @@ int pbfmm_init_fma(pbfmm_handle *h, int64_t n_dofs, const double *xyz, int64_t n
       m.dbl_ptr[i + 1] = (int32_t)m.dbl_idx.size();
     }
     m.dir.assign(dirichlet_mask, dirichlet_mask + n_dofs);
-    e.have_dirichlet = false;
-    for (auto v : m.dir)
-      if (v) e.have_dirichlet = true;
     // dof -> cells
     m.d2c_ptr.assign(n_dofs + 1, 0);
     for (int64_t i = 0; i < n_cells * dpc; ++i) m.d2c_ptr[m.cdofs[i] + 1]++;
@@ -240,11 +257,14 @@ int pbfmm_init_fma(pbfmm_handle *h, int64_t n_dofs, const double *xyz, int64_t n
     std::vector<int32_t> fill(m.d2c_ptr.begin(), m.d2c_ptr.end() - 1);
     for (int64_t c = 0; c < n_cells; ++c)
       for (int j = 0; j < dpc; ++j) m.d2c_idx[fill[m.cdofs[c * dpc + j]]++] = (int32_t)c;
+    if (h->stage > 0) renew_engine(h);
+    Engine &e = h->eng;
+    e.have_dirichlet = std::any_of(m.dir.begin(), m.dir.end(), [](uint8_t v) { return v != 0; });
+    e.mesh = std::move(m);
     e.n = n_dofs;
     e.dpc = dpc;
     h->stage = 1;
     h->alpha_ready = false;
-    e.have_constraints = false;
     return PBFMM_OK;
   }, false);
 }
@@ -1068,7 +1088,7 @@ int pbfmm_set_side_fusion(pbfmm_handle *h, int32_t precision, int32_t mode) {
   if (precision != PBFMM_FP64 && precision != PBFMM_MIXED)
     return fail(h, PBFMM_ERR_ARG, "set_side_fusion: unknown precision");
   const int pi = precision == PBFMM_MIXED ? 1 : 0;
-  h->eng.side_fusion[pi] = mode;
+  h->eng.side_fusion[pi] = h->eng.set_plan[pi] = mode;
   if (mode == -1) h->eng.plan_apps[pi] = -1;  // timed before the next application or solve
   return PBFMM_OK;
 }
@@ -1094,7 +1114,7 @@ int pbfmm_set_graph_mode(pbfmm_handle *h, int32_t mode) {
   if (mode < -1 || mode > 1) return fail(h, PBFMM_ERR_ARG, "set_graph_mode: mode must be -1, 0 or 1");
   Engine &e = h->eng;
   e.graph_enabled = mode != 0;
-  e.graph_use[0] = e.graph_use[1] = mode;
+  e.graph_use[0] = e.graph_use[1] = e.set_graph = mode;
   e.graph_steps[0] = e.graph_steps[1] = Engine::kGraphAfter;  // -1: timed in the next steps
   return PBFMM_OK;
 }

@@ -160,6 +160,19 @@ struct Engine {
   void collect_phase_times();
 
   void init_device(int dev, void *stream);
+  // What callers set through the API, from the engine of an earlier mesh;
+  // everything else of a handle belongs to its mesh.
+  void take_choices(const Engine &o) {
+    prec_rows = o.prec_rows;
+    mixed_scheme = o.mixed_scheme;
+    inner_reduction = o.inner_reduction;
+    relax_switch = o.relax_switch;
+    reorth_eta = o.reorth_eta;
+    time_phases = o.time_phases;
+    for (int f = 0; f < 2; ++f) side_fusion[f] = set_plan[f] = o.set_plan[f];
+    graph_use[0] = graph_use[1] = set_graph = o.set_graph;
+    graph_enabled = o.graph_enabled;
+  }
   ~Engine();
   void upload_mesh_and_tree();
   void upload_near_plan();
@@ -229,6 +242,8 @@ struct Engine {
   template <typename T>
   void launch_m2l_slots(const T *ops, const T *IN, T *LE);
   int side_fusion[2] = {-1, -1};
+  // the caller's own choices (pbfmm_set_side_fusion, pbfmm_set_graph_mode), -1: timed
+  int set_plan[2] = {-1, -1}, set_graph = -1;
   // One Arnoldi step's operator (preconditioner + vmult, step_op) captured
   // into a HIP graph per step precision ([0] FP64, [1] FP32) on the fixed
   // buffers d_vn (the step's input, the last basis vector) -> d_wk, used when

@@ -2909,7 +2909,7 @@ void Engine::assemble_near(bool want_f32) {
   up(d_scnt, cnt);
 
   const int64_t nv = std::max<int64_t>(near.nnz, 1) * 2;
-  f32.opvals_p.release();  // of an earlier mesh
+  f32.opvals_p.release();  // of an earlier assembly
   alloc(f64.vals, (size_t)nv * sizeof(double));
   DevBuf d_quads, d_units, d_colpos;  // freed at the end, after the stream has run
   if (near.nleaf > 0 && near.nnz > 0) {
