@@ -232,7 +232,8 @@ struct Engine {
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   void make_side_stream();
   void fork_side();
-  int m2l_beside() const;  // workgroups of an M2L launch beside the SpMV, 0: one per chunk
+  int cus = 256;  // compute units of the device
+  int m2l_beside(bool f32, int nk) const;  // workgroups of an M2L launch beside the SpMV, 0: one per chunk
   // slot M2L: targets, their slot ranges (CSR) and each pair's slot, the
   // slots of one target consecutive (its pairs in ascending order)
   DevBuf d_red_tgt, d_red_beg, d_slot_pos;

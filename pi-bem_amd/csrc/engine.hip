@@ -1382,13 +1382,14 @@ static_assert(kM2LChunk == 32 && kChunk1 == 64, "k_translate maps 2 x 32 or 1 x 
 // K = 84 307 / 190, near what its atomic adds take alone (305 / 177);
 // 211,368 pairs at order 7: 5 wavefronts of 80 rows 122 / 75, 8 of 64 rows
 // 92 / 54, into slots 109 / 45 and 56 / 31.
+__host__ __device__ constexpr int tr_column_waves(int nr) { return nr % 2 == 0 || nr > 4 ? 2 : 4; }
 template <int P, typename T, int KIND>
 struct TrLayout {
   static constexpr int KP = Kp<P>::value, KC = Kp<P>::cols;
   static constexpr int BS = KC + 2;
   static constexpr int CS = sizeof(T) == 4 ? KP + 4 : KP + 1;
   static constexpr int NR = KP / 16;        // 16-row tiles
-  static constexpr int CW = NR % 2 == 0 || NR > 4 ? 2 : 4;
+  static constexpr int CW = tr_column_waves(NR);
   static constexpr int NT = 64 * NR * CW;   // threads per block
   static constexpr int elems = 64 * (BS > CS ? BS : CS);
   static constexpr size_t bytes = (size_t)elems * sizeof(T);
@@ -1593,7 +1594,7 @@ __global__ void __launch_bounds__((TrLayout<P, T, KIND>::NT)) k_translate(TrArgs
 }
 
 // M2L by fewer workgroups than chunks (a multiple
-// of 8, see kM2LBeside): each takes every (gridDim.x / 8)th chunk of its XCD's
+// of 8, see m2l_beside): each takes every (gridDim.x / 8)th chunk of its XCD's
 // run.  A kernel of its own, since the loop's registers cost the others
 // occupancy (order 8 FP64 M2L into slots 272 -> 358 us).
 template <typename T, int P, int NK>
@@ -2600,6 +2601,7 @@ static std::vector<D> cast_vec(const std::vector<S> &v) {
 void Engine::init_device(int dev, void *st) {
   device = dev;
   HIPCHK(hipSetDevice(dev));
+  HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   if (st) {
     stream = (hipStream_t)st;
     own_stream = false;
@@ -3305,13 +3307,21 @@ void Engine::fork_side() {
 // workgroup per chunk / one per CU: 393,218 DoFs FP64 1,266 / 1,142, FP32
 // 716 / 627; 98,306 390 / 343, 239 / 208.  Both kernels' products of 98,306
 // DoFs (host vectors) 1,026 / 887.  Where M2L is the longer of the two it
-// wants all of the chip: 40,346 DoFs, order 7, leaf 20 (62 values per pair)
-// 190 / 201; both kernels' products of 38,402 DoFs, leaf 80 (481 per pair)
-// 439 / 493.  The line lies between there and 98,306 DoFs at leaf 80 (643).
-constexpr int kM2LBeside = 256;
-constexpr int64_t kBesideValues = 512;
-int Engine::m2l_beside() const {
-  return near.nnz > kBesideValues * (int64_t)far.m2l.tgt.size() ? kM2LBeside : 0;
+// wants all of the chip: 24,578 DoFs, order 6, leaf 32 (95 values per pair)
+// 109 / 117.  Where the lines lie, per chunk / per CU at values per pair:
+//   FP64 operator, 256: 201 135 / 141 us, 317 97 / 95, 325 579 / 541, 452 81 /
+//   78, 481 142 / 135, 507 (order 8) 367 / 327.
+//   FP32 operator: its SpMV is half as long beside an M2L of more than half
+//   the time.  With workgroups of 12 wavefronts and more (orders 5, 8 and up)
+//   256 too: 316 258 / 236 (order 8), 194 / 174 (order 5); with 8 or 4, 512:
+//   316 181 / 193, 325 317 / 358, 450 77 / 80, 507 169 / 172, and 1030 even.
+//   Both kernels' products (two expansions to a pair), 512: 317 309 / 333,
+//   481 424 / 427, 643 973 / 879.
+int Engine::m2l_beside(bool f32, int nk) const {
+  const int nr = kp / 16;
+  const bool wide = nr * tr_column_waves(nr) >= 12;
+  const int64_t values = nk == 1 && (!f32 || wide) ? 256 : 512;
+  return near.nnz > values * (int64_t)far.m2l.tgt.size() ? cus / 8 * 8 : 0;
 }
 
 // Downward pass and near field.  NK = 2: outN = N.phi, outD = D.dphi;
@@ -3339,7 +3349,7 @@ void Engine::products(const double *phi, const double *dphi, double *outN, doubl
     launch_m2l_slots<T>(F.m2l.template as<T>(), F.me.template as<T>(), F.le.template as<T>());
   else
     launch_translate<T, 1, NK>(*this, stream, m2l_cl, 0, nchunks<NK>(far.m2l), F.m2l.template as<T>(),
-                               F.me.template as<T>(), F.le.template as<T>(), nullptr, beside ? m2l_beside() : 0);
+                               F.me.template as<T>(), F.le.template as<T>(), nullptr, beside ? m2l_beside(sizeof(T) == 4, NK) : 0);
   mark(6);
   const int64_t nitems = (int64_t)far.m2p_item_node.size();
   auto m2p = [&]() {  // adds to the SpMV's rows
@@ -3609,7 +3619,7 @@ void Engine::matvec_fused(const double *x, double *out, double *dst, int side) {
     near_done = true;
   }
   if (fork_later) fork_spmv();
-  const int m2l_wg = fork_later ? m2l_beside() : 0;
+  const int m2l_wg = fork_later ? m2l_beside(sizeof(T) == 4, 1) : 0;
   // M2L, carrying M2P (sides 2, 3) and the SpMV (side 3, or whatever no M2M
   // launch took)
   const int c1 = nchunks<1>(far.m2l);
