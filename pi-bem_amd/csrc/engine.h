@@ -48,7 +48,7 @@ struct FarDev {
   DevBuf opvals_p;  // FP32 only: opvals in row pairs (k_round_f32_pairs)
   // opvals in column vectors of 16 bytes (k_round_cols), per-leaf offsets
   DevBuf opvals_q, qval_beg;
-  DevBuf slots;  // slot M2L: [pair][2 Kt], on first use
+  DevBuf slots;  // slot M2L: [pair][kp], on first use
 };
 
 // Mixed precision: the relaxed scheme spends its first steps (about a
@@ -238,6 +238,7 @@ struct Engine {
   // slots of one target consecutive (its pairs in ascending order)
   DevBuf d_red_tgt, d_red_beg, d_slot_pos;
   int n_red_tgt = 0;
+  size_t slot_bytes(size_t value_bytes) const;
   template <typename T>
   T *m2l_slots();
   template <typename T>

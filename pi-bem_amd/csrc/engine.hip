@@ -3453,7 +3453,10 @@ void Engine::consumer_levels() {
 }
 
 // The slot M2L's buffers on first use: per target the pair indices of the
-// M2L chunk list (ascending), and [pair][2 Kt] slots of the precision.
+// M2L chunk list (ascending), and [pair][kp] slots of the precision.
+size_t Engine::slot_bytes(size_t value_bytes) const {
+  return std::max<size_t>(far.m2l.tgt.size(), 1) * kp * value_bytes;
+}
 template <typename T>
 T *Engine::m2l_slots() {
   FarDev<T> &F = far_of<T>(*this);
@@ -3476,7 +3479,7 @@ T *Engine::m2l_slots() {
     up(d_slot_pos, slot);
     n_red_tgt = (int)tg.size();
   }
-  const size_t bytes = (size_t)std::max<int64_t>(npair, 1) * kp * sizeof(T);
+  const size_t bytes = slot_bytes(sizeof(T));
   if (F.slots.bytes < bytes) alloc(F.slots, bytes);
   return F.slots.template as<T>();
 }
@@ -3795,17 +3798,28 @@ void Engine::settle_plan(int precision) {
 }
 
 int Engine::use_side_fusion(bool f32) {
-  const int f = f32 ? 1 : 0;
-  if (side_fusion[f] >= 0) return side_fusion[f];
-  if (solving == 0) {
-    // a caller's capture takes neither synchronisation nor timing
+  const int f = f32 ? 1 : 0, set = side_fusion[f];
+  int plan = set >= 0 ? set : first_plan(f32);
+  // what the plan would make on first use
+  const DevBuf &slots = f32 ? this->f32.slots : f64.slots;
+  const bool no_slots = (plan & 4) && (!d_red_beg.p || slots.bytes < slot_bytes(f32 ? 4 : 8));
+  const bool no_stream = (plan & 8) && !side_stream;
+  if (no_slots || no_stream || (set < 0 && solving == 0)) {
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     HIPCHK(hipStreamIsCapturing(stream, &capturing));
-    if (capturing != hipStreamCaptureStatusNone) return first_plan(f32);
-    if (plan_apps[f] < 0 || plan_apps[f] >= kPlanAfter) return time_plans(f32);
+    if (capturing != hipStreamCaptureStatusNone) {
+      // a caller's capture takes no allocation, synchronisation or timing:
+      // M2L with atomic adds for slots that are not there, and the SpMV on
+      // the caller's stream for a second one that is not
+      if (no_slots) plan &= ~4;
+      if (no_stream) plan &= 3;
+      return plan;
+    }
   }
+  if (set >= 0) return set;
+  if (solving == 0 && (plan_apps[f] < 0 || plan_apps[f] >= kPlanAfter)) return time_plans(f32);
   if (plan_apps[f] >= 0) ++plan_apps[f];
-  return first_plan(f32);
+  return plan;
 }
 
 // BEMProblem::vmult.  Without Dirichlet DoFs the reference shifts src and dst
