@@ -2475,10 +2475,12 @@ __global__ void k_seg_scale(int64_t n, const int *__restrict__ seg, const double
 
 // Segmented GMRES building blocks: every part of a forest runs its own
 // Arnoldi process inside shared basis vectors.  Dots over part-aligned chunks
-// (part[j * nch + c]), which the kernels that use the sums finish themselves:
-// a launch of this size takes 3 to 4 us whatever it does, and with launches
-// for the sums and the norm a step took nine of them instead of five (twelve
-// spheroids of 1.5k to 5.4k DoFs, mixed solve 5.31 -> 4.77 ms).
+// (part[j * nch + c]).  In parts of few chunks the kernels that use the sums
+// finish them themselves: a launch of this size takes 3 to 4 us whatever it
+// does, and with launches for the sums and the norm a step took nine of them
+// instead of five (twelve spheroids of 1.5k to 5.4k DoFs, mixed solve 5.31 ->
+// 4.77 ms).  In larger parts (kOwnSums) every workgroup would repeat a long
+// sum, so a launch does it once.
 __global__ void __launch_bounds__(kRedThreads) k_mdot_seg(const int64_t *__restrict__ cbeg, int64_t ldv,
                                                           const double *__restrict__ V, const double *__restrict__ w,
                                                           double *__restrict__ part) {
@@ -2490,17 +2492,27 @@ __global__ void __launch_bounds__(kRedThreads) k_mdot_seg(const int64_t *__restr
   const double r = block_sum(acc, sh);
   if (threadIdx.x == 0) part[(int64_t)j * gridDim.x + blockIdx.x] = r;
 }
-// w -= sum_j V_j h[part][j], h[part][j] the sum of the part's chunks in
-// part[j * nch + c], by every workgroup of the part in the same order; the
-// first stores it in h_out[part * ldh + j].  Workgroup (c, y) takes rows
-// 256 y .. of chunk c, so that it has one part, and stores the sum of squares
-// of its new w in npart[c * gridDim.y + y] when npart is given.  nv <= 128.
+// h[part * ldh + j] = the sum of the part's chunks in part[j * nch + c]
+__global__ void __launch_bounds__(64) k_finish_seg(int nch, const int *__restrict__ sch_off, int ldh,
+                                                   const double *__restrict__ part, double *__restrict__ h) {
+  const int s = blockIdx.x, j = blockIdx.y;
+  double acc = 0;
+  for (int c = sch_off[s] + threadIdx.x; c < sch_off[s + 1]; c += 64) acc += part[(int64_t)j * nch + c];
+  acc = wave_sum(acc);
+  if (threadIdx.x == 0) h[(int64_t)s * ldh + j] = acc;
+}
+// w -= sum_j V_j h[part][j], h as k_finish_seg left it (part null), or the sum
+// of the part's chunks in part[j * nch + c] by every workgroup of the part in
+// the same order; the first then stores it in h[part * ldh + j].  Workgroup
+// (c, y) takes rows 256 y .. of chunk c, so that it has one part, and stores
+// the sum of squares of its new w in npart[c * gridDim.y + y] when npart is
+// given.
 __global__ void __launch_bounds__(kRedThreads) k_gemv_sub_seg(const int64_t *__restrict__ cbeg,
                                                               const int *__restrict__ seg,
                                                               const int *__restrict__ sch_off, int64_t ldv, int nv,
                                                               const double *__restrict__ V,
                                                               const double *__restrict__ part, int ldh,
-                                                              double *__restrict__ h_out, double *__restrict__ w,
+                                                              double *__restrict__ hv, double *__restrict__ w,
                                                               double *__restrict__ npart) {
   __shared__ double hs[kRedThreads], sh[kRedThreads / 64];
   const int c = blockIdx.x, nch = gridDim.x, t = (int)threadIdx.x;
@@ -2512,12 +2524,14 @@ __global__ void __launch_bounds__(kRedThreads) k_gemv_sub_seg(const int64_t *__r
   for (int j0 = 0; j0 < nv; j0 += kRedThreads) {  // a batch's restart has no upper limit
     const int nj = min(kRedThreads, nv - j0);
     if (j0 > 0) __syncthreads();
-    if (t < nj) {
+    if (t < nj && !part) {
+      hs[t] = hv[(int64_t)s * ldh + j0 + t];
+    } else if (t < nj) {
       double h = 0;
 #pragma unroll 4
       for (int q = c0; q < c1; ++q) h += part[(int64_t)(j0 + t) * nch + q];
       hs[t] = h;
-      if (c == c0 && blockIdx.y == 0) h_out[(int64_t)s * ldh + j0 + t] = h;
+      if (c == c0 && blockIdx.y == 0) hv[(int64_t)s * ldh + j0 + t] = h;
     }
     __syncthreads();
     if (row)
@@ -3216,7 +3230,10 @@ static void launch_spmm(Engine &e, const double *x, double *out, int R) {
 // 0.303 ms FP64; leaf 80: 0.492 against 0.354, 0.929 against 0.674); FP32 with
 // few values also the workgroup per leaf, row-major and in row pairs (24,578
 // DoFs, leaf 20: 16.4 and 14.7 us, column vectors 17.2 us).  The others stay
-// for pbfmm_set_spmv_kernel.  A kernel whose first launch takes
+// for pbfmm_set_spmv_kernel: on ellipsoids none of them is ahead by more than
+// 1%, on hulls mirrored at the waterline (3,872 to 22,876 DoFs, leaf 20 to 96,
+// all DoFs the columns of every row) FP64 kernels 0 and 2 take 3 to 60% and
+// 50 to 270% longer for the operator.  A kernel whose first launch takes
 // half as long again as the best time so far is not timed further.
 template <typename T, int NK>
 void Engine::tune_spmv() {
@@ -4689,6 +4706,7 @@ void Engine::seg_norms(const double *v, std::vector<double> &out) {
 struct SegCtx {
   int64_t N = 0;                 // total vector length
   int S = 0, nch = 0;            // parts; part-aligned reduction chunks
+  int part_nch = 0;              // chunks of the largest part
   const int *seg = nullptr;      // part of each entry
   const int64_t *seg_off = nullptr, *rch = nullptr;
   const int *sch = nullptr;
@@ -4707,6 +4725,12 @@ static void seg_norms_ctx(Engine &e, const SegCtx &c, const double *v, std::vect
   e.sync();
   for (double &x : out) x = std::sqrt(x);
 }
+
+// Chunks of the largest part up to which k_gemv_sub_seg sums them by itself.
+// Lockstep solves of two right-hand sides, mixed, own sums / a launch for
+// them: 19 chunks (38,402 DoFs) 9.77 / 9.85 ms, 49 25.56 / 25.51, 118 58.7 /
+// 58.9, 193 (393,218 DoFs) 94.6 / 92.5.
+constexpr int kOwnSums = 128;
 
 // r0 (device) with per-part norms r0n, when given, is the residual b - A x
 // of the starting x: the first cycle then skips its operator application.
@@ -4733,8 +4757,10 @@ static int gmres_core_seg(Engine &e, const SegCtx &c, const double *b, double *x
   double *npart = part + (size_t)nch * (m + 2);
   auto project = [&](int nv, double *vec, double *h, double *np) {  // vec -= V h, h = V . vec
     hipLaunchKernelGGL(k_mdot_seg, dim3(nch, nv), dim3(kRedThreads), 0, e.stream, rch, n, V, vec, part);
+    if (c.part_nch > kOwnSums)
+      hipLaunchKernelGGL(k_finish_seg, dim3(S, nv), dim3(64), 0, e.stream, nch, sch, ldh, part, h);
     hipLaunchKernelGGL(k_gemv_sub_seg, dim3(nch, kSubs), dim3(kRedThreads), 0, e.stream, rch, seg, sch, n, nv, V,
-                       part, ldh, h, vec, np);
+                       c.part_nch > kOwnSums ? nullptr : part, ldh, h, vec, np);
   };
   // relaxed mixed precision (sw given): the FP64 operator until every
   // active part's estimate is below its switch level sw[s], then the inner
@@ -4972,6 +4998,7 @@ int Engine::gmres_forest(const double *b, double *x, double tol, int restart, in
   c.N = n;
   c.S = S;
   c.nch = n_rch;
+  for (int s = 0; s < S; ++s) c.part_nch = std::max(c.part_nch, (int)nblk(seg_off[s + 1] - seg_off[s], kRedChunk));
   c.seg = d_seg.as<int>();
   c.seg_off = d_seg_off.as<int64_t>();
   c.rch = d_rch_beg.as<int64_t>();
@@ -5166,6 +5193,7 @@ int Engine::gmres_multi(const double *b, double *x, int R, double tol, int resta
   c.N = N;
   c.S = R;
   c.nch = mr_nch;
+  c.part_nch = (int)nblk(n, kRedChunk);
   c.seg = mr_seg.as<int>();
   c.seg_off = mr_seg_off.as<int64_t>();
   c.rch = mr_rch.as<int64_t>();
