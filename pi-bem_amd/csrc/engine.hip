@@ -173,23 +173,20 @@ __global__ void k_pack_quads(int64_t n, const double *__restrict__ qx, const dou
   out[4 * g + 3] = double2{qw[g], 0.0};
 }
 
-// The column of each of an entry's DoFs in its leaf's sorted columns.
+// The column of each of an entry's DoFs in its leaf's sorted columns; *missing
+// is set where one is none of them (a malformed plan).
 __global__ void __launch_bounds__(256) k_entry_cols(const int *__restrict__ ent_beg, const int *__restrict__ ent_cell,
                                                     const int *__restrict__ cdofs, int dpc,
                                                     const int *__restrict__ col_beg, const int *__restrict__ cols,
-                                                    int *__restrict__ colpos) {
+                                                    int *__restrict__ colpos, int *__restrict__ missing) {
   const int leaf = blockIdx.x;
   const int64_t e0 = (int64_t)ent_beg[leaf] * dpc, e1 = (int64_t)ent_beg[leaf + 1] * dpc;
   const int cb = col_beg[leaf], C = col_beg[leaf + 1] - cb;
   for (int64_t i = e0 + blockIdx.y * 256 + threadIdx.x; i < e1; i += (int64_t)gridDim.y * 256) {
     const int e = (int)(i / dpc), d = cdofs[(int64_t)ent_cell[e] * dpc + (int)(i - (int64_t)e * dpc)];
-    int lo = 0, hi = C - 1;  // every DoF of an entry is a column
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (cols[cb + mid] < d) lo = mid + 1;
-      else hi = mid;
-    }
-    colpos[i] = lo;
+    const int at = find_sorted(cols + cb, 0, C, d);
+    if (at < 0) *missing = 1;
+    colpos[i] = max(at, 0);
   }
 }
 
@@ -1067,21 +1064,18 @@ __global__ void __launch_bounds__(256) k_p2m_unit(
   }
 }
 
-// The column of each DoF of a quad point's cell among its leaf's columns.
+// The column of each DoF of a quad point's cell among its leaf's columns;
+// *missing is set where one is none of them.
 __global__ void k_quad_cols(int64_t n, int dpc, int nrule, const int *__restrict__ qpt, const int *__restrict__ qleaf,
                             const int *__restrict__ cdofs, const int *__restrict__ col_beg,
-                            const int *__restrict__ col_dof, int *__restrict__ qcol) {
+                            const int *__restrict__ col_dof, int *__restrict__ qcol, int *__restrict__ missing) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= n) return;
   const int64_t pt = i / dpc;
   const int d = cdofs[(int64_t)(qpt[pt] / nrule) * dpc + (int)(i - pt * dpc)];
-  int lo = col_beg[qleaf[pt]], hi = col_beg[qleaf[pt] + 1] - 1;  // every DoF of its cells is a column
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (col_dof[mid] < d) lo = mid + 1;
-    else hi = mid;
-  }
-  qcol[i] = lo;
+  const int beg = col_beg[qleaf[pt]], at = find_sorted(col_dof, beg, col_beg[qleaf[pt] + 1], d);
+  if (at < 0) *missing = 1;
+  qcol[i] = at < 0 ? beg : at;
 }
 
 // Set-up, FP64, one workgroup per leaf whose unit multipoles fit in LDS: the
@@ -2781,6 +2775,14 @@ void Engine::upload_far(bool want_f32) {
 // (7 M) 380 / 345, 38,402 Q2 at leaf 20 (15 M) 533 / 473, 98,306 1,027 / 887.
 constexpr int64_t kPairsBeside = 1000000;
 
+// Throws where k_entry_cols or k_quad_cols found a DoF in no column.
+static void check_columns(const Engine &e, const DevBuf &missing, const char *what) {
+  int32_t bad = 0;
+  HIPCHK(hipMemcpyAsync(&bad, missing.p, sizeof(bad), hipMemcpyDeviceToHost, e.stream));
+  HIPCHK(hipStreamSynchronize(e.stream));
+  if (bad) throw std::runtime_error(std::string("plan check: ") + what);
+}
+
 // Unit multipoles of every leaf (FP64, rounded once for the FP32 operator).
 void Engine::build_unit_multipoles(bool want_f32) {
   const int64_t ncol = (int64_t)far.p2m_col_dof.size();
@@ -2814,12 +2816,13 @@ void Engine::build_unit_multipoles(bool want_f32) {
         }
       }
     }
-    DevBuf qpt, qleaf, qcol, dqbeg, dfit, dfit_half;
+    DevBuf qpt, qleaf, qcol, dqbeg, dfit, dfit_half, missing;
+    up(missing, std::vector<int32_t>{0});
     auto quad_cols = [&](const DevBuf &pt, const DevBuf &leaf, DevBuf &col, int64_t count) {
       alloc(col, (size_t)count * dpc * sizeof(int));
       hipLaunchKernelGGL(k_quad_cols, dim3(nblk(count * dpc, 256)), dim3(256), 0, stream, count * dpc, dpc, nq,
                          pt.as<int>(), leaf.as<int>(), d_cdofs.as<int>(), d_p2m_col_beg.as<int>(),
-                         d_p2m_col_dof.as<int>(), col.as<int>());
+                         d_p2m_col_dof.as<int>(), col.as<int>(), missing.as<int>());
     };
     up(qpt, far.p2m_qpt);
     up(qleaf, far.p2m_qleaf);
@@ -2861,6 +2864,7 @@ void Engine::build_unit_multipoles(bool want_f32) {
     }
     // the products' second stream is made (0.2 ms) while the GPU is busy here
     if (near.nnz >= kPairsBeside) make_side_stream();
+    check_columns(*this, missing, "p2m column");
     sync();  // qpt, qleaf, qcol, dqbeg, dfit, dfit_half are freed on return
   }
   // the operator's unit multipoles (U1 on Neumann, -U2 on Dirichlet DoFs)
@@ -2927,7 +2931,8 @@ void Engine::assemble_near(bool want_f32) {
   const int64_t nv = std::max<int64_t>(near.nnz, 1) * 2;
   f32.opvals_p.release();  // of an earlier assembly
   alloc(f64.vals, (size_t)nv * sizeof(double));
-  DevBuf d_quads, d_units, d_colpos;  // freed at the end, after the stream has run
+  DevBuf d_quads, d_units, d_colpos, missing;  // freed at the end, after the stream has run
+  up(missing, std::vector<int32_t>{0});
   if (near.nleaf > 0 && near.nnz > 0) {
     if (nq > 64 || dpc > 9) throw std::runtime_error("near assembly: more than 64 quad points or 9 DoFs per cell");
     // tiles of kAsmRows rows x kAsmCols columns of every leaf's block
@@ -2945,7 +2950,7 @@ void Engine::assemble_near(bool want_f32) {
     alloc(d_colpos, near.ent_cell.size() * dpc * sizeof(int));
     hipLaunchKernelGGL(k_entry_cols, dim3(near.nleaf, 4), dim3(256), 0, stream, d_ent_beg.as<int>(),
                        d_ent_cell.as<int>(), d_cdofs.as<int>(), dpc, d_col_beg.as<int>(), d_cols.as<int>(),
-                       d_colpos.as<int>());
+                       d_colpos.as<int>(), missing.as<int>());
     AsmArgs a{d_row_beg.as<int>(), d_rows.as<int>(), d_col_beg.as<int>(), d_cols.as<int>(), d_ent_beg.as<int>(),
               d_ent_cell.as<int>(), d_ent_mask.as<uint64_t>(), d_ent_near.as<uint8_t>(), d_colpos.as<int>(),
               d_val_beg.as<int64_t>(), nq, d_dbl_ptr.as<int>(), d_dbl_idx.as<int>(), d_xyz.as<double>(),
@@ -3001,6 +3006,7 @@ void Engine::assemble_near(bool want_f32) {
     tune_spmv<float, 2>();
     tune_spmv<float, 1>();
   }
+  check_columns(*this, missing, "near column position");
   sync();
 }
 

@@ -35,6 +35,19 @@ struct NoInit : std::allocator<T> {
   }
 };
 template <typename T> using RawVec = std::vector<T, NoInit<T>>;
+// Place of d among the sorted v[lo .. hi), -1 where it is none of them.
+#ifdef __HIPCC__
+__host__ __device__
+#endif
+inline int find_sorted(const int32_t *v, int lo, int hi, int32_t d) {
+  const int end = hi;
+  while (lo < hi) {
+    const int mid = lo + (hi - lo) / 2;
+    if (v[mid] < d) lo = mid + 1;
+    else hi = mid;
+  }
+  return lo < end && v[lo] == d ? lo : -1;
+}
 // Pairs per GEMM chunk of the batched translations (64 GEMM columns): 32 pairs
 // when both kernels' expansions travel (2 columns per pair), 64 pairs when
 // one combined expansion does.
