@@ -400,6 +400,7 @@ def measure_config(config, steps, warmup, leaf=None):
     log(f"config {config}: N={n} cells={pr.mesh.n_cells} p={pr.p} leaf {pr.max_nodes_per_leaf}")
     stream = hip.Stream()
     f, bp, setup = setup_handle(pr, stream)
+    f.time_choices()  # many solves on one handle: its plans are timed before the first
     log("setup: " + " ".join(f"{k}={v:.2f}" for k, v in setup.items()))
     wc = f.work_counts()
     solves = time_solves(f, bp, pr, stream, steps, warmup)
@@ -642,8 +643,7 @@ def mode_matvec(args):
     # do), so that the phase-timed runs below use the M2L form it chose; with
     # --plan the plan is set instead and no timing runs, so that every launch
     # of the run is a kernel alone on the device (per-kernel durations)
-    if args.plan >= 0:
-        f.set_side_fusion(prec, args.plan)
+    f.set_side_fusion(prec, args.plan if args.plan >= 0 else -1)
     bp.vmult_dev(a.value, oN.value, prec)
     # phase-timed, as the operator phases bench.py reports: every phase in its
     # own launch (the solve's fused launches are profiled with --mode solve)

@@ -380,7 +380,7 @@ int pbfmm_tuning_state(pbfmm_handle *h, int32_t *state);
  * reference): the preconditioner and the operator application of one Arnoldi
  * step of pbfmm_gmres_dev / pbfmm_solve_system run from a fixed input into a
  * fixed output, so the launches can be captured once and replayed.  -1
- * (default): after 512 steps of a precision (in the next steps after a call
+ * (default): after 256 steps of a precision (in the next steps after a call
  * with -1) the graph is captured and three replays are timed against three
  * direct runs, and the faster is kept; 0 direct launches only; 1 graph
  * replays.  A graph is captured again whenever a choice or buffer it holds

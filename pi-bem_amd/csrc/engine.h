@@ -215,9 +215,10 @@ struct Engine {
   // takes about 25 applications (time_plans), half of a solve, so a handle
   // that solves a few times keeps first_plan; single applications are timed
   // once a caller has made as many as a solve makes.  kGraphAfter: GMRES
-  // steps before the graph is timed (a capture and seven steps, paid back by
-  // hundreds of steps if at all).
-  static constexpr int kPlanAfter = 48, kSolvePlanAfter = 256, kGraphAfter = 512;
+  // steps before the graph is timed: a capture and seven steps, paid back by
+  // 140 steps where replays gain most (24,578 DoFs, leaf 96, FP64: 96 -> 89
+  // us a step) and never where they lose (FP32 there: 67 and 73 us).
+  static constexpr int kPlanAfter = 48, kSolvePlanAfter = 256, kGraphAfter = 256;
   int plan_apps[2] = {0, 0}, graph_steps[2] = {0, 0};  // plan_apps -1: time before the next application or solve
   // A solve keeps one launch plan from its first application to its last
   // (plans differ in the order of FP32 sums), so nothing is timed inside one.

@@ -4095,8 +4095,7 @@ std::vector<int64_t> Engine::graph_key(int precision) const {
 }
 
 // step_op(d_vn -> d_wk) as a graph replay when that was measured faster.
-// The first kGraphAfter steps per precision run directly (the choice costs
-// eight steps and a capture and gains 3% where it gains), the next captures
+// The first kGraphAfter steps per precision run directly, the next captures
 // the step after one more direct run (allocations on first use happen outside
 // the capture) and times three direct runs against three replays; from then
 // on the faster one runs, recaptured whenever graph_key changes.

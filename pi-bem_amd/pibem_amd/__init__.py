@@ -142,6 +142,14 @@ class BEMFMA:
         -1 times them again (pbfmm_set_side_fusion)."""
         self._chk(self._L.pbfmm_set_side_fusion(self._h, int(precision), int(mode)))
 
+    def time_choices(self):
+        """Has the next solves time the launch plan and the graph of either
+        precision at once, for a handle that will solve many times
+        (pbfmm_set_side_fusion and pbfmm_set_graph_mode with -1)."""
+        self.set_side_fusion(PBFMM_FP64, -1)
+        self.set_side_fusion(PBFMM_MIXED, -1)
+        self.set_graph_mode(-1)
+
     def tuning_state(self):
         """Choices the handle's timings made so far (-1 = not timed yet):
         SpMV kernels, side fusion modes, mixed scheme, FP64/FP32 operator
@@ -557,6 +565,7 @@ def tune_leaf_size(problem, precision=PBFMM_MIXED, solves=2, start=20, ladder=LE
         pr = dataclasses.replace(problem, max_nodes_per_leaf=int(leaf))
         t0 = time.perf_counter()
         f = setup(pr, precision, device)
+        f.time_choices()  # the handle is kept for many solves
         bp = BEMProblem(f)
         rhs = hip.DeviceArray.from_numpy(bp.compute_rhs(pr.tmp_rhs))
         hip.synchronize()
