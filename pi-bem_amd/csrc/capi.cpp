@@ -49,6 +49,7 @@ int guarded(pbfmm_handle *h, F &&f, bool device = true) {
     if (rc == PBFMM_OK) h->err.clear();
     return rc;
   } catch (const HipError &ex) {
+    (void)hipGetLastError();  // reported here: the next call does not find it again
     return fail(h, PBFMM_ERR_HIP, ex.what());
   } catch (const std::bad_alloc &) {
     return fail(h, PBFMM_ERR_ALLOC, "host allocation failed");
@@ -292,6 +293,7 @@ int pbfmm_generate_octree_blocking(pbfmm_handle *h) {
     if (int rc = not_batch(h, "generate_octree_blocking")) return rc;
     if (int rc = need(h, 1, "generate_octree_blocking")) return rc;
     Engine &e = h->eng;
+    h->stage = 1;  // a step that fails leaves the ones after it undone
     std::vector<double> gx, gw;
     gauss_legendre01(h->prm.quad_order, gx, gw);
     Quadrature2D rule = tensor_rule(gx, gw, gx, gw);
@@ -330,6 +332,7 @@ int pbfmm_direct_integrals(pbfmm_handle *h) {
     if (int rc = not_batch(h, "direct_integrals")) return rc;
     if (int rc = need(h, 2, "direct_integrals")) return rc;
     Engine &e = h->eng;
+    h->stage = 2;
     build_near_plan(e.mesh, e.qd, e.tree, e.near);
     if (e.near.nnz >= (int64_t(1) << 40)) return fail(h, PBFMM_ERR_ARG, "direct_integrals: near field too large");
     e.upload_mesh_and_tree();
@@ -347,6 +350,7 @@ int pbfmm_multipole_integrals(pbfmm_handle *h) {
     if (int rc = not_batch(h, "multipole_integrals")) return rc;
     if (int rc = need(h, 3, "multipole_integrals")) return rc;
     Engine &e = h->eng;
+    h->stage = 3;
     build_far_plan(e.tree, e.p, e.far);
     build_p2m_plan(e.mesh, e.qd, e.tree, e.far);
     validate_plans(e);

@@ -3963,6 +3963,7 @@ void Engine::prec_blocks(std::vector<double> &blk) {
 }
 
 void Engine::build_preconditioner() {
+  have_prec = false;  // until it is there
   // blocks: near leaves with the same parent block, in near-leaf order; a
   // parent of more than prec_rows rows is cut into ceil(rows / prec_rows)
   // blocks of about equal rows
@@ -4586,6 +4587,7 @@ int Engine::gmres(const double *b, double *x, double tol, int restart, int maxit
   settle_plan(precision);
   Solving in_solve(solving);
   if (restart != gm_restart) {
+    gm_restart = 0;  // until all of them are there
     alloc(d_V, (size_t)(restart + 1) * n * 8);
     alloc(d_w, n * 8);
     alloc(d_r, n * 8);
@@ -4982,6 +4984,7 @@ int Engine::gmres_forest(const double *b, double *x, double tol, int restart, in
   Solving in_solve(solving);
   const int S = (int)seg_off.size() - 1;
   if (restart != gm_restart) {
+    gm_restart = 0;  // until all of them are there
     alloc(d_V, (size_t)(restart + 1) * n * 8);
     alloc(d_w, n * 8);
     alloc(d_r, n * 8);
@@ -5034,6 +5037,7 @@ int Engine::gmres_forest(const double *b, double *x, double tol, int restart, in
 void Engine::multi_setup(int R) {
   if (R == mr_R) return;
   if (R < 1) throw std::runtime_error("multi_setup: no right-hand sides");
+  mr_R = 0;  // until the lists and buffers are there
   const int nb = tree.nb;
   if ((int64_t)R * nb >= (int64_t(1) << 31)) throw std::runtime_error("too many right-hand sides for this tree");
   // pairs of each chunk for every rhs (block ids rhs * nb + block), cut
@@ -5172,6 +5176,7 @@ int Engine::gmres_multi(const double *b, double *x, int R, double tol, int resta
   multi_setup(R);
   const int64_t N = (int64_t)R * n;
   if (restart != mr_restart) {
+    mr_restart = 0;  // until all of them are there
     alloc(mr_V, (size_t)(restart + 1) * N * 8);
     alloc(mr_w, N * 8);
     alloc(mr_r, N * 8);
