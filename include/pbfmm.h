@@ -354,7 +354,7 @@ int pbfmm_set_spmv_kernel(pbfmm_handle *h, int32_t precision, int32_t kernel);
  * 92: with M2P before the SpMV there; -1 times plans 0, 3, 5, 8, 24, 56 and
  * 92 before the next application or solve).  Without a call a plan chosen by
  * sizes runs; the plans are timed, once, before the 49th single application
- * of a precision or before a solve on a handle that has made 256 applications
+ * of a precision or before a solve on a handle that has made 1024 applications
  * in it.  A solve keeps one plan from its start to its end.  For tests and
  * tuning.  No counterpart in the reference. */
 int pbfmm_set_side_fusion(pbfmm_handle *h, int32_t precision, int32_t mode);
@@ -380,10 +380,10 @@ int pbfmm_tuning_state(pbfmm_handle *h, int32_t *state);
  * reference): the preconditioner and the operator application of one Arnoldi
  * step of pbfmm_gmres_dev / pbfmm_solve_system run from a fixed input into a
  * fixed output, so the launches can be captured once and replayed.  -1
- * (default): after 256 steps of a precision (in the next steps after a call
- * with -1) the graph is captured and three replays are timed against three
- * direct runs, and the faster is kept; 0 direct launches only; 1 graph
- * replays.  A graph is captured again whenever a choice or buffer it holds
+ * (default): after 512 steps of a precision and the timing of its launch plan
+ * (in the next steps after a call with -1) the graph is captured and three
+ * replays are timed against three direct runs, and the faster is kept; 0
+ * direct launches only; 1 graph replays.  A graph is captured again whenever a choice or buffer it holds
  * changes.  Batch handles and many right-hand sides launch directly. */
 int pbfmm_set_graph_mode(pbfmm_handle *h, int32_t mode);
 /* The timing behind the graph choice, ms per step: [0] [1] FP64 direct /

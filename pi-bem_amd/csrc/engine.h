@@ -212,14 +212,20 @@ struct Engine {
   static constexpr int kTimedPlans[] = {3, 5, 8, 24, 56, 92};  // besides 0 (time_plans)
   // Applications of a precision before its plans are timed: single ones
   // (pbfmm_vmult), and those a handle has run when a solve starts.  Timing
-  // takes about 25 applications (time_plans), half of a solve, so a handle
-  // that solves a few times keeps first_plan; single applications are timed
-  // once a caller has made as many as a solve makes.  kGraphAfter: GMRES
-  // steps before the graph is timed: a capture and seven steps, paid back by
-  // 140 steps where replays gain most (24,578 DoFs, leaf 96, FP64: 96 -> 89
-  // us a step) and never where they lose (FP32 there: 67 and 73 us).
-  static constexpr int kPlanAfter = 48, kSolvePlanAfter = 256, kGraphAfter = 256;
-  int plan_apps[2] = {0, 0}, graph_steps[2] = {0, 0};  // plan_apps -1: time before the next application or solve
+  // takes about 25 applications (time_plans; 393,218 DoFs, FP32: 16 ms beside
+  // a solve of 39) and gains 2% where it gains, so a handle that solves twenty
+  // times keeps first_plan; single applications are timed once a caller has
+  // made as many as a solve makes.  kGraphAfter: GMRES steps before the graph
+  // is timed, a capture and ten steps (6 ms there), paid back by 140 steps
+  // where replays gain most (24,578 DoFs, leaf 96, FP64: 96 -> 89 us a step)
+  // and never where they lose (FP32 there: 67 and 73 us).  A program that
+  // solves more often asks for both at once (-1 through the API).
+  static constexpr int kPlanAfter = 48, kSolvePlanAfter = 1024, kGraphAfter = 512;
+  // plan_apps -1: time before the next application or solve; graph_steps
+  // kGraphNow: in the next steps.  Unasked, the graph is timed with a plan
+  // that has been.
+  static constexpr int kGraphNow = 1 << 30;
+  int plan_apps[2] = {0, 0}, graph_steps[2] = {0, 0};
   // A solve keeps one launch plan from its first application to its last
   // (plans differ in the order of FP32 sums), so nothing is timed inside one.
   struct Solving {
@@ -231,7 +237,7 @@ struct Engine {
   void settle_plan(int precision);
   hipStream_t side_stream = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-  void make_side_stream();
+  void make_side_stream(bool chosen);
   void fork_side();
   int cus = 256;  // compute units of the device
   int m2l_beside(bool f32, int nk) const;  // workgroups of an M2L launch beside the SpMV, 0: one per chunk

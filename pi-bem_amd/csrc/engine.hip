@@ -2774,6 +2774,9 @@ void Engine::upload_far(bool want_f32) {
 // DoFs (0.3 M values) 148 / 188, 6,146 (1.4 M) 235 / 213, 24,578 at leaf 20
 // (7 M) 380 / 345, 38,402 Q2 at leaf 20 (15 M) 533 / 473, 98,306 1,027 / 887.
 constexpr int64_t kPairsBeside = 1000000;
+// The operator's SpMV on the second stream in the plan chosen by sizes, from
+// this many values on (first_plan).
+constexpr int64_t kSpmvBeside = 8000000;
 
 // Throws where k_entry_cols or k_quad_cols found a DoF in no column.
 static void check_columns(const Engine &e, const DevBuf &missing, const char *what) {
@@ -2862,8 +2865,8 @@ void Engine::build_unit_multipoles(bool want_f32) {
       HIPCHK(hipGetLastError());
       sync();  // the index copies are freed on return
     }
-    // the products' second stream is made (0.2 ms) while the GPU is busy here
-    if (near.nnz >= kPairsBeside) make_side_stream();
+    // the products' second stream, made outside any caller's capture
+    if (near.nnz >= kPairsBeside) make_side_stream(near.nnz >= kSpmvBeside);
     check_columns(*this, missing, "p2m column");
     sync();  // qpt, qleaf, qcol, dqbeg, dfit, dfit_half are freed on return
   }
@@ -3309,16 +3312,65 @@ void Engine::generate(const double *phi, const double *dphi) {
   HIPCHK(hipGetLastError());
 }
 
-void Engine::make_side_stream() {
+// flag[0] set by another stream's kernel, waited for at most `ticks`; flag[1]: whether it was seen
+__global__ void k_await_flag(int *flag, long long ticks) {
+  const long long t0 = wall_clock64();
+  int seen = 0;
+  while (!seen && wall_clock64() - t0 < ticks) {
+    seen = __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_s_sleep(8);
+  }
+  flag[1] = seen;
+}
+__global__ void k_raise_flag(int *flag) { __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+// Whether st runs beside this handle's stream.  A process has four hardware
+// queues, and two streams on one of them take turns: a kernel on the handle's
+// stream waits (0.2 ms at most) for one launched after it on st.
+static bool runs_beside(const Engine &e, hipStream_t st) {
+  DevBuf flag;
+  alloc(flag, 2 * sizeof(int));
+  hipLaunchKernelGGL(k_raise_flag, dim3(1), dim3(1), 0, st, flag.as<int>());  // st's first launch takes longer
+  HIPCHK(hipStreamSynchronize(st));
+  HIPCHK(hipMemsetAsync(flag.p, 0, 2 * sizeof(int), e.stream));
+  HIPCHK(hipStreamSynchronize(e.stream));
+  int khz = 0, got[2] = {0, 0};
+  HIPCHK(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, e.device));
+  hipLaunchKernelGGL(k_await_flag, dim3(1), dim3(1), 0, e.stream, flag.as<int>(), (long long)khz / 5);
+  hipLaunchKernelGGL(k_raise_flag, dim3(1), dim3(1), 0, st, flag.as<int>());
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(st));
+  HIPCHK(hipMemcpyAsync(got, flag.p, sizeof(got), hipMemcpyDeviceToHost, e.stream));
+  HIPCHK(hipStreamSynchronize(e.stream));
+  return got[1] != 0;
+}
+
+// The handle's second stream.  Where a plan chosen by sizes relies on it
+// (chosen), it is of up to four new ones (the queues are given out in turn)
+// the first that runs beside the handle's own: on its queue, the SpMV beside
+// M2L ran after it, and of four handles of 393,218 DoFs one took 738 us an
+// FP32 application where the others took 560 to 580.  (0.2 ms a stream, 0.1
+// to try it.)
+void Engine::make_side_stream(bool chosen) {
   if (side_stream) return;
   HIPCHK(hipEventCreateWithFlags(&ev_fork, hipEventDisableTiming));
   HIPCHK(hipEventCreateWithFlags(&ev_join, hipEventDisableTiming));
-  HIPCHK(hipStreamCreateWithFlags(&side_stream, hipStreamNonBlocking));
+  hipStream_t made[4] = {};
+  int n_made = 0, keep = 0;
+  for (bool found = false; !found && n_made < (chosen ? 4 : 1);) {
+    HIPCHK(hipStreamCreateWithFlags(&made[n_made], hipStreamNonBlocking));
+    found = chosen && runs_beside(*this, made[n_made]);
+    if (found) keep = n_made;
+    ++n_made;
+  }
+  side_stream = made[keep];
+  for (int k = 0; k < n_made; ++k)
+    if (k != keep) (void)hipStreamDestroy(made[k]);
 }
 
 // The second stream, ordered after what the handle's stream holds.
 void Engine::fork_side() {
-  make_side_stream();
+  make_side_stream(false);
   HIPCHK(hipEventRecord(ev_fork, stream));
   HIPCHK(hipStreamWaitEvent(side_stream, ev_fork, 0));
 }
@@ -3753,7 +3805,7 @@ int Engine::first_plan(bool f32) const {
   if (nnz <= 3000000) return m2p > nnz / 1000 ? 3 : 0;
   if (nnz <= 10000000 && m2l >= 100000) return 5;
   if (f32 && nnz >= 10000000 && m2l > nnz / 200) return 92;
-  return nnz >= (f32 ? 25000000 : 8000000) ? 24 : 0;
+  return nnz >= (f32 ? 25000000 : kSpmvBeside) ? 24 : 0;
 }
 // Times the plans on scratch vectors and keeps the fastest for the handle.
 // A plan's time is the best of three runs of a few applications (other
@@ -4100,14 +4152,17 @@ std::vector<int64_t> Engine::graph_key(int precision) const {
 }
 
 // step_op(d_vn -> d_wk) as a graph replay when that was measured faster.
-// The first kGraphAfter steps per precision run directly, the next captures
+// The first kGraphAfter steps per precision run directly, and as many as there
+// are until its launch plan has been timed; the next captures
 // the step after one more direct run (allocations on first use happen outside
 // the capture) and times three direct runs against three replays; from then
 // on the faster one runs, recaptured whenever graph_key changes.
 void Engine::step_op_graph(int precision) {
   const int f = precision == PBFMM_MIXED && have_f32 ? 1 : 0;
   double *vin = d_vn.as<double>(), *w = d_wk.as<double>();
-  if (!graph_enabled || graph_use[f] == 0 || (graph_use[f] < 0 && graph_steps[f]++ < kGraphAfter)) {
+  const bool later = graph_use[f] < 0 && graph_steps[f] < kGraphNow &&
+                     (graph_steps[f]++ < kGraphAfter || side_fusion[f] < 0);
+  if (!graph_enabled || graph_use[f] == 0 || later) {
     step_op(vin, w, precision);
     return;
   }
