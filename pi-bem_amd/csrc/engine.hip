@@ -1372,7 +1372,7 @@ static_assert(kM2LChunk == 32 && kChunk1 == 64, "k_translate maps 2 x 32 or 1 x 
 // are no multiple of the 4 SIMDs leaves the matrix cores of some of them
 // idle (the first waves of every workgroup go to the same SIMDs).  M2L of
 // 579,952 pairs at order 8, FP64 / FP32: 6 wavefronts, K = 96 372 / 233 us
-// (without gather and output 259, matrix cores 57% busy), 12 wavefronts,
+// (without gather and output 259), 12 wavefronts,
 // K = 84 307 / 190, near what its atomic adds take alone (305 / 177);
 // 211,368 pairs at order 7: 5 wavefronts of 80 rows 122 / 75, 8 of 64 rows
 // 92 / 54, into slots 109 / 45 and 56 / 31.
@@ -3799,13 +3799,22 @@ double Engine::norm2(const double *v) {
 //   stream, plan 24 (FP64 24,578 DoFs at leaf 96 89.7 / 85.2, 98,306 at leaf
 //   80 428 / 407; FP32 98,306 261 / 228, 393,218 775 / 641), with slots where
 //   M2L pairs are many for the values, FP32: plan 92 (38,402 DoFs at leaf 20
-//   136 / 114, 98,306 at leaf 32 236 / 202).
+//   136 / 114, 98,306 at leaf 32 236 / 202);
+//   with 1000 or more values for each M2L pair (large leaves, mirrored
+//   bodies, whose sources are stored several times) the SpMV bounds the
+//   application and M2L needs no CUs kept for it beside it: plan 8, FP64 / FP32
+//   us of plan 24 against 8: mirrored hull of 12,376 DoFs (153 M values, 6,752
+//   a pair) 426 / 264, 414 / 255; 98,306 DoFs at leaf 128 (1,078 a pair)
+//   412 / 243, 406 / 236; 38,402 at leaf 200 (2,095) 325 / 185, 297 / 171.
+//   Below, 393,218 DoFs at leaf 80 (770): FP64 925, plan 8 972; 98,306
+//   (640, order 8) 340 / 202, 379 / 232.
 int Engine::first_plan(bool f32) const {
   const int64_t nnz = near.nnz, m2l = (int64_t)far.m2l.tgt.size(), m2p = (int64_t)far.m2p_item_node.size();
   if (nnz <= 3000000) return m2p > nnz / 1000 ? 3 : 0;
   if (nnz <= 10000000 && m2l >= 100000) return 5;
   if (f32 && nnz >= 10000000 && m2l > nnz / 200) return 92;
-  return nnz >= (f32 ? 25000000 : kSpmvBeside) ? 24 : 0;
+  if (nnz < (f32 ? 25000000 : kSpmvBeside)) return 0;
+  return nnz / 1000 >= m2l ? 8 : 24;
 }
 // Times the plans on scratch vectors and keeps the fastest for the handle.
 // A plan's time is the best of three runs of a few applications (other
