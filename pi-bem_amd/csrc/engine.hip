@@ -3795,26 +3795,36 @@ double Engine::norm2(const double *v) {
 //   16.0, plan 3 16.4; 6,146 DoFs at leaf 64 33.0, plan 3 35.6).
 //   many M2L pairs beside them (24,578 DoFs, leaf 20, 7 M values): plan 5,
 //   100.1 / 84.5; FP64 133.4 / 114.6.
+//   larger, FP32 from 10 M values, with M2L pairs many for them: plan 92, the
+//   SpMV on the second stream and M2L into slots (38,402 DoFs at leaf 20
+//   136 / 114, 98,306 at leaf 32 236 / 202).
 //   larger, FP64 from 8 M and FP32 from 25 M values: the SpMV on the second
-//   stream, plan 24 (FP64 24,578 DoFs at leaf 96 89.7 / 85.2, 98,306 at leaf
-//   80 428 / 407; FP32 98,306 261 / 228, 393,218 775 / 641), with slots where
-//   M2L pairs are many for the values, FP32: plan 92 (38,402 DoFs at leaf 20
-//   136 / 114, 98,306 at leaf 32 236 / 202);
-//   with 1000 or more values for each M2L pair (large leaves, mirrored
-//   bodies, whose sources are stored several times) the SpMV bounds the
-//   application and M2L needs no CUs kept for it beside it: plan 8, FP64 / FP32
-//   us of plan 24 against 8: mirrored hull of 12,376 DoFs (153 M values, 6,752
-//   a pair) 426 / 264, 414 / 255; 98,306 DoFs at leaf 128 (1,078 a pair)
-//   412 / 243, 406 / 236; 38,402 at leaf 200 (2,095) 325 / 185, 297 / 171.
-//   Below, 393,218 DoFs at leaf 80 (770): FP64 925, plan 8 972; 98,306
-//   (640, order 8) 340 / 202, 379 / 232.
+//   stream from the start, plan 8, or from M2L on, beside M2L on one workgroup
+//   per CU, plan 24 (FP64 24,578 DoFs at leaf 96 89.7 / 85.2, 98,306 at leaf
+//   80 428 / 407; FP32 98,306 261 / 228, 393,218 775 / 641).  Plan 24 gains
+//   where M2L's workgroups fill a CU's wavefront slots and M2L is long enough
+//   to cover the SpMV: FP64 from 8 wavefronts a workgroup (order 5 up), FP32
+//   from 12 (orders 5, 8 and up), below 1000 values for each pair.
+//   Otherwise plan 8.  FP64 / FP32, plan 8 against 24:
+//     order 4 (4 wavefronts): 345,602 DoFs, leaf 80 750 / 418, 768 / 449;
+//     98,306, leaf 64 212 / 133, 217 / 144.
+//     order 5 (12): 345,602, leaf 80 859 / 516, 792 / 462; 98,306, leaf 80
+//     273 / 171, 260 / 168.
+//     orders 6, 7 (8): 393,218, leaf 80 972 / 522, 925 / 530 (order 7 1,063 /
+//     538, 1,006 / 554); 64,898, leaf 80 219 / 129, 235 / 145.
+//     order 8 (12): 393,218, leaf 80 1,293 / 713, 1,151 / 621; 98,306, leaf 96
+//     376 / 225, 341 / 203.
+//     from 1000 values a pair (large leaves, mirrored bodies): hull of 12,376
+//     DoFs (6,752) 414 / 255, 426 / 264; 98,306 at order 8, leaf 128 (1,078)
+//     406 / 236, 412 / 243; 38,402, leaf 200 (2,095) 297 / 171, 325 / 185.
 int Engine::first_plan(bool f32) const {
   const int64_t nnz = near.nnz, m2l = (int64_t)far.m2l.tgt.size(), m2p = (int64_t)far.m2p_item_node.size();
   if (nnz <= 3000000) return m2p > nnz / 1000 ? 3 : 0;
   if (nnz <= 10000000 && m2l >= 100000) return 5;
   if (f32 && nnz >= 10000000 && m2l > nnz / 200) return 92;
   if (nnz < (f32 ? 25000000 : kSpmvBeside)) return 0;
-  return nnz / 1000 >= m2l ? 8 : 24;
+  const int waves = kp / 16 * tr_column_waves(kp / 16);
+  return waves < (f32 ? 12 : 8) || nnz / 1000 >= m2l ? 8 : 24;
 }
 // Times the plans on scratch vectors and keeps the fastest for the handle.
 // A plan's time is the best of three runs of a few applications (other
