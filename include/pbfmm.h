@@ -380,11 +380,12 @@ int pbfmm_tuning_state(pbfmm_handle *h, int32_t *state);
  * reference): the preconditioner and the operator application of one Arnoldi
  * step of pbfmm_gmres_dev / pbfmm_solve_system run from a fixed input into a
  * fixed output, so the launches can be captured once and replayed.  -1
- * (default): after 512 steps of a precision and the timing of its launch plan
- * (in the next steps after a call with -1) the graph is captured and three
- * replays are timed against three direct runs, and the faster is kept; 0
- * direct launches only; 1 graph replays.  A graph is captured again whenever a choice or buffer it holds
- * changes.  Batch handles and many right-hand sides launch directly. */
+ * (default): after 64 steps of a precision (in the next steps after a call
+ * with -1) the graph is captured behind one step, of the six after it three
+ * run directly and three as replays, and the faster is kept; 0 direct launches
+ * only; 1 graph replays.  A graph is captured again whenever a choice or
+ * buffer it holds changes, and timed again when the plans' timing changes the
+ * plan.  Batch handles and many right-hand sides launch directly. */
 int pbfmm_set_graph_mode(pbfmm_handle *h, int32_t mode);
 /* The timing behind the graph choice, ms per step: [0] [1] FP64 direct /
  * graph, [2] [3] FP32 direct / graph (0 until timed). */

@@ -1119,7 +1119,7 @@ int pbfmm_set_graph_mode(pbfmm_handle *h, int32_t mode) {
   Engine &e = h->eng;
   e.graph_enabled = mode != 0;
   e.graph_use[0] = e.graph_use[1] = e.set_graph = mode;
-  e.graph_steps[0] = e.graph_steps[1] = Engine::kGraphNow;  // -1: timed in the next steps
+  e.graph_steps[0] = e.graph_steps[1] = Engine::kGraphAfter;  // -1: timed in the next steps
   return PBFMM_OK;
 }
 

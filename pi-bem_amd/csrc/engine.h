@@ -216,15 +216,11 @@ struct Engine {
   // a solve of 39) and gains 2% where it gains, so a handle that solves twenty
   // times keeps first_plan; single applications are timed once a caller has
   // made as many as a solve makes.  kGraphAfter: GMRES steps before the graph
-  // is timed, a capture and ten steps (6 ms there), paid back by 140 steps
-  // where replays gain most (24,578 DoFs, leaf 96, FP64: 96 -> 89 us a step)
-  // and never where they lose (FP32 there: 67 and 73 us).  A program that
-  // solves more often asks for both at once (-1 through the API).
-  static constexpr int kPlanAfter = 48, kSolvePlanAfter = 1024, kGraphAfter = 512;
-  // plan_apps -1: time before the next application or solve; graph_steps
-  // kGraphNow: in the next steps.  Unasked, the graph is timed with a plan
-  // that has been.
-  static constexpr int kGraphNow = 1 << 30;
+  // is timed (step_op_graph).  That costs a capture, 0.3 to 0.7 ms, and gains
+  // up to 20 us a step (mirrored hull of 8,326 DoFs, FP64: 251 -> 228).  A
+  // program that solves more often asks for both at once (-1 through the API).
+  static constexpr int kPlanAfter = 48, kSolvePlanAfter = 1024, kGraphAfter = 64;
+  // plan_apps -1: time before the next application or solve
   int plan_apps[2] = {0, 0}, graph_steps[2] = {0, 0};
   // A solve keeps one launch plan from its first application to its last
   // (plans differ in the order of FP32 sums), so nothing is timed inside one.
@@ -263,6 +259,20 @@ struct Engine {
   hipGraphExec_t op_graph[2] = {nullptr, nullptr};
   std::vector<int64_t> op_graph_key[2];
   DevBuf d_vn, d_wk;
+  // Steps timed for the choice, direct and replayed in turn (step_op_graph)
+  struct GraphTrial {
+    static constexpr int kSteps = 6;
+    int steps = 0;
+    hipEvent_t ev[2 * kSteps] = {};
+    void drop() {
+      for (hipEvent_t &e : ev) {
+        if (e) (void)hipEventDestroy(e);
+        e = nullptr;
+      }
+      steps = 0;
+    }
+  };
+  GraphTrial graph_trial[2];
   float graph_ms[2][2] = {{0, 0}, {0, 0}};  // timed ms per step: direct, graph
   int64_t constraint_version = 0;
   void step_op(const double *vin, double *w, int precision);

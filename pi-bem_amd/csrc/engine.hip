@@ -2638,6 +2638,7 @@ void Engine::drop_graphs() {
     if (op_graph[f]) (void)hipGraphExecDestroy(op_graph[f]);
     op_graph[f] = nullptr;
     op_graph_key[f].clear();
+    graph_trial[f].drop();
   }
 }
 
@@ -3883,7 +3884,10 @@ int Engine::time_plans(bool f32) {
   if (stay * 0.99f <= best) pick = usual;
   for (hipEvent_t e : ev) (void)hipEventDestroy(e);
   d_cost.release();
-  if (pick != usual) op_cost_ratio = 0;  // the precisions' cost ratio was another plan's
+  if (pick != usual) {  // what was measured with the other plan
+    op_cost_ratio = 0;
+    if (set_graph < 0) graph_use[f32 ? 1 : 0] = -1;
+  }
   return side_fusion[f32 ? 1 : 0] = pick;
 }
 
@@ -4171,24 +4175,26 @@ std::vector<int64_t> Engine::graph_key(int precision) const {
 }
 
 // step_op(d_vn -> d_wk) as a graph replay when that was measured faster.
-// The first kGraphAfter steps per precision run directly, and as many as there
-// are until its launch plan has been timed; the next captures
-// the step after one more direct run (allocations on first use happen outside
-// the capture) and times three direct runs against three replays; from then
-// on the faster one runs, recaptured whenever graph_key changes.
+// The first kGraphAfter steps per precision run directly, the next as well and
+// is captured behind it (allocations on first use happen outside the capture).
+// Of the six after that every second one replays, between events: each is a
+// step of the solve, so the measurement costs the capture alone.  From then on
+// the faster one runs, recaptured whenever graph_key changes.
 void Engine::step_op_graph(int precision) {
   const int f = precision == PBFMM_MIXED && have_f32 ? 1 : 0;
   double *vin = d_vn.as<double>(), *w = d_wk.as<double>();
-  const bool later = graph_use[f] < 0 && graph_steps[f] < kGraphNow &&
-                     (graph_steps[f]++ < kGraphAfter || side_fusion[f] < 0);
+  const bool later = graph_use[f] < 0 && graph_steps[f] < kGraphAfter;
   if (!graph_enabled || graph_use[f] == 0 || later) {
+    if (later) ++graph_steps[f];
     step_op(vin, w, precision);
     return;
   }
+  GraphTrial &tr = graph_trial[f];
   if (!op_graph[f] || op_graph_key[f] != graph_key(precision)) {
     if (op_graph[f]) (void)hipGraphExecDestroy(op_graph[f]);
     op_graph[f] = nullptr;
-    step_op(vin, w, precision);  // allocations on first use, outside the capture
+    tr.steps = 0;
+    step_op(vin, w, precision);
     hipGraph_t g = nullptr;
     HIPCHK(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
     try {
@@ -4206,33 +4212,34 @@ void Engine::step_op_graph(int precision) {
       throw HipError("operator graph instantiation failed");
     }
     op_graph_key[f] = graph_key(precision);
+    return;
   }
-  if (graph_use[f] < 0) {
-    hipEvent_t t0, t1, t2;
-    HIPCHK(hipEventCreate(&t0));
-    HIPCHK(hipEventCreate(&t1));
-    HIPCHK(hipEventCreate(&t2));
-    HIPCHK(hipGraphLaunch(op_graph[f], stream));  // warm
-    HIPCHK(hipEventRecord(t0, stream));
-    for (int r = 0; r < 3; ++r) step_op(vin, w, precision);
-    HIPCHK(hipEventRecord(t1, stream));
-    for (int r = 0; r < 3; ++r) HIPCHK(hipGraphLaunch(op_graph[f], stream));
-    HIPCHK(hipEventRecord(t2, stream));
-    HIPCHK(hipEventSynchronize(t2));
-    float md = 0, mg = 0;
-    HIPCHK(hipEventElapsedTime(&md, t0, t1));
-    HIPCHK(hipEventElapsedTime(&mg, t1, t2));
-    (void)hipEventDestroy(t0);
-    (void)hipEventDestroy(t1);
-    (void)hipEventDestroy(t2);
-    graph_use[f] = mg < 0.98f * md ? 1 : 0;
-    graph_ms[f][0] = md / 3;
-    graph_ms[f][1] = mg / 3;
+  const bool timed = graph_use[f] < 0, replay = !timed || tr.steps % 2 == 1;
+  if (timed) {
+    for (hipEvent_t &e : tr.ev)
+      if (!e) HIPCHK(hipEventCreate(&e));
+    HIPCHK(hipEventRecord(tr.ev[2 * tr.steps], stream));
   }
-  if (graph_use[f] == 1)
+  if (replay) {
     HIPCHK(hipGraphLaunch(op_graph[f], stream));
-  else
+    if (plan_apps[f] >= 0) ++plan_apps[f];  // as use_side_fusion counts
+  } else {
     step_op(vin, w, precision);
+  }
+  if (!timed) return;
+  HIPCHK(hipEventRecord(tr.ev[2 * tr.steps + 1], stream));
+  if (++tr.steps < GraphTrial::kSteps) return;
+  tr.steps = 0;
+  HIPCHK(hipEventSynchronize(tr.ev[2 * GraphTrial::kSteps - 1]));
+  float best[2] = {0, 0};
+  for (int k = 0; k < GraphTrial::kSteps; ++k) {
+    float ms = 0;
+    HIPCHK(hipEventElapsedTime(&ms, tr.ev[2 * k], tr.ev[2 * k + 1]));
+    best[k % 2] = k < 2 ? ms : std::min(best[k % 2], ms);
+  }
+  tr.drop();
+  for (int k = 0; k < 2; ++k) graph_ms[f][k] = best[k];
+  graph_use[f] = best[1] < 0.98f * best[0] ? 1 : 0;
 }
 
 // Restarted GMRES with classical Gram-Schmidt and one reorthogonalisation
