@@ -1372,8 +1372,7 @@ static_assert(kM2LChunk == 32 && kChunk1 == 64, "k_translate maps 2 x 32 or 1 x 
 // are no multiple of the 4 SIMDs leaves the matrix cores of some of them
 // idle (the first waves of every workgroup go to the same SIMDs).  M2L of
 // 579,952 pairs at order 8, FP64 / FP32: 6 wavefronts, K = 96 372 / 233 us
-// (without gather and output 259), 12 wavefronts,
-// K = 84 307 / 190, near what its atomic adds take alone (305 / 177);
+// (without gather and output 259), 12 wavefronts, K = 84 307 / 190;
 // 211,368 pairs at order 7: 5 wavefronts of 80 rows 122 / 75, 8 of 64 rows
 // 92 / 54, into slots 109 / 45 and 56 / 31.
 __host__ __device__ constexpr int tr_column_waves(int nr) { return nr % 2 == 0 || nr > 4 ? 2 : 4; }
