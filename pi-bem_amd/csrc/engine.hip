@@ -3798,10 +3798,11 @@ double Engine::norm2(const double *v) {
 //   larger, FP32 from 10 M values, with M2L pairs many for them: plan 92, the
 //   SpMV on the second stream and M2L into slots (38,402 DoFs at leaf 20
 //   136 / 114, 98,306 at leaf 32 236 / 202).
-//   larger, FP64 from 8 M and FP32 from 25 M values: the SpMV on the second
+//   larger, FP64 from 8 M and FP32 from 18.5 M values: the SpMV on the second
 //   stream from the start, plan 8, or from M2L on, beside M2L on one workgroup
 //   per CU, plan 24 (FP64 24,578 DoFs at leaf 96 89.7 / 85.2, 98,306 at leaf
-//   80 428 / 407; FP32 98,306 261 / 228, 393,218 775 / 641).  Plan 24 gains
+//   80 428 / 407; FP32 98,306 261 / 228, 393,218 775 / 641; 24,578 at
+//   leaf 96, 18.6 M, 69 / 64, sphere with 18.1 M 62 / 65).  Plan 24 gains
 //   where M2L's workgroups fill a CU's wavefront slots and M2L is long enough
 //   to cover the SpMV: FP64 from 8 wavefronts a workgroup (order 5 up), FP32
 //   from 12 (orders 5, 8 and up), below 1000 values for each pair.
@@ -3822,7 +3823,7 @@ int Engine::first_plan(bool f32) const {
   if (nnz <= 3000000) return m2p > nnz / 1000 ? 3 : 0;
   if (nnz <= 10000000 && m2l >= 100000) return 5;
   if (f32 && nnz >= 10000000 && m2l > nnz / 200) return 92;
-  if (nnz < (f32 ? 25000000 : kSpmvBeside)) return 0;
+  if (nnz < (f32 ? 18500000 : kSpmvBeside)) return 0;
   const int waves = kp / 16 * tr_column_waves(kp / 16);
   return waves < (f32 ? 12 : 8) || nnz / 1000 >= m2l ? 8 : 24;
 }
